@@ -9,8 +9,7 @@
 // Numbers: activations and activation gradients are BF16 (channels last,
 // [n][z][y][x][c]); weights are FP32 masters updated by Adam and repacked to
 // BF16 MFMA fragments after every step; all products accumulate in FP32 on
-// the matrix cores (v_mfma_f32_16x16x32_bf16 for the convolutions,
-// v_mfma_f32_16x16x16_bf16 for the weight gradients); the head (1x1x1
+// the matrix cores (v_mfma_f32_16x16x32_bf16); the head (1x1x1
 // convolution to one channel plus alpha times the input) and the loss are
 // FP32.
 //
@@ -21,8 +20,8 @@
 // taps form one K = 32 step.  The backward pass with respect to the input is
 // the same kernel with the taps mirrored and the channel roles swapped
 // (weights repacked once per step), its epilogue multiplying by the ReLU
-// mask of the layer below.  Weight gradients contract over voxels (K = 16
-// voxels of an x row) with the input slice and the output-gradient block
+// mask of the layer below.  Weight gradients contract over voxels (K = 32:
+// two x rows of 16) with the input slice and the output-gradient block
 // both staged in LDS; each work-group sums a fixed subset of blocks and a
 // second kernel adds the partial sums in a fixed order, so gradients are
 // deterministic.
@@ -157,109 +156,167 @@ __global__ void __launch_bounds__(256) k_cr_conv(const unsigned short* __restric
     }
 }
 
-// Weight gradients of one 16-channel input slice (blockIdx.y) and one
-// 16-channel output block (blockIdx.z), summed over the output blocks
-// g, g + G, g + 2G, ... (g = blockIdx.x): part[g][tap][ci][co] (FP32).
-// Waves take taps w, w + 4, w + 8, ...; K = the 16 voxels of one x row.
-__global__ void __launch_bounds__(256) k_cr_wgrad(const unsigned short* __restrict__ in, int in_cs, int in_co,
-                                                  int cin, const unsigned short* __restrict__ dy, int dy_cs,
-                                                  int dy_co, int cout, float* __restrict__ part, CrShape s,
-                                                  int G) {
-    __shared__ unsigned short xs[CR_HVOX * 17];
-    __shared__ unsigned short ys[CR_BX * CR_BY * CR_BZ * 17];
-    const int g = blockIdx.x, c = blockIdx.y, nb = blockIdx.z;
+// Four 16-bit LDS values per lane, transposed over each group of 16 lanes:
+// lane 4 r + c of a group reads 8 bytes (row r, columns 4 c .. 4 c + 3) and
+// lane j receives column j of rows 0 .. 3.  With a row per voxel and a column
+// per channel this turns channels-last data into the K-major fragments of a
+// contraction over voxels.
+__device__ __forceinline__ cr_s4 cr_read_tr(const unsigned short* p) {
+    typedef __attribute__((address_space(3))) cr_s4 lds_s4;
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)p);
+}
+__device__ __forceinline__ cr_b8 cr_frag_tr(const unsigned short* p0, const unsigned short* p1) {
+    const cr_s4 a = cr_read_tr(p0), b = cr_read_tr(p1);
+    return __builtin_bit_cast(cr_b8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+constexpr int CR_WBX = 16, CR_WBY = 8, CR_WBZ = 4;     // voxel block of a weight-gradient step
+constexpr int CR_WHX = CR_WBX + 2, CR_WHY = CR_WBY + 2, CR_WHZ = CR_WBZ + 2;
+constexpr int CR_WT = 192;                             // three waves
+
+// Weight and bias gradients of one 16-channel input slice (blockIdx.y) and
+// NO blocks of 16 output channels (from blockIdx.z * NO), summed over the
+// voxel blocks g, g + G, g + 2 G, ... (g = blockIdx.x) of the cube
+// [lo, hi)^3 outside which dy is zero: part[g][tap][ci][co], then
+// part[g][27 cin cout + co] (FP32).
+//
+// Bound by LDS reads: both operands are staged channels last and read through
+// the transposing LDS load, 512 bytes an instruction.  K = 32 is two x rows of
+// 16 voxels.  A wave owns three of the nine (dy, dx) taps with all three dz:
+// it holds the output gradients of the block's four z planes in registers, so
+// each input fragment (one of six planes) serves up to three products, 18
+// input reads for 36 products.  Staging 16 x 8 x 4 voxels with their halo
+// reads 2.1 times the input.  The form before it (one 16-bit LDS read per
+// element, K = 16) took 512 us a layer on average for four 80^3 crops.
+template <int NO>
+__global__ void __launch_bounds__(CR_WT) k_cr_wgrad(const unsigned short* __restrict__ in, int in_cs, int in_co,
+                                                    int cin, const unsigned short* __restrict__ dy, int dy_cs,
+                                                    int dy_co, int cout, float* __restrict__ part, CrShape s, int lo,
+                                                    int hi, int G) {
+    __shared__ __align__(16) unsigned short xs[CR_WHX * CR_WHY * CR_WHZ * 16];
+    __shared__ __align__(16) unsigned short ys[NO][CR_WBX * CR_WBY * CR_WBZ * 16];
+    const int g = blockIdx.x, c = blockIdx.y, o0 = blockIdx.z * NO * 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int m = lane & 15, kq = lane >> 4;
-    cr_f4 acc[7];
+    // this lane's part of a transposed read: voxel row m / 4 of its group of
+    // four, channels 4 (m % 4) ..; the group's first voxel is x = 8 (kq % 2)
+    // of row kq / 2 (the second read takes the next four voxels)
+    const int lrow = kq >> 1, lvx = (kq & 1) * 8 + (m >> 2), lch = (m & 3) * 4;
+    const int e = hi - lo;
+    const int bx_n = (e + CR_WBX - 1) / CR_WBX, by_n = (e + CR_WBY - 1) / CR_WBY, bz_n = (e + CR_WBZ - 1) / CR_WBZ;
+    const int nblocks = s.n * bz_n * by_n * bx_n;
+    cr_f4 acc[9][NO], bacc[NO];
 #pragma unroll
-    for (int t = 0; t < 7; t++) acc[t] = cr_f4{0.f, 0.f, 0.f, 0.f};
-    const int nblocks = s.n * s.tz * s.ty * s.tx;
+    for (int nb = 0; nb < NO; nb++) {
+        bacc[nb] = cr_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 9; t++) acc[t][nb] = cr_f4{0.f, 0.f, 0.f, 0.f};
+    }
+    cr_b8 ones;
+#pragma unroll
+    for (int i = 0; i < 8; i++) ones[i] = (__bf16)1.f;
     for (int blk0 = g; blk0 < nblocks; blk0 += G) {
         int blk = blk0;
-        const int bx = blk % s.tx; blk /= s.tx;
-        const int by = blk % s.ty; blk /= s.ty;
-        const int bz = blk % s.tz;
-        const int b = blk / s.tz;
-        const int x0 = bx * CR_BX, y0 = by * CR_BY, z0 = bz * CR_BZ;
+        const int x0 = lo + blk % bx_n * CR_WBX; blk /= bx_n;
+        const int y0 = lo + blk % by_n * CR_WBY; blk /= by_n;
+        const int z0 = lo + blk % bz_n * CR_WBZ;
+        const int b = blk / bz_n;
         __syncthreads();
-        for (int t = threadIdx.x; t < CR_HVOX * 16; t += 256) {
-            const int v = t >> 4, ch = t & 15;
-            const int lx = v % CR_HX, ly = (v / CR_HX) % CR_HY, lz = v / (CR_HX * CR_HY);
+        for (int t = threadIdx.x; t < CR_WHX * CR_WHY * CR_WHZ * 2; t += CR_WT) {
+            const int v = t >> 1, half = t & 1;
+            const int lx = v % CR_WHX, ly = (v / CR_WHX) % CR_WHY, lz = v / (CR_WHX * CR_WHY);
             const int gx = x0 - 1 + lx, gy = y0 - 1 + ly, gz = z0 - 1 + lz;
-            unsigned short val = 0;
+            uint4 val = {0u, 0u, 0u, 0u};
             if (gx >= 0 && gx < s.w && gy >= 0 && gy < s.h && gz >= 0 && gz < s.d)
-                val = in[cr_vox(s, b, gz, gy, gx) * in_cs + in_co + c * 16 + ch];
-            xs[v * 17 + ch] = val;
+                val = *reinterpret_cast<const uint4*>(in + cr_vox(s, b, gz, gy, gx) * in_cs + in_co + c * 16 +
+                                                      half * 8);
+            *reinterpret_cast<uint4*>(xs + t * 8) = val;
         }
-        for (int t = threadIdx.x; t < CR_BX * CR_BY * CR_BZ * 16; t += 256) {
-            const int v = t >> 4, ch = t & 15;
-            const int lx = v % CR_BX, ly = (v / CR_BX) % CR_BY, lz = v / (CR_BX * CR_BY);
-            const int gx = x0 + lx, gy = y0 + ly, gz = z0 + lz;
-            unsigned short val = 0;
-            if (gx < s.w && gy < s.h && gz < s.d) val = dy[cr_vox(s, b, gz, gy, gx) * dy_cs + dy_co + nb * 16 + ch];
-            ys[v * 17 + ch] = val;
-        }
+#pragma unroll
+        for (int nb = 0; nb < NO; nb++)
+            for (int t = threadIdx.x; t < CR_WBX * CR_WBY * CR_WBZ * 2; t += CR_WT) {
+                const int v = t >> 1, half = t & 1;
+                const int lx = v % CR_WBX, ly = (v / CR_WBX) % CR_WBY, lz = v / (CR_WBX * CR_WBY);
+                const int gx = x0 + lx, gy = y0 + ly, gz = z0 + lz;
+                uint4 val = {0u, 0u, 0u, 0u};
+                if (gx < hi && gy < hi && gz < hi)
+                    val = *reinterpret_cast<const uint4*>(dy + cr_vox(s, b, gz, gy, gx) * dy_cs + dy_co + o0 +
+                                                          nb * 16 + half * 8);
+                *reinterpret_cast<uint4*>(ys[nb] + t * 8) = val;
+            }
         __syncthreads();
 #pragma unroll 1
-        for (int row = 0; row < CR_BY * CR_BZ; row++) {
-            const int ry = row & 3, rz = row >> 2;
-            cr_s4 bb;
+        for (int yp = 0; yp < CR_WBY; yp += 2) {
+            cr_b8 bf[CR_WBZ][NO];
 #pragma unroll
-            for (int i = 0; i < 4; i++) bb[i] = (short)ys[((rz * CR_BY + ry) * CR_BX + 4 * kq + i) * 17 + m];
+            for (int z = 0; z < CR_WBZ; z++)
 #pragma unroll
-            for (int ti = 0; ti < 7; ti++) {
-                const int tap = wave + 4 * ti;
-                if (tap < 27) {
-                    const int dz = tap / 9 - 1, dyy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-                    const int vrow = ((rz + 1 + dz) * CR_HY + (ry + 1 + dyy)) * CR_HX + 1 + dx;
-                    cr_s4 a;
+                for (int nb = 0; nb < NO; nb++) {
+                    const unsigned short* q = ys[nb] + ((z * CR_WBY + yp + lrow) * CR_WBX + lvx) * 16 + lch;
+                    bf[z][nb] = cr_frag_tr(q, q + 4 * 16);
+                }
+            if (wave == 0) {
 #pragma unroll
-                    for (int i = 0; i < 4; i++) a[i] = (short)xs[(vrow + 4 * kq + i) * 17 + m];
-                    acc[ti] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb, acc[ti], 0, 0, 0);
+                for (int z = 0; z < CR_WBZ; z++)
+#pragma unroll
+                    for (int nb = 0; nb < NO; nb++)
+                        bacc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, bf[z][nb], bacc[nb], 0, 0, 0);
+            }
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                // (dy, dx) = (wave, k) - 1
+                const unsigned short* q = xs + ((yp + lrow + wave) * CR_WHX + lvx + k) * 16 + lch;
+#pragma unroll
+                for (int zz = 0; zz < CR_WHZ; zz++) {
+                    const unsigned short* r = q + zz * CR_WHX * CR_WHY * 16;
+                    const cr_b8 af = cr_frag_tr(r, r + 4 * 16);
+#pragma unroll
+                    for (int dz = 0; dz < 3; dz++) {
+                        const int z = zz - dz;  // input plane zz (with halo) = output plane z + dz
+                        if (z < 0 || z >= CR_WBZ) continue;
+#pragma unroll
+                        for (int nb = 0; nb < NO; nb++)
+                            acc[dz * 3 + k][nb] =
+                                __builtin_amdgcn_mfma_f32_16x16x32_bf16(af, bf[z][nb], acc[dz * 3 + k][nb], 0, 0, 0);
+                    }
                 }
             }
         }
     }
     // D[ci = 4 kq + i][co = m]
+    const size_t nw = (size_t)27 * cin * cout;
+    float* P = part + (size_t)g * (nw + cout);
 #pragma unroll
-    for (int ti = 0; ti < 7; ti++) {
-        const int tap = wave + 4 * ti;
-        if (tap >= 27) break;
+    for (int nb = 0; nb < NO; nb++) {
+        const int co = o0 + nb * 16 + m;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int ci = c * 16 + 4 * kq + i, co = nb * 16 + m;
-            part[(((size_t)g * 27 + tap) * cin + ci) * cout + co] = acc[ti][i];
+        for (int t = 0; t < 9; t++) {
+            const int tap = (t / 3) * 9 + wave * 3 + t % 3;
+#pragma unroll
+            for (int i = 0; i < 4; i++) P[((size_t)tap * cin + c * 16 + 4 * kq + i) * cout + co] = acc[t][nb][i];
         }
+        if (c == 0 && wave == 0 && kq == 0) P[nw + co] = bacc[nb][0];
     }
 }
 
-// Sum of the G partial gradients (in order g = 0 .. G-1) into grad.
-__global__ void k_cr_reduce(const float* __restrict__ part, int G, size_t n, float* __restrict__ grad) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
+// Sum of the G partial gradients of n values into grad.  A work-group takes
+// 64 values, four threads a value with a quarter of the partials each; every
+// quarter and the four quarters are added in order, so the sum is the same in
+// every run.
+__global__ void __launch_bounds__(256) k_cr_reduce(const float* __restrict__ part, int G, size_t n,
+                                                   float* __restrict__ grad) {
+    __shared__ float red[4][64];
+    const int l = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const size_t t = (size_t)blockIdx.x * 64 + l;
+    const int per = (G + 3) / 4, g1 = min(G, (q + 1) * per);
     float sum = 0.f;
-    for (int g = 0; g < G; g++) sum += part[(size_t)g * n + t];
-    grad[t] = sum;
-}
-
-// Bias gradient partial sums: part[g][c] = sum over voxels v = g, g + G, ...
-// of dy[v][c] (one work-group per g, threads over channels and voxel lanes).
-__global__ void __launch_bounds__(256) k_cr_bgrad(const unsigned short* __restrict__ dy, int dy_cs, int dy_co,
-                                                  int cout, size_t nvox, float* __restrict__ part, int G) {
-    __shared__ float red[256];
-    const int g = blockIdx.x;
-    const int ch = threadIdx.x % cout, lanes = 256 / cout, li = threadIdx.x / cout;
-    float sum = 0.f;
-    if (li < lanes)
-        for (size_t v = (size_t)g * lanes + li; v < nvox; v += (size_t)G * lanes)
-            sum += cr_bf2f(dy[v * dy_cs + dy_co + ch]);
-    red[threadIdx.x] = (li < lanes) ? sum : 0.f;
+    if (t < n) {
+#pragma unroll 8
+        for (int g = q * per; g < g1; g++) sum += part[(size_t)g * n + t];
+    }
+    red[q][l] = sum;
     __syncthreads();
-    if (threadIdx.x < cout) {
-        float t = 0.f;
-        for (int k = 0; k < lanes; k++) t += red[k * cout + threadIdx.x];
-        part[(size_t)g * cout + threadIdx.x] = t;
-    }
+    if (q == 0 && t < n) grad[t] = ((red[0][l] + red[1][l]) + red[2][l]) + red[3][l];
 }
 
 // 2 x 2 x 2 average pooling: out (c channels) from in at half resolution.
@@ -371,54 +428,71 @@ __global__ void k_cr_head(const unsigned short* __restrict__ act, const float* _
 // Loss and head backward over the central tile^3 of every T^3 crop
 // (halo h): L = sum (out - tgt)^2 / count; g = 2 (out - tgt) / count there and
 // 0 in the halo; gact[v][c] = g w1[c] (act > 0); per work-group partial sums
-// part[blk][0..19] = {dw1[16], db1, dalpha, loss, -}.
+// part[wg][20] = {dw1[16], db1, dalpha, loss, 0}.  Work-groups walk the voxels
+// in strides of the grid (CR_HEADG of them), each lane keeping its own sums;
+// lanes are added by a fixed shuffle tree, then the waves in order.
+constexpr int CR_HEADG = 1024;
 __global__ void __launch_bounds__(256) k_cr_head_bwd(const unsigned short* __restrict__ act,
                                                      const float* __restrict__ x0f, const float* __restrict__ out,
                                                      const float* __restrict__ tgt, const float* __restrict__ hp,
                                                      int T, int halo, size_t nvox, float inv_count,
                                                      unsigned short* __restrict__ gact, float* __restrict__ part) {
-    __shared__ float red[256 * 20];
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    float loc[20];
+    __shared__ float red[4][20];
+    float w1[16], loc[19];
 #pragma unroll
-    for (int k = 0; k < 20; k++) loc[k] = 0.f;
-    if (t < nvox) {
+    for (int c = 0; c < 16; c++) w1[c] = hp[c];
+#pragma unroll
+    for (int k = 0; k < 19; k++) loc[k] = 0.f;
+    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < nvox; t += (size_t)gridDim.x * 256) {
         const int x = (int)(t % T), y = (int)((t / T) % T), z = (int)((t / ((size_t)T * T)) % T);
         const bool in = x >= halo && x < T - halo && y >= halo && y < T - halo && z >= halo && z < T - halo;
         const float d = out[t] - tgt[t];
         const float g = in ? 2.f * d * inv_count : 0.f;
-        uint4 w[2];
+        uint4 w[2], av4[2];
         unsigned short* wp = reinterpret_cast<unsigned short*>(w);
+        const unsigned short* ap = reinterpret_cast<const unsigned short*>(av4);
+        av4[0] = *reinterpret_cast<const uint4*>(act + t * 16);
+        av4[1] = *reinterpret_cast<const uint4*>(act + t * 16 + 8);
 #pragma unroll
         for (int c = 0; c < 16; c++) {
-            const unsigned short a = act[t * 16 + c];
-            const float av = cr_bf2f(a);
-            loc[c] = g * av;
-            wp[c] = cr_f2bf((a != 0 && (a & 0x8000u) == 0) ? g * hp[c] : 0.f);
+            const unsigned short a = ap[c];
+            loc[c] += g * cr_bf2f(a);
+            wp[c] = cr_f2bf((a != 0 && (a & 0x8000u) == 0) ? g * w1[c] : 0.f);
         }
         *reinterpret_cast<uint4*>(gact + t * 16) = w[0];
         *reinterpret_cast<uint4*>(gact + t * 16 + 8) = w[1];
-        loc[16] = g;
-        loc[17] = g * x0f[t];
-        loc[18] = in ? d * d * inv_count : 0.f;
+        loc[16] += g;
+        loc[17] += g * x0f[t];
+        loc[18] += in ? d * d * inv_count : 0.f;
     }
 #pragma unroll
-    for (int k = 0; k < 20; k++) red[k * 256 + threadIdx.x] = loc[k];
+    for (int k = 0; k < 19; k++) {
+        for (int o = 32; o > 0; o >>= 1) loc[k] += __shfl_xor(loc[k], o);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = loc[k];
+    }
     __syncthreads();
     if (threadIdx.x < 20) {
-        float s = 0.f;
-        for (int i = 0; i < 256; i++) s += red[threadIdx.x * 256 + i];
-        part[(size_t)blockIdx.x * 20 + threadIdx.x] = s;
+        const int k = threadIdx.x;
+        part[(size_t)blockIdx.x * 20 + k] = k < 19 ? ((red[0][k] + red[1][k]) + red[2][k]) + red[3][k] : 0.f;
     }
 }
 
-// Sum of nblk partial rows of width 20 (fixed order) into res[20].
-__global__ void k_cr_head_reduce(const float* __restrict__ part, int nblk, float* __restrict__ res) {
-    const int k = threadIdx.x;
-    if (k >= 20) return;
+// Sum of nblk partial rows of width 20 in FP64 into res[20] and, of the first
+// kHead, into the head's gradient: 32 threads a column, each a strided share
+// in order, then the 32 shares in order.
+__global__ void __launch_bounds__(640) k_cr_head_reduce(const float* __restrict__ part, int nblk, int nhead,
+                                                        float* __restrict__ res, float* __restrict__ ghead) {
+    __shared__ double red[32][20];
+    const int k = threadIdx.x % 20, q = threadIdx.x / 20;
     double s = 0.0;
-    for (int b = 0; b < nblk; b++) s += part[(size_t)b * 20 + k];
-    res[k] = (float)s;
+    for (int b = q; b < nblk; b += 32) s += part[(size_t)b * 20 + k];
+    red[q][k] = s;
+    __syncthreads();
+    if (q == 0) {
+        for (int i = 1; i < 32; i++) s += red[i][k];
+        res[k] = (float)s;
+        if (k < nhead) ghead[k] = (float)s;
+    }
 }
 
 // Adam (Kingma & Ba 2015) on the flat parameter vector with bias-corrected
@@ -555,8 +629,6 @@ struct utr_corr {
 
 namespace {
 
-constexpr int kCrG = 256;  // partial sums per weight gradient
-
 utr::CrShape cr_shape(int n, int e) {
     utr::CrShape s;
     s.n = n;
@@ -591,30 +663,52 @@ int cr_conv(utr_corr* c, int layer, bool fwd, const bf16_t* in, int in_cs, int i
     return UTR_OK;
 }
 
+// Weight-gradient launch of a layer over n cubes [0, e)^3: output blocks per
+// work-group, and partial sums G such that about kCrWgradWgs work-groups (two
+// to three resident per CU) share the voxel blocks evenly.
+constexpr int kCrWgradWgs = 768;
+int cr_wgrad_no(int cout) { return cout % 32 == 0 ? 2 : 1; }
+int cr_wgrad_groups(int cin, int cout, int n, int e) {
+    const int nb = n * ((e + utr::CR_WBX - 1) / utr::CR_WBX) * ((e + utr::CR_WBY - 1) / utr::CR_WBY) *
+                   ((e + utr::CR_WBZ - 1) / utr::CR_WBZ);
+    const int per_g = (cin / 16) * (cout / 16 / cr_wgrad_no(cout));
+    const int want = std::max(1, std::min(nb, (kCrWgradWgs + per_g - 1) / per_g));
+    const int each = (nb + want - 1) / want;
+    return (nb + each - 1) / each;
+}
+
+// dy is zero outside [lo, hi)^3.
 int cr_wgrad(utr_corr* c, int layer, const bf16_t* in, int in_cs, int in_co, const bf16_t* dy, int dy_cs,
-             int dy_co, utr::CrShape s) {
+             int dy_co, utr::CrShape s, int lo, int hi) {
     const CrLayer& Ly = c->L[layer];
-    utr::k_cr_wgrad<<<dim3(kCrG, Ly.cin / 16, Ly.cout / 16), 256, 0, c->st>>>(in, in_cs, in_co, Ly.cin, dy, dy_cs,
-                                                                            dy_co, Ly.cout, c->part.p, s, kCrG);
+    const size_t nw = (size_t)27 * Ly.cin * Ly.cout + Ly.cout;
+    const int no = cr_wgrad_no(Ly.cout), G = cr_wgrad_groups(Ly.cin, Ly.cout, s.n, hi - lo);
+    if ((size_t)G * nw > c->part.n) return set_err(UTR_E_STATE, "corrector: gradient workspace too small");
+    const dim3 grid(G, Ly.cin / 16, Ly.cout / 16 / no);
+    if (no == 2)
+        utr::k_cr_wgrad<2><<<grid, utr::CR_WT, 0, c->st>>>(in, in_cs, in_co, Ly.cin, dy, dy_cs, dy_co, Ly.cout,
+                                                           c->part.p, s, lo, hi, G);
+    else
+        utr::k_cr_wgrad<1><<<grid, utr::CR_WT, 0, c->st>>>(in, in_cs, in_co, Ly.cin, dy, dy_cs, dy_co, Ly.cout,
+                                                           c->part.p, s, lo, hi, G);
     UTR_HIP_TRY(hipGetLastError());
-    const size_t nw = (size_t)27 * Ly.cin * Ly.cout;
-    utr::k_cr_reduce<<<(unsigned)((nw + 255) / 256), 256, 0, c->st>>>(c->part.p, kCrG, nw, c->g.p + Ly.woff);
-    UTR_HIP_TRY(hipGetLastError());
-    const size_t nvox = (size_t)s.n * s.d * s.h * s.w;
-    utr::k_cr_bgrad<<<kCrG, 256, 0, c->st>>>(dy, dy_cs, dy_co, Ly.cout, nvox, c->part.p, kCrG);
-    UTR_HIP_TRY(hipGetLastError());
-    utr::k_cr_reduce<<<1, 256, 0, c->st>>>(c->part.p, kCrG, (size_t)Ly.cout, c->g.p + Ly.boff);
+    // weights and bias of a layer are contiguous in the gradient vector
+    utr::k_cr_reduce<<<(unsigned)((nw + 63) / 64), 256, 0, c->st>>>(c->part.p, G, nw, c->g.p + Ly.woff);
     UTR_HIP_TRY(hipGetLastError());
     return UTR_OK;
 }
 
 unsigned cr_blocks(size_t n) { return (unsigned)((n + 255) / 256); }
 
-// Largest 27 * cin * cout over the layers (the weight-gradient partials of
-// one layer; the bias partials need less).
-size_t cr_max_wsize() {
+// Floats the partial sums of any layer's weight gradient need, for any number
+// of crops up to the batch and any cube inside the layer's.
+size_t cr_part_size() {
     size_t mx = 0;
-    for (const auto& d : kCrLayers) mx = std::max(mx, (size_t)27 * d.cin * d.cout);
+    for (const auto& d : kCrLayers) {
+        const int per_g = (d.cin / 16) * (d.cout / 16 / cr_wgrad_no(d.cout));
+        const size_t nw = (size_t)27 * d.cin * d.cout + d.cout;
+        mx = std::max(mx, nw * (size_t)((kCrWgradWgs + per_g - 1) / per_g));
+    }
     return mx;
 }
 
@@ -629,7 +723,7 @@ int cr_alloc(utr_corr* c) {
         c->gd1b.alloc(n1 * 16), c->gd1a.alloc(n1 * 16), c->gC1.alloc(n1 * 48), c->gd2b.alloc(n2 * 32),
         c->gd2a.alloc(n2 * 32), c->gC2.alloc(n2 * 96), c->ge3b.alloc(n3 * 64), c->ge3a.alloc(n3 * 64),
         c->gp2.alloc(n3 * 32), c->ge2a.alloc(n2 * 32), c->gp1.alloc(n2 * 16), c->ge1a.alloc(n1 * 16),
-        c->part.alloc((size_t)kCrG * cr_max_wsize()), c->hpart.alloc(((n1 + 255) / 256) * 20), c->res.alloc(32),
+        c->part.alloc(cr_part_size()), c->hpart.alloc((size_t)utr::CR_HEADG * 20), c->res.alloc(32),
         c->crops_in.alloc(n1), c->crops_out.alloc(n1)};
     for (hipError_t x : e)
         if (x != hipSuccess)
@@ -682,45 +776,58 @@ int cr_backward(utr_corr* c, int nb, const float* tgt) {
     const utr::CrShape s1 = cr_shape(nb, T), s2 = cr_shape(nb, T / 2), s3 = cr_shape(nb, T / 4);
     const size_t n1 = (size_t)nb * T * T * T, n2 = n1 / 8, n3 = n1 / 64;
     const double cnt = (double)nb * c->tile * c->tile * c->tile;
-    const unsigned hb = cr_blocks(n1);
+    const unsigned hb = std::min(cr_blocks(n1), (unsigned)utr::CR_HEADG);
     int rc;
     utr::k_cr_head_bwd<<<hb, 256, 0, c->st>>>(c->d1b.p, c->x0f.p, c->out.p, tgt, c->w.p + c->headoff, T, c->halo, n1,
                                               (float)(1.0 / cnt), c->gd1b.p, c->hpart.p);
     UTR_HIP_TRY(hipGetLastError());
-    utr::k_cr_head_reduce<<<1, 64, 0, c->st>>>(c->hpart.p, (int)hb, c->res.p);
+    utr::k_cr_head_reduce<<<1, 640, 0, c->st>>>(c->hpart.p, (int)hb, kCrHead, c->res.p, c->g.p + c->headoff);
     UTR_HIP_TRY(hipGetLastError());
-    UTR_HIP_TRY(hipMemcpyAsync(c->g.p + c->headoff, c->res.p, sizeof(float) * kCrHead, hipMemcpyDeviceToDevice,
-                               c->st));
+    // The loss covers [halo, T - halo)^3, so each layer's output gradient is
+    // zero outside that cube grown by one voxel per convolution behind it
+    // (halved, rounded outwards, at each coarser level); its weight gradient
+    // contracts over that cube only.
+    struct Cube {
+        int lo, hi;
+    };
+    auto grow = [](Cube q, int e) { return Cube{std::max(0, q.lo - 1), std::min(e, q.hi + 1)}; };
+    auto half = [](Cube q) { return Cube{q.lo / 2, (q.hi + 1) / 2}; };
+    const Cube q9 = {c->halo, T - c->halo}, q8 = grow(q9, T), qC1 = grow(q8, T);
+    const Cube q7 = half(qC1), q6 = grow(q7, T / 2), qC2 = grow(q6, T / 2);
+    const Cube q5 = half(qC2), q4 = grow(q5, T / 4), qp2 = grow(q4, T / 4);
+    const Cube q3 = {std::min(qC2.lo, 2 * qp2.lo), std::max(qC2.hi, 2 * qp2.hi)};
+    const Cube q2 = grow(q3, T / 2), qp1 = grow(q2, T / 2);
+    const Cube q1 = {std::min(qC1.lo, 2 * qp1.lo), std::max(qC1.hi, 2 * qp1.hi)}, q0 = grow(q1, T);
     // d1b, d1a
-    if ((rc = cr_wgrad(c, 9, c->d1a.p, 16, 0, c->gd1b.p, 16, 0, s1))) return rc;
+    if ((rc = cr_wgrad(c, 9, c->d1a.p, 16, 0, c->gd1b.p, 16, 0, s1, q9.lo, q9.hi))) return rc;
     if ((rc = cr_conv(c, 9, false, c->gd1b.p, 16, 0, c->gd1a.p, 16, 0, c->d1a.p, 16, 0, s1))) return rc;
-    if ((rc = cr_wgrad(c, 8, c->C1.p, 48, 0, c->gd1a.p, 16, 0, s1))) return rc;
+    if ((rc = cr_wgrad(c, 8, c->C1.p, 48, 0, c->gd1a.p, 16, 0, s1, q8.lo, q8.hi))) return rc;
     if ((rc = cr_conv(c, 8, false, c->gd1a.p, 16, 0, c->gC1.p, 48, 0, c->C1.p, 48, 0, s1))) return rc;
     // up(d2b) -> d2b, d2a
     utr::k_cr_up_bwd<<<cr_blocks(n2 * 32), 256, 0, c->st>>>(c->gC1.p, 48, 0, c->gd2b.p, 32, 0, 32, s2);
-    if ((rc = cr_wgrad(c, 7, c->d2a.p, 32, 0, c->gd2b.p, 32, 0, s2))) return rc;
+    if ((rc = cr_wgrad(c, 7, c->d2a.p, 32, 0, c->gd2b.p, 32, 0, s2, q7.lo, q7.hi))) return rc;
     if ((rc = cr_conv(c, 7, false, c->gd2b.p, 32, 0, c->gd2a.p, 32, 0, c->d2a.p, 32, 0, s2))) return rc;
-    if ((rc = cr_wgrad(c, 6, c->C2.p, 96, 0, c->gd2a.p, 32, 0, s2))) return rc;
+    if ((rc = cr_wgrad(c, 6, c->C2.p, 96, 0, c->gd2a.p, 32, 0, s2, q6.lo, q6.hi))) return rc;
     if ((rc = cr_conv(c, 6, false, c->gd2a.p, 32, 0, c->gC2.p, 96, 0, c->C2.p, 96, 0, s2))) return rc;
     // up(e3b) -> e3b, e3a
     utr::k_cr_up_bwd<<<cr_blocks(n3 * 64), 256, 0, c->st>>>(c->gC2.p, 96, 0, c->ge3b.p, 64, 0, 64, s3);
-    if ((rc = cr_wgrad(c, 5, c->e3a.p, 64, 0, c->ge3b.p, 64, 0, s3))) return rc;
+    if ((rc = cr_wgrad(c, 5, c->e3a.p, 64, 0, c->ge3b.p, 64, 0, s3, q5.lo, q5.hi))) return rc;
     if ((rc = cr_conv(c, 5, false, c->ge3b.p, 64, 0, c->ge3a.p, 64, 0, c->e3a.p, 64, 0, s3))) return rc;
-    if ((rc = cr_wgrad(c, 4, c->p2.p, 32, 0, c->ge3a.p, 64, 0, s3))) return rc;
+    if ((rc = cr_wgrad(c, 4, c->p2.p, 32, 0, c->ge3a.p, 64, 0, s3, q4.lo, q4.hi))) return rc;
     if ((rc = cr_conv(c, 4, false, c->ge3a.p, 64, 0, c->gp2.p, 32, 0, nullptr, 0, 0, s3))) return rc;
     // pool(e2b) -> e2b (skip and pooled paths), e2a
     utr::k_cr_pool_bwd<<<cr_blocks(n2 * 32), 256, 0, c->st>>>(c->gC2.p, 96, 64, c->gp2.p, 32, 0, c->C2.p, 96, 64, 32,
                                                                s2);
-    if ((rc = cr_wgrad(c, 3, c->e2a.p, 32, 0, c->gC2.p, 96, 64, s2))) return rc;
+    if ((rc = cr_wgrad(c, 3, c->e2a.p, 32, 0, c->gC2.p, 96, 64, s2, q3.lo, q3.hi))) return rc;
     if ((rc = cr_conv(c, 3, false, c->gC2.p, 96, 64, c->ge2a.p, 32, 0, c->e2a.p, 32, 0, s2))) return rc;
-    if ((rc = cr_wgrad(c, 2, c->p1.p, 16, 0, c->ge2a.p, 32, 0, s2))) return rc;
+    if ((rc = cr_wgrad(c, 2, c->p1.p, 16, 0, c->ge2a.p, 32, 0, s2, q2.lo, q2.hi))) return rc;
     if ((rc = cr_conv(c, 2, false, c->ge2a.p, 32, 0, c->gp1.p, 16, 0, nullptr, 0, 0, s2))) return rc;
     // pool(e1b) -> e1b, e1a
     utr::k_cr_pool_bwd<<<cr_blocks(n1 * 16), 256, 0, c->st>>>(c->gC1.p, 48, 32, c->gp1.p, 16, 0, c->C1.p, 48, 32, 16,
                                                                s1);
-    if ((rc = cr_wgrad(c, 1, c->e1a.p, 16, 0, c->gC1.p, 48, 32, s1))) return rc;
+    if ((rc = cr_wgrad(c, 1, c->e1a.p, 16, 0, c->gC1.p, 48, 32, s1, q1.lo, q1.hi))) return rc;
     if ((rc = cr_conv(c, 1, false, c->gC1.p, 48, 32, c->ge1a.p, 16, 0, c->e1a.p, 16, 0, s1))) return rc;
-    if ((rc = cr_wgrad(c, 0, c->x0.p, 16, 0, c->ge1a.p, 16, 0, s1))) return rc;
+    if ((rc = cr_wgrad(c, 0, c->x0.p, 16, 0, c->ge1a.p, 16, 0, s1, q0.lo, q0.hi))) return rc;
     UTR_HIP_TRY(hipGetLastError());
     return UTR_OK;
 }

@@ -13,18 +13,16 @@
 // convolution to one channel plus alpha times the input) and the loss are
 // FP32.
 //
-// Convolution as an implicit GEMM: M = 16 consecutive x positions of one
-// output row, N = 16 output channels, K = (tap, input channel).  A work-group
-// owns a 16 x 4 x 4 (x, y, z) output block; each 16-channel slice of the
-// input block with its one-voxel halo (18 x 6 x 6) is staged in LDS, and two
-// taps form one K = 32 step.  The backward pass with respect to the input is
-// the same kernel with the taps mirrored and the channel roles swapped
-// (weights repacked once per step), its epilogue multiplying by the ReLU
-// mask of the layer below.  Weight gradients contract over voxels (K = 32:
-// two x rows of 16) with the input slice and the output-gradient block
-// both staged in LDS; each work-group sums a fixed subset of blocks and a
-// second kernel adds the partial sums in a fixed order, so gradients are
-// deterministic.
+// Convolution as an implicit GEMM: 16 output channels by 4 x 4 voxels, K =
+// (two taps, 16 input channels); each 16-channel slice of a work-group's input
+// block with its one-voxel halo is staged in LDS.  The backward pass with
+// respect to the input is the same kernel with the taps mirrored and the
+// channel roles swapped (weights repacked once per step), its epilogue
+// multiplying by the ReLU mask of the layer below.  Weight gradients contract
+// over voxels (K = 32: two x rows of 16) with the input slice and the
+// output-gradient block both staged in LDS; each work-group sums a fixed
+// subset of blocks and a second kernel adds the partial sums in a fixed order,
+// so gradients are deterministic.
 namespace utr {
 
 typedef short cr_s4 __attribute__((ext_vector_type(4)));
@@ -46,15 +44,10 @@ __host__ __device__ __forceinline__ unsigned short cr_f2bf(float f) {
     return (unsigned short)(u >> 16);
 }
 
-constexpr int CR_BX = 16, CR_BY = 4, CR_BZ = 4;        // output block of a work-group
-constexpr int CR_HX = CR_BX + 2, CR_HY = CR_BY + 2, CR_HZ = CR_BZ + 2;
-constexpr int CR_HVOX = CR_HX * CR_HY * CR_HZ;         // 648 staged voxels
-constexpr int CR_VS = 24;                              // LDS halves per staged voxel (16 + pad, 48 B)
-constexpr int CR_TSTEPS = 14;                          // K = 32 steps per 16-channel slice (27 taps + 1 zero)
+constexpr int CR_STEPS = 15;  // K = 32 steps per 16-channel slice: five (dy, dx) tap pairs x three dz
 
 struct CrShape {
     int n, d, h, w;         // batch and spatial extent
-    int tx, ty, tz;         // blocks along x, y, z
 };
 
 // Voxel index of (b, z, y, x).
@@ -62,95 +55,164 @@ __device__ __forceinline__ size_t cr_vox(const CrShape& s, int b, int z, int y, 
     return (((size_t)b * s.d + z) * s.h + y) * s.w + x;
 }
 
-// 3x3x3 convolution, stride 1, zero padding 1, NB blocks of 16 output
-// channels.  in: cin channels at channel offset in_co of rows of in_cs
-// halves; wf: BF16 fragments ((slice * 14 + step) * NB + nb) * 64 + lane,
-// 8 halves each; bias may be null; relu: max(0, .) after the bias; mask
-// (may be null): multiply by (mask > 0) at the output voxel and channel.
-template <int NB>
-__global__ void __launch_bounds__(256) k_cr_conv(const unsigned short* __restrict__ in, int in_cs, int in_co,
-                                                 int cin, const uint4* __restrict__ wf,
-                                                 const float* __restrict__ bias, int relu,
-                                                 const unsigned short* __restrict__ mask, int mask_cs,
-                                                 int mask_co, unsigned short* __restrict__ out, int out_cs,
-                                                 int out_co, CrShape s) {
-    __shared__ __align__(16) unsigned short xs[CR_HVOX * CR_VS];
-    int blk = blockIdx.x;
-    const int bx = blk % s.tx; blk /= s.tx;
-    const int by = blk % s.ty; blk /= s.ty;
-    const int bz = blk % s.tz;
-    const int b = blk / s.tz;
-    const int x0 = bx * CR_BX, y0 = by * CR_BY, z0 = bz * CR_BZ;
+// Four FP32 values rounded to BF16 (nearest even) as one 8-byte word.
+__device__ __forceinline__ uint2 cr_pack4(const float* v) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+    const f4 f = {v[0], v[1], v[2], v[3]};
+    return __builtin_bit_cast(uint2, __builtin_convertvector(f, b4));
+}
+
+struct CrConv {
+    const unsigned short* in;  // cin channels at channel offset in_co of rows of in_cs halves
+    int in_cs, in_co, cin;
+    const uint4* wf;           // weight fragments (k_cr_pack), nbt blocks of 16 output channels
+    int nbt;
+    const float* bias;         // may be null
+    int relu;                  // max(0, .) after the bias
+    const unsigned short* mask;  // may be null: multiply by (mask > 0) at the output voxel and channel
+    int mask_cs, mask_co;
+    unsigned short* out;
+    int out_cs, out_co;
+    CrShape s;
+};
+
+constexpr int CR_Z = 4;  // output planes of a work-group's block
+
+// 3x3x3 convolution, stride 1, zero padding 1, as an implicit GEMM: output
+// channels are the matrix rows, 16 voxels (a 4 x 4 patch of one z plane) its
+// columns, K = 32 is two (dy, dx) taps of 16 input channels.  A work-group of
+// four waves owns PX x PY patches in x and y, CR_Z planes in z and NB blocks of
+// 16 output channels (from blockIdx.y * NB); each wave takes PX PY / 4 patches
+// through all planes.
+//
+// What bounds it: for 16 channels the activations' traffic, for more the LDS
+// reads against the matrix cores.  Rows = channels lets a lane hold four
+// consecutive channels of one voxel, so a tile leaves in one 8-byte store per
+// lane (the transposed form stored 2 bytes at a time).  With the three dz of a
+// tap pair held in registers an input fragment read from LDS serves up to three
+// output planes: six reads for twelve matrix instructions a pair and patch
+// instead of one each.  Staged voxels keep their two 8-channel halves apart and
+// rows padded to an odd multiple of 64 bytes, so that the eight lanes of a read
+// phase fall on distinct banks.
+template <int PX, int PY, int NB>
+__global__ void __launch_bounds__(256) k_cr_conv(CrConv A) {
+    constexpr int HX = 4 * PX + 2, HY = 4 * PY + 2, HZ = CR_Z + 2;
+    constexpr int PITCH = 4 * PX + 4, HALF = HZ * HY * PITCH + 4;  // 16-byte units; HALF = 4 mod 8
+    constexpr int NV = HX * HY * HZ, P = PX * PY / 4;
+    constexpr int PER = (2 * NV + 255) / 256;
+    static_assert(PITCH % 8 == 4 && HALF % 8 == 4, "bank layout");
+    __shared__ __align__(16) uint4 xs[2 * HALF];
+    const CrShape s = A.s;
+    const int bxn = (s.w + 4 * PX - 1) / (4 * PX), byn = (s.h + 4 * PY - 1) / (4 * PY),
+              bzn = (s.d + CR_Z - 1) / CR_Z;
+    int tile, nb0;
+    if (!xcd_tile(bxn * byn * bzn * s.n, A.nbt / NB, tile, nb0)) return;
+    nb0 *= NB;
+    const int x0 = tile % bxn * (4 * PX); tile /= bxn;
+    const int y0 = tile % byn * (4 * PY); tile /= byn;
+    const int z0 = tile % bzn * CR_Z;
+    const int b = tile / bzn;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int m = lane & 15, kq = lane >> 4;
-    cr_f4 acc[CR_BY][NB];
+    const int m = lane & 15, kq = lane >> 4, mx = m & 3, my = m >> 2;
+    cr_f4 acc[P][CR_Z][NB];
 #pragma unroll
-    for (int r = 0; r < CR_BY; r++)
+    for (int p = 0; p < P; p++)
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) acc[r][nb] = cr_f4{0.f, 0.f, 0.f, 0.f};
-    const int nslice = cin >> 4;
+        for (int z = 0; z < CR_Z; z++)
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) acc[p][z][nb] = cr_f4{0.f, 0.f, 0.f, 0.f};
+    // this lane's fragment address for each tap pair (tap 9 of the last pair
+    // does not exist: it reads tap 8's voxel and is set to zero)
+    int fa[5];
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+        const int t = min(2 * q + (kq >> 1), 8);
+        fa[q] = (kq & 1) * HALF + (my + t / 3) * PITCH + mx + t % 3;
+    }
+    const int nslice = A.cin >> 4;
+    const uint4* wp = A.wf + lane;
     for (int c = 0; c < nslice; c++) {
-        __syncthreads();
-        for (int t = threadIdx.x; t < CR_HVOX * 2; t += 256) {
-            const int v = t >> 1, half = t & 1;
-            const int lx = v % CR_HX, ly = (v / CR_HX) % CR_HY, lz = v / (CR_HX * CR_HY);
-            const int gx = x0 - 1 + lx, gy = y0 - 1 + ly, gz = z0 - 1 + lz;
-            uint4 val = {0u, 0u, 0u, 0u};
-            if (gx >= 0 && gx < s.w && gy >= 0 && gy < s.h && gz >= 0 && gz < s.d)
-                val = *reinterpret_cast<const uint4*>(in + cr_vox(s, b, gz, gy, gx) * in_cs + in_co + c * 16 +
-                                                      half * 8);
-            *reinterpret_cast<uint4*>(xs + v * CR_VS + half * 8) = val;
+        uint4 val[PER];
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int t = (int)threadIdx.x + 256 * k, v = t >> 1;
+            const int gx = x0 - 1 + v % HX, gy = y0 - 1 + (v / HX) % HY, gz = z0 - 1 + v / (HX * HY);
+            val[k] = uint4{0u, 0u, 0u, 0u};
+            if (t < 2 * NV && (unsigned)gx < (unsigned)s.w && (unsigned)gy < (unsigned)s.h &&
+                (unsigned)gz < (unsigned)s.d)
+                val[k] = *reinterpret_cast<const uint4*>(A.in + cr_vox(s, b, gz, gy, gx) * A.in_cs + A.in_co +
+                                                         c * 16 + (t & 1) * 8);
+        }
+        if (c) __syncthreads();
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int t = (int)threadIdx.x + 256 * k, v = t >> 1;
+            if (t < 2 * NV) xs[(t & 1) * HALF + (v / HX) * PITCH + v % HX] = val[k];
         }
         __syncthreads();
-        const uint4* wc = wf + (size_t)c * CR_TSTEPS * NB * 64;
-#pragma unroll 2
-        for (int st = 0; st < CR_TSTEPS; st++) {
-            const int tap = 2 * st + (kq >> 1);
-            const bool live = tap < 27;
-            const int dz = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dx = tap % 3 - 1;
-            cr_b8 bfr[NB];
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) {
-                const uint4 q = wc[(st * NB + nb) * 64 + lane];
-                bfr[nb] = *reinterpret_cast<const cr_b8*>(&q);
-            }
+        for (int q = 0; q < 5; q++) {
+            cr_b8 w[3][NB];
 #pragma unroll
-            for (int r = 0; r < CR_BY; r++) {
-                uint4 a = {0u, 0u, 0u, 0u};
-                if (live) {
-                    const int v = ((wave + 1 + dz) * CR_HY + (r + 1 + dy)) * CR_HX + (m + 1 + dx);
-                    a = *reinterpret_cast<const uint4*>(xs + v * CR_VS + (kq & 1) * 8);
-                }
-                const cr_b8 afr = *reinterpret_cast<const cr_b8*>(&a);
+            for (int dz = 0; dz < 3; dz++)
 #pragma unroll
                 for (int nb = 0; nb < NB; nb++)
-                    acc[r][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr, bfr[nb], acc[r][nb], 0, 0, 0);
+                    w[dz][nb] = __builtin_bit_cast(
+                        cr_b8, wp[(size_t)(((c * 5 + q) * 3 + dz) * A.nbt + nb0 + nb) * 64]);
+#pragma unroll
+            for (int p = 0; p < P; p++) {
+                const int pid = wave * P + p;
+                const uint4* r = xs + fa[q] + (pid / PX) * 4 * PITCH + (pid % PX) * 4;
+#pragma unroll
+                for (int zz = 0; zz < HZ; zz++) {
+                    uint4 f = r[zz * HY * PITCH];
+                    if (q == 4 && kq >= 2) f = uint4{0u, 0u, 0u, 0u};
+                    const cr_b8 xf = __builtin_bit_cast(cr_b8, f);
+#pragma unroll
+                    for (int dz = 0; dz < 3; dz++) {
+                        const int z = zz - dz;
+                        if (z < 0 || z >= CR_Z) continue;
+#pragma unroll
+                        for (int nb = 0; nb < NB; nb++)
+                            acc[p][z][nb] =
+                                __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[dz][nb], xf, acc[p][z][nb], 0, 0, 0);
+                    }
+                }
             }
         }
     }
-    // D[row = 4 kq + i][col = m]: voxel x0 + 4 kq + i, channel nb * 16 + m
-    const int z = z0 + wave;
-    if (z >= s.d) return;
+    // D[row = 4 kq + i][col = m]: channel 16 nb + 4 kq + i of the patch's voxel m
 #pragma unroll
-    for (int r = 0; r < CR_BY; r++) {
-        const int y = y0 + r;
-        if (y >= s.h) continue;
+    for (int p = 0; p < P; p++) {
+        const int pid = wave * P + p;
+        const int x = x0 + (pid % PX) * 4 + mx, y = y0 + (pid / PX) * 4 + my;
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
-            const int ch = nb * 16 + m;
-            const float bv = bias ? bias[ch] : 0.f;
+        for (int z = 0; z < CR_Z; z++) {
+            if (x >= s.w || y >= s.h || z0 + z >= s.d) continue;
+            const size_t vox = cr_vox(s, b, z0 + z, y, x);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int x = x0 + 4 * kq + i;
-                if (x >= s.w) continue;
-                const size_t vox = cr_vox(s, b, z, y, x);
-                float val = acc[r][nb][i] + bv;
-                if (relu) val = fmaxf(val, 0.f);
-                if (mask) {
-                    const unsigned short mv = mask[vox * mask_cs + mask_co + ch];
-                    if (!(mv != 0 && (mv & 0x8000u) == 0)) val = 0.f;
+            for (int nb = 0; nb < NB; nb++) {
+                const int ch = (nb0 + nb) * 16 + 4 * kq;
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[i] = acc[p][z][nb][i];
+                if (A.bias) {
+                    const float4 bv = *reinterpret_cast<const float4*>(A.bias + ch);
+                    v[0] += bv.x; v[1] += bv.y; v[2] += bv.z; v[3] += bv.w;
                 }
-                out[vox * out_cs + out_co + ch] = cr_f2bf(val);
+                if (A.relu) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) v[i] = fmaxf(v[i], 0.f);
+                }
+                if (A.mask) {
+                    const uint2 mv = *reinterpret_cast<const uint2*>(A.mask + vox * A.mask_cs + A.mask_co + ch);
+                    const unsigned h[4] = {mv.x & 0xffffu, mv.x >> 16, mv.y & 0xffffu, mv.y >> 16};
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        if (!(h[i] != 0 && (h[i] & 0x8000u) == 0)) v[i] = 0.f;
+                }
+                *reinterpret_cast<uint2*>(A.out + vox * A.out_cs + A.out_co + ch) = cr_pack4(v);
             }
         }
     }
@@ -510,30 +572,31 @@ __global__ void k_cr_adam(float* __restrict__ w, const float* __restrict__ g, fl
 }
 
 // BF16 MFMA fragments of one layer's weights W[27][cin][cout] (FP32):
-// forward (fwd != 0: K = (tap, ci), N = co) or input gradient (K = (mirrored
-// tap, co), N = ci).  Fragment ((slice * 14 + step) * NB + nb) * 64 + lane
-// holds, for lane (n = lane % 16, kq = lane / 16), the 8 values of tap
-// 2 step + kq / 2, K channels slice * 16 + (kq % 2) * 8 + j, N channel
-// nb * 16 + n (zero for the 28th tap).
+// forward (fwd != 0: K = (tap, ci), rows = co) or input gradient (K =
+// (mirrored tap, co), rows = ci).  Fragment (((slice * 5 + pair) * 3 + dz) * NB
+// + nb) * 64 + lane holds, for lane (n = lane % 16, kq = lane / 16), the 8
+// values of tap 9 dz + 2 pair + kq / 2, K channels slice * 16 + (kq % 2) * 8
+// + j, output channel nb * 16 + n (zero where 2 pair + kq / 2 = 9).
 __global__ void k_cr_pack(const float* __restrict__ W, int cin, int cout, int fwd, uint4* __restrict__ wf) {
     const int kin = fwd ? cin : cout, nout = fwd ? cout : cin;
     const int NB = nout / 16, ns = kin / 16;
-    const size_t total = (size_t)ns * CR_TSTEPS * NB * 64;
+    const size_t total = (size_t)ns * CR_STEPS * NB * 64;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= total) return;
     const int lane = (int)(t % 64);
     size_t r = t / 64;
     const int nb = (int)(r % NB); r /= NB;
-    const int st = (int)(r % CR_TSTEPS);
-    const int c = (int)(r / CR_TSTEPS);
+    const int dz = (int)(r % 3); r /= 3;
+    const int pair = (int)(r % 5);
+    const int c = (int)(r / 5);
     const int n = lane & 15, kq = lane >> 4;
-    const int tap = 2 * st + (kq >> 1);
+    const int t9 = 2 * pair + (kq >> 1), tap = 9 * dz + t9;
     uint4 q;
     unsigned short* h = reinterpret_cast<unsigned short*>(&q);
     for (int j = 0; j < 8; j++) {
         const int k = c * 16 + (kq & 1) * 8 + j, o = nb * 16 + n;
         float val = 0.f;
-        if (tap < 27) val = fwd ? W[((size_t)tap * cin + k) * cout + o] : W[((size_t)(26 - tap) * cin + o) * cout + k];
+        if (t9 < 9) val = fwd ? W[((size_t)tap * cin + k) * cout + o] : W[((size_t)(26 - tap) * cin + o) * cout + k];
         h[j] = cr_f2bf(val);
     }
     wf[t] = q;
@@ -633,34 +696,46 @@ utr::CrShape cr_shape(int n, int e) {
     utr::CrShape s;
     s.n = n;
     s.d = s.h = s.w = e;
-    s.tx = (e + utr::CR_BX - 1) / utr::CR_BX;
-    s.ty = (e + utr::CR_BY - 1) / utr::CR_BY;
-    s.tz = (e + utr::CR_BZ - 1) / utr::CR_BZ;
     return s;
+}
+
+// Blocks of 16 x 8 voxels in x and y where they make at least two work-groups
+// per CU, 8 x 8 otherwise (the coarsest level of a few crops).
+template <int PX, int PY>
+int cr_conv_launch(utr_corr* c, const utr::CrConv& A) {
+    const auto& s = A.s;
+    const unsigned tiles = (unsigned)(s.n * ((s.w + 4 * PX - 1) / (4 * PX)) * ((s.h + 4 * PY - 1) / (4 * PY)) *
+                                      ((s.d + utr::CR_Z - 1) / utr::CR_Z));
+    const int nb = A.nbt % 3 == 0 ? 3 : A.nbt % 2 == 0 ? 2 : 1;
+    const unsigned grid = utr::xcd_grid(tiles * (unsigned)(A.nbt / nb));
+    if (nb == 3) utr::k_cr_conv<PX, PY, 3><<<grid, 256, 0, c->st>>>(A);
+    else if (nb == 2) utr::k_cr_conv<PX, PY, 2><<<grid, 256, 0, c->st>>>(A);
+    else utr::k_cr_conv<PX, PY, 1><<<grid, 256, 0, c->st>>>(A);
+    UTR_HIP_TRY(hipGetLastError());
+    return UTR_OK;
 }
 
 int cr_conv(utr_corr* c, int layer, bool fwd, const bf16_t* in, int in_cs, int in_co, bf16_t* out, int out_cs,
             int out_co, const bf16_t* mask, int mask_cs, int mask_co, utr::CrShape s) {
     const CrLayer& Ly = c->L[layer];
-    const int kin = fwd ? Ly.cin : Ly.cout, nout = fwd ? Ly.cout : Ly.cin;
-    const unsigned grid = (unsigned)(s.n * s.tz * s.ty * s.tx);
-    const uint4* wf = fwd ? Ly.wf.p : Ly.wb.p;
-    const float* bias = fwd ? c->w.p + Ly.boff : nullptr;
-    const int relu = fwd ? 1 : 0;
-#define CR_CONV(NB)                                                                                           \
-    utr::k_cr_conv<NB><<<grid, 256, 0, c->st>>>(in, in_cs, in_co, kin, wf, bias, relu, mask, mask_cs, mask_co, \
-                                                out, out_cs, out_co, s)
-    switch (nout / 16) {
-        case 1: CR_CONV(1); break;
-        case 2: CR_CONV(2); break;
-        case 3: CR_CONV(3); break;
-        case 4: CR_CONV(4); break;
-        case 6: CR_CONV(6); break;
-        default: return set_err(UTR_E_INVALID, "corrector: unsupported channel count");
-    }
-#undef CR_CONV
-    UTR_HIP_TRY(hipGetLastError());
-    return UTR_OK;
+    utr::CrConv A;
+    A.in = in;
+    A.in_cs = in_cs;
+    A.in_co = in_co;
+    A.cin = fwd ? Ly.cin : Ly.cout;
+    A.nbt = (fwd ? Ly.cout : Ly.cin) / 16;
+    A.wf = fwd ? Ly.wf.p : Ly.wb.p;
+    A.bias = fwd ? c->w.p + Ly.boff : nullptr;
+    A.relu = fwd ? 1 : 0;
+    A.mask = mask;
+    A.mask_cs = mask_cs;
+    A.mask_co = mask_co;
+    A.out = out;
+    A.out_cs = out_cs;
+    A.out_co = out_co;
+    A.s = s;
+    const long big = (long)s.n * ((s.w + 15) / 16) * ((s.h + 7) / 8) * ((s.d + 3) / 4);
+    return big >= 512 ? cr_conv_launch<4, 2>(c, A) : cr_conv_launch<2, 2>(c, A);
 }
 
 // Weight-gradient launch of a layer over n cubes [0, e)^3: output blocks per
@@ -735,7 +810,7 @@ int cr_alloc(utr_corr* c) {
 int cr_repack(utr_corr* c) {
     for (int l = 0; l < 10; l++) {
         CrLayer& Ly = c->L[l];
-        const size_t nf = (size_t)(Ly.cin / 16) * utr::CR_TSTEPS * (Ly.cout / 16) * 64;
+        const size_t nf = (size_t)(Ly.cin / 16) * utr::CR_STEPS * (Ly.cout / 16) * 64;
         utr::k_cr_pack<<<cr_blocks(nf), 256, 0, c->st>>>(c->w.p + Ly.woff, Ly.cin, Ly.cout, 1, Ly.wf.p);
         UTR_HIP_TRY(hipGetLastError());
         utr::k_cr_pack<<<cr_blocks(nf), 256, 0, c->st>>>(c->w.p + Ly.woff, Ly.cin, Ly.cout, 0, Ly.wb.p);
@@ -908,8 +983,8 @@ int utr_corr_create(int tile, int halo, int batch, unsigned long long seed, utr_
     if (c->w.alloc(c->np) || c->g.alloc(c->np) || c->m.alloc(c->np) || c->v.alloc(c->np))
         return fail(set_err(UTR_E_NOMEM, "corrector: parameter allocation failed"));
     for (int l = 0; l < 10; l++) {
-        const size_t nf = (size_t)(c->L[l].cin / 16) * utr::CR_TSTEPS * (c->L[l].cout / 16) * 64;
-        const size_t nb = (size_t)(c->L[l].cout / 16) * utr::CR_TSTEPS * (c->L[l].cin / 16) * 64;
+        const size_t nf = (size_t)(c->L[l].cin / 16) * utr::CR_STEPS * (c->L[l].cout / 16) * 64;
+        const size_t nb = (size_t)(c->L[l].cout / 16) * utr::CR_STEPS * (c->L[l].cin / 16) * 64;
         if (c->L[l].wf.alloc(nf) || c->L[l].wb.alloc(nb))
             return fail(set_err(UTR_E_NOMEM, "corrector: fragment allocation failed"));
     }

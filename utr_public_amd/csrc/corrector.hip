@@ -63,28 +63,101 @@ __device__ __forceinline__ uint2 cr_pack4(const float* v) {
     return __builtin_bit_cast(uint2, __builtin_convertvector(f, b4));
 }
 
+__device__ __forceinline__ float cr_bflo(unsigned w) { return __builtin_bit_cast(float, w << 16); }
+__device__ __forceinline__ float cr_bfhi(unsigned w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
+// v[i] = 0 where the BF16 activation i of w is not positive.
+__device__ __forceinline__ void cr_relu_mask(float* v, uint2 w) {
+    const unsigned h[4] = {w.x & 0xffffu, w.x >> 16, w.y & 0xffffu, w.y >> 16};
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        if (!(h[i] != 0 && (h[i] & 0x8000u) == 0)) v[i] = 0.f;
+}
+
+// Channels of a layer's input: the first nup 16-channel slices are a coarser
+// tensor read at half the coordinates (nearest 2x upsampling), the others one
+// at the layer's own resolution.  Both are dense, channels last.
+struct CrIn {
+    const unsigned short* up;
+    int up_c, nup;             // channels and 16-channel slices of the coarser tensor
+    const unsigned short* p;
+    int c;                     // channels of p
+};
+
+// 16 bytes (half 0 or 1) of 16-channel slice c at voxel (z, y, x).
+__device__ __forceinline__ uint4 cr_load(const CrIn& I, const CrShape& s, int c, int half, int b, int z, int y, int x) {
+    if (c < I.nup)
+        return *reinterpret_cast<const uint4*>(
+            I.up + ((((size_t)b * (s.d >> 1) + (z >> 1)) * (s.h >> 1) + (y >> 1)) * (s.w >> 1) + (x >> 1)) * I.up_c +
+            c * 16 + half * 8);
+    return *reinterpret_cast<const uint4*>(I.p + cr_vox(s, b, z, y, x) * I.c + (c - I.nup) * 16 + half * 8);
+}
+
+// The network's FP32 input: crops [b][T][T][T] (ntx = 0), or crop first + b of
+// the tile grid of a volume, covering [t0 - halo, t0 + tile + halo) per axis
+// with zeros outside the volume; times scale.
+struct CrVol {
+    const float* p;
+    float scale;
+    int nx, ny, nz, tile, halo, ntx, nty, first;
+};
+__device__ __forceinline__ bool cr_vol_at(const CrVol& V, int T, int b, int z, int y, int x, size_t& at) {
+    if (V.ntx == 0) {
+        at = (((size_t)b * T + z) * T + y) * T + x;
+        return true;
+    }
+    const int id = V.first + b;
+    const int gx = id % V.ntx * V.tile - V.halo + x, gy = id / V.ntx % V.nty * V.tile - V.halo + y,
+              gz = id / (V.ntx * V.nty) * V.tile - V.halo + z;
+    at = ((size_t)gz * V.ny + gy) * V.nx + gx;
+    return (unsigned)gx < (unsigned)V.nx && (unsigned)gy < (unsigned)V.ny && (unsigned)gz < (unsigned)V.nz;
+}
+
+// What follows a convolution.
+enum CrEpi {
+    CR_ACT,    // bias, ReLU; BF16 out
+    CR_POOL,   // the same, and its 2x2x2 average to out2 at half resolution
+    CR_GRAD,   // BF16 out, times (mask > 0) if a mask is given
+    CR_SPLIT,  // gradient of an upsampled-and-concatenated input: blocks below nup summed over 2x2x2 to out2 (mask2
+               // > 0 at half resolution), the others to out (mask > 0)
+    CR_HEAD,   // bias, ReLU and the head: FP32 alpha x + b1 + sum_c w1[c] act[c] to vout
+    CR_LOSS    // the same compared with the target: loss, head gradients (part) and the gradient of act to out
+};
+
 struct CrConv {
-    const unsigned short* in;  // cin channels at channel offset in_co of rows of in_cs halves
-    int in_cs, in_co, cin;
+    CrIn in;
+    int cin;
     const uint4* wf;           // weight fragments (k_cr_pack), nbt blocks of 16 output channels
     int nbt;
-    const float* bias;         // may be null
-    int relu;                  // max(0, .) after the bias
-    const unsigned short* mask;  // may be null: multiply by (mask > 0) at the output voxel and channel
-    int mask_cs, mask_co;
-    unsigned short* out;
-    int out_cs, out_co;
+    const float* bias;
+    unsigned short* out;       // out_c channels
+    int out_c;
+    unsigned short* out2;      // CR_POOL, CR_SPLIT
+    int out2_c, nup;
+    const unsigned short *mask, *mask2;  // same channels as out, out2
     CrShape s;
+    int lo, hi;                // outputs are formed in the cube [lo, hi)^3 (even bounds for CR_POOL and CR_SPLIT)
+    int ilo, ihi;              // the input is zero outside [ilo, ihi)^3
+    // CR_HEAD, CR_LOSS
+    CrVol vol;
+    const float* hp;           // {w1[16], b1, alpha}
+    float* vout;
+    float oscale;              // CR_HEAD: output = value * oscale
+    const float* tgt;
+    float tscale, inv_count;
+    float* part;               // [work-group][20]: {dw1[16], db1, dalpha, loss, 0}
 };
 
 constexpr int CR_Z = 4;  // output planes of a work-group's block
 
+// Waves per SIMD the register budget is set for.
+constexpr int cr_occ(int nb) { return nb == 3 ? 3 : 4; }
+
 // 3x3x3 convolution, stride 1, zero padding 1, as an implicit GEMM: output
 // channels are the matrix rows, 16 voxels (a 4 x 4 patch of one z plane) its
-// columns, K = 32 is two (dy, dx) taps of 16 input channels.  A work-group of
-// four waves owns PX x PY patches in x and y, CR_Z planes in z and NB blocks of
-// 16 output channels (from blockIdx.y * NB); each wave takes PX PY / 4 patches
-// through all planes.
+// columns, K = 32 is two (dy, dx) taps of 16 input channels.  A work-group
+// owns PX x PY patches in x and y, CR_Z planes in z and NB blocks of 16 output
+// channels; each of its PX PY waves takes one patch through all planes (two
+// patches a wave spilled registers at four waves per SIMD).
 //
 // What bounds it: for 16 channels the activations' traffic, for more the LDS
 // reads against the matrix cores.  Rows = channels lets a lane hold four
@@ -95,40 +168,44 @@ constexpr int CR_Z = 4;  // output planes of a work-group's block
 // instead of one each.  Staged voxels keep their two 8-channel halves apart and
 // rows padded to an odd multiple of 64 bytes, so that the eight lanes of a read
 // phase fall on distinct banks.
-template <int PX, int PY, int NB>
-__global__ void __launch_bounds__(256) k_cr_conv(CrConv A) {
+//
+// The passes around a convolution are its own loads and stores (CrIn, CrEpi):
+// upsampling and concatenation, pooling, their adjoints, the head and the loss
+// each read and wrote whole activations in kernels of their own before.
+template <int PX, int PY, int NB, int EPI>
+__global__ void __launch_bounds__(64 * PX * PY, cr_occ(NB)) k_cr_conv(CrConv A) {
     constexpr int HX = 4 * PX + 2, HY = 4 * PY + 2, HZ = CR_Z + 2;
     constexpr int PITCH = 4 * PX + 4, HALF = HZ * HY * PITCH + 4;  // 16-byte units; HALF = 4 mod 8
-    constexpr int NV = HX * HY * HZ, P = PX * PY / 4;
-    constexpr int PER = (2 * NV + 255) / 256;
+    constexpr int NV = HX * HY * HZ, NT = 64 * PX * PY;
+    constexpr int PER = (2 * NV + NT - 1) / NT;
     static_assert(PITCH % 8 == 4 && HALF % 8 == 4, "bank layout");
     __shared__ __align__(16) uint4 xs[2 * HALF];
     const CrShape s = A.s;
-    const int bxn = (s.w + 4 * PX - 1) / (4 * PX), byn = (s.h + 4 * PY - 1) / (4 * PY),
-              bzn = (s.d + CR_Z - 1) / CR_Z;
+    const int ext = A.hi - A.lo;
+    const int bxn = (ext + 4 * PX - 1) / (4 * PX), byn = (ext + 4 * PY - 1) / (4 * PY),
+              bzn = (ext + CR_Z - 1) / CR_Z;
     int tile, nb0;
     if (!xcd_tile(bxn * byn * bzn * s.n, A.nbt / NB, tile, nb0)) return;
+    [[maybe_unused]] const int wg = tile;
     nb0 *= NB;
-    const int x0 = tile % bxn * (4 * PX); tile /= bxn;
-    const int y0 = tile % byn * (4 * PY); tile /= byn;
-    const int z0 = tile % bzn * CR_Z;
+    const int x0 = A.lo + tile % bxn * (4 * PX); tile /= bxn;
+    const int y0 = A.lo + tile % byn * (4 * PY); tile /= byn;
+    const int z0 = A.lo + tile % bzn * CR_Z;
     const int b = tile / bzn;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int m = lane & 15, kq = lane >> 4, mx = m & 3, my = m >> 2;
-    cr_f4 acc[P][CR_Z][NB];
+    cr_f4 acc[CR_Z][NB];
 #pragma unroll
-    for (int p = 0; p < P; p++)
+    for (int z = 0; z < CR_Z; z++)
 #pragma unroll
-        for (int z = 0; z < CR_Z; z++)
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) acc[p][z][nb] = cr_f4{0.f, 0.f, 0.f, 0.f};
+        for (int nb = 0; nb < NB; nb++) acc[z][nb] = cr_f4{0.f, 0.f, 0.f, 0.f};
     // this lane's fragment address for each tap pair (tap 9 of the last pair
     // does not exist: it reads tap 8's voxel and is set to zero)
     int fa[5];
 #pragma unroll
     for (int q = 0; q < 5; q++) {
         const int t = min(2 * q + (kq >> 1), 8);
-        fa[q] = (kq & 1) * HALF + (my + t / 3) * PITCH + mx + t % 3;
+        fa[q] = (kq & 1) * HALF + (wave / PX * 4 + my + t / 3) * PITCH + wave % PX * 4 + mx + t % 3;
     }
     const int nslice = A.cin >> 4;
     const uint4* wp = A.wf + lane;
@@ -136,18 +213,16 @@ __global__ void __launch_bounds__(256) k_cr_conv(CrConv A) {
         uint4 val[PER];
 #pragma unroll
         for (int k = 0; k < PER; k++) {
-            const int t = (int)threadIdx.x + 256 * k, v = t >> 1;
+            const int t = (int)threadIdx.x + NT * k, v = t >> 1;
             const int gx = x0 - 1 + v % HX, gy = y0 - 1 + (v / HX) % HY, gz = z0 - 1 + v / (HX * HY);
             val[k] = uint4{0u, 0u, 0u, 0u};
-            if (t < 2 * NV && (unsigned)gx < (unsigned)s.w && (unsigned)gy < (unsigned)s.h &&
-                (unsigned)gz < (unsigned)s.d)
-                val[k] = *reinterpret_cast<const uint4*>(A.in + cr_vox(s, b, gz, gy, gx) * A.in_cs + A.in_co +
-                                                         c * 16 + (t & 1) * 8);
+            if (t < 2 * NV && min(gx, min(gy, gz)) >= A.ilo && max(gx, max(gy, gz)) < A.ihi)
+                val[k] = cr_load(A.in, s, c, t & 1, b, gz, gy, gx);
         }
         if (c) __syncthreads();
 #pragma unroll
         for (int k = 0; k < PER; k++) {
-            const int t = (int)threadIdx.x + 256 * k, v = t >> 1;
+            const int t = (int)threadIdx.x + NT * k, v = t >> 1;
             if (t < 2 * NV) xs[(t & 1) * HALF + (v / HX) * PITCH + v % HX] = val[k];
         }
         __syncthreads();
@@ -160,60 +235,196 @@ __global__ void __launch_bounds__(256) k_cr_conv(CrConv A) {
                 for (int nb = 0; nb < NB; nb++)
                     w[dz][nb] = __builtin_bit_cast(
                         cr_b8, wp[(size_t)(((c * 5 + q) * 3 + dz) * A.nbt + nb0 + nb) * 64]);
+            const uint4* r = xs + fa[q];
 #pragma unroll
-            for (int p = 0; p < P; p++) {
-                const int pid = wave * P + p;
-                const uint4* r = xs + fa[q] + (pid / PX) * 4 * PITCH + (pid % PX) * 4;
+            for (int zz = 0; zz < HZ; zz++) {
+                uint4 f = r[zz * HY * PITCH];
+                if (q == 4 && kq >= 2) f = uint4{0u, 0u, 0u, 0u};
+                const cr_b8 xf = __builtin_bit_cast(cr_b8, f);
 #pragma unroll
-                for (int zz = 0; zz < HZ; zz++) {
-                    uint4 f = r[zz * HY * PITCH];
-                    if (q == 4 && kq >= 2) f = uint4{0u, 0u, 0u, 0u};
-                    const cr_b8 xf = __builtin_bit_cast(cr_b8, f);
+                for (int dz = 0; dz < 3; dz++) {
+                    const int z = zz - dz;
+                    if (z < 0 || z >= CR_Z) continue;
 #pragma unroll
-                    for (int dz = 0; dz < 3; dz++) {
-                        const int z = zz - dz;
-                        if (z < 0 || z >= CR_Z) continue;
-#pragma unroll
-                        for (int nb = 0; nb < NB; nb++)
-                            acc[p][z][nb] =
-                                __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[dz][nb], xf, acc[p][z][nb], 0, 0, 0);
-                    }
+                    for (int nb = 0; nb < NB; nb++)
+                        acc[z][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[dz][nb], xf, acc[z][nb], 0, 0, 0);
                 }
             }
         }
     }
     // D[row = 4 kq + i][col = m]: channel 16 nb + 4 kq + i of the patch's voxel m
+    [[maybe_unused]] float hw[4], hb1 = 0.f, halpha = 0.f, loc[4] = {0.f, 0.f, 0.f, 0.f}, lg = 0.f, lgx = 0.f, ll = 0.f;
+    if constexpr (EPI == CR_HEAD || EPI == CR_LOSS) {
 #pragma unroll
-    for (int p = 0; p < P; p++) {
-        const int pid = wave * P + p;
-        const int x = x0 + (pid % PX) * 4 + mx, y = y0 + (pid / PX) * 4 + my;
+        for (int i = 0; i < 4; i++) hw[i] = A.hp[4 * kq + i];
+        hb1 = A.hp[16];
+        halpha = A.hp[17];
+    }
+    const int x = x0 + wave % PX * 4 + mx, y = y0 + wave / PX * 4 + my;
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) {
+        const int ch = (nb0 + nb) * 16 + 4 * kq;
+        float4 bv = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (EPI != CR_GRAD && EPI != CR_SPLIT) bv = *reinterpret_cast<const float4*>(A.bias + ch);
+        float sum[4];  // running 2x2x2 sum of a pair of planes
 #pragma unroll
         for (int z = 0; z < CR_Z; z++) {
-            if (x >= s.w || y >= s.h || z0 + z >= s.d) continue;
+            const bool in = x < A.hi && y < A.hi && z0 + z < A.hi;
             const size_t vox = cr_vox(s, b, z0 + z, y, x);
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) {
-                const int ch = (nb0 + nb) * 16 + 4 * kq;
-                float v[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) v[i] = acc[p][z][nb][i];
-                if (A.bias) {
-                    const float4 bv = *reinterpret_cast<const float4*>(A.bias + ch);
-                    v[0] += bv.x; v[1] += bv.y; v[2] += bv.z; v[3] += bv.w;
-                }
-                if (A.relu) {
-#pragma unroll
-                    for (int i = 0; i < 4; i++) v[i] = fmaxf(v[i], 0.f);
-                }
-                if (A.mask) {
-                    const uint2 mv = *reinterpret_cast<const uint2*>(A.mask + vox * A.mask_cs + A.mask_co + ch);
-                    const unsigned h[4] = {mv.x & 0xffffu, mv.x >> 16, mv.y & 0xffffu, mv.y >> 16};
-#pragma unroll
-                    for (int i = 0; i < 4; i++)
-                        if (!(h[i] != 0 && (h[i] & 0x8000u) == 0)) v[i] = 0.f;
-                }
-                *reinterpret_cast<uint2*>(A.out + vox * A.out_cs + A.out_co + ch) = cr_pack4(v);
+            float v[4] = {acc[z][nb][0] + bv.x, acc[z][nb][1] + bv.y, acc[z][nb][2] + bv.z,
+                          acc[z][nb][3] + bv.w};
+            if constexpr (EPI == CR_GRAD) {
+                if (!in) continue;
+                if (A.mask) cr_relu_mask(v, *reinterpret_cast<const uint2*>(A.mask + vox * A.out_c + ch));
+                *reinterpret_cast<uint2*>(A.out + vox * A.out_c + ch) = cr_pack4(v);
+                continue;
             }
+            const bool pooled = EPI == CR_POOL || (EPI == CR_SPLIT && nb0 + nb < A.nup);
+            if constexpr (EPI != CR_SPLIT) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) v[i] = fmaxf(v[i], 0.f);
+                const uint2 h = cr_pack4(v);
+                if constexpr (EPI == CR_ACT || EPI == CR_POOL)
+                    if (in) *reinterpret_cast<uint2*>(A.out + vox * A.out_c + ch) = h;
+                // what follows sees the rounded activations
+                v[0] = cr_bflo(h.x); v[1] = cr_bfhi(h.x); v[2] = cr_bflo(h.y); v[3] = cr_bfhi(h.y);
+            } else if (!pooled && in) {
+                const int o = ch - A.nup * 16;
+                cr_relu_mask(v, *reinterpret_cast<const uint2*>(A.mask + vox * A.out_c + o));
+                *reinterpret_cast<uint2*>(A.out + vox * A.out_c + o) = cr_pack4(v);
+            }
+            if constexpr (EPI == CR_POOL || EPI == CR_SPLIT) {
+                if (!pooled) continue;  // uniform
+                // x pairs are lanes m and m ^ 1, y pairs m and m ^ 4, z
+                // pairs two of this lane's planes; the cube's bounds are
+                // even, so a pair is inside it or outside as a whole
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    v[i] += __shfl_xor(v[i], 1);
+                    v[i] += __shfl_xor(v[i], 4);
+                    sum[i] = (z & 1) ? sum[i] + v[i] : v[i];
+                }
+                if ((z & 1) && in && ((mx | my) & 1) == 0) {
+                    const size_t vc = (((size_t)b * (s.d >> 1) + ((z0 + z) >> 1)) * (s.h >> 1) + (y >> 1)) *
+                                          (s.w >> 1) + (x >> 1);
+                    if constexpr (EPI == CR_POOL) {
+#pragma unroll
+                        for (int i = 0; i < 4; i++) sum[i] *= 0.125f;
+                    } else {
+                        cr_relu_mask(sum, *reinterpret_cast<const uint2*>(A.mask2 + vc * A.out2_c + ch));
+                    }
+                    *reinterpret_cast<uint2*>(A.out2 + vc * A.out2_c + ch) = cr_pack4(sum);
+                }
+            }
+            if constexpr (EPI == CR_HEAD || EPI == CR_LOSS) {
+                float o = hw[0] * v[0] + hw[1] * v[1] + hw[2] * v[2] + hw[3] * v[3];
+                o += __shfl_xor(o, 16);
+                o += __shfl_xor(o, 32);
+                size_t at = 0;
+                const bool have = in && cr_vol_at(A.vol, s.w, b, z0 + z, y, x, at);
+                const float xv = have ? A.vol.p[at] * A.vol.scale : 0.f;
+                o += hb1 + halpha * xv;
+                if constexpr (EPI == CR_HEAD) {
+                    if (have && kq == 0) A.vout[at] = o * A.oscale;
+                } else if (in) {
+                    const float d = o - A.tgt[vox] * A.tscale, g = 2.f * d * A.inv_count;
+                    float ga[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        loc[i] += g * v[i];
+                        ga[i] = v[i] > 0.f ? g * hw[i] : 0.f;
+                    }
+                    *reinterpret_cast<uint2*>(A.out + vox * 16 + 4 * kq) = cr_pack4(ga);
+                    lg += g;
+                    lgx += g * xv;
+                    ll += d * d * A.inv_count;
+                }
+            }
+        }
+    }
+    if constexpr (EPI == CR_LOSS) {
+        // lanes of one channel group by a fixed shuffle tree, then the waves in order
+        float* red = reinterpret_cast<float*>(xs);  // [waves][20]
+        __syncthreads();
+        float t[7] = {loc[0], loc[1], loc[2], loc[3], lg, lgx, ll};
+#pragma unroll
+        for (int i = 0; i < 7; i++)
+            for (int o = 8; o > 0; o >>= 1) t[i] += __shfl_xor(t[i], o);
+        if (m == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) red[wave * 20 + 4 * kq + i] = t[i];
+            if (kq == 0) {
+#pragma unroll
+                for (int i = 0; i < 3; i++) red[wave * 20 + 16 + i] = t[4 + i];
+                red[wave * 20 + 19] = 0.f;
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < 20) {
+            const int k = threadIdx.x;
+            float sum = red[k];
+            for (int w = 1; w < PX * PY; w++) sum += red[w * 20 + k];
+            A.part[(size_t)wg * 20 + k] = sum;
+        }
+    }
+}
+
+// The first convolution: one input channel, so the 27 taps are one K = 32 step
+// (the other 15 channels of its parameters meet zeros and are not read).  The
+// FP32 input is read, scaled and rounded here; a lane gathers its eight taps
+// from a block of BF16 scalars in LDS.  Bound by the activations it writes.
+constexpr int CR_FP = 20;  // LDS row pitch (18 staged)
+__device__ __forceinline__ void cr_stage_vol(unsigned short* xs, const CrVol& V, const CrShape& s, int b, int z0, int y0,
+                                             int x0, int lo, int hi, int nt) {
+    for (int t = threadIdx.x; t < 18 * 10 * 6; t += nt) {
+        const int gx = x0 - 1 + t % 18, gy = y0 - 1 + (t / 18) % 10, gz = z0 - 1 + t / 180;
+        float v = 0.f;
+        size_t at;
+        if (min(gx, min(gy, gz)) >= lo && max(gx, max(gy, gz)) < hi && cr_vol_at(V, s.w, b, gz, gy, gx, at))
+            v = V.p[at] * V.scale;
+        xs[(t / 18) * CR_FP + t % 18] = cr_f2bf(v);
+    }
+}
+
+__global__ void __launch_bounds__(256) k_cr_first(CrVol V, const uint4* __restrict__ wf, const float* __restrict__ bias,
+                                                  unsigned short* __restrict__ out, CrShape s, int lo, int hi) {
+    __shared__ unsigned short xs[10 * 6 * CR_FP];
+    const int ext = hi - lo;
+    const int bxn = (ext + 15) / 16, byn = (ext + 7) / 8, bzn = (ext + 3) / 4;
+    int tile, one;
+    if (!xcd_tile(bxn * byn * bzn * s.n, 1, tile, one)) return;
+    const int x0 = lo + tile % bxn * 16; tile /= bxn;
+    const int y0 = lo + tile % byn * 8; tile /= byn;
+    const int z0 = lo + tile % bzn * 4;
+    const int b = tile / bzn;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m = lane & 15, kq = lane >> 4, mx = m & 3, my = m >> 2;
+    cr_stage_vol(xs, V, s, b, z0, y0, x0, 0, s.w, 256);
+    const cr_b8 w = __builtin_bit_cast(cr_b8, wf[lane]);
+    const float4 bv = *reinterpret_cast<const float4*>(bias + 4 * kq);
+    int off[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int t = min(kq * 8 + j, 26);
+        off[j] = (t / 9 * 10 + t / 3 % 3 + my) * CR_FP + t % 3 + mx;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        const int pid = wave * 2 + p;
+        const int x = x0 + (pid & 3) * 4 + mx, y = y0 + (pid >> 2) * 4 + my;
+#pragma unroll
+        for (int z = 0; z < 4; z++) {
+            const unsigned short* r = xs + (z * 10 + (pid >> 2) * 4) * CR_FP + (pid & 3) * 4;
+            unsigned h[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) h[j] = kq * 8 + j < 27 ? r[off[j]] : 0;
+            const uint4 f = {h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
+            const cr_f4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, __builtin_bit_cast(cr_b8, f),
+                                                                   cr_f4{bv.x, bv.y, bv.z, bv.w}, 0, 0, 0);
+            if (x >= hi || y >= hi || z0 + z >= hi) continue;
+            const float v[4] = {fmaxf(d[0], 0.f), fmaxf(d[1], 0.f), fmaxf(d[2], 0.f), fmaxf(d[3], 0.f)};
+            *reinterpret_cast<uint2*>(out + cr_vox(s, b, z0 + z, y, x) * 16 + 4 * kq) = cr_pack4(v);
         }
     }
 }
@@ -251,10 +462,8 @@ constexpr int CR_WT = 192;                             // three waves
 // reads 2.1 times the input.  The form before it (one 16-bit LDS read per
 // element, K = 16) took 512 us a layer on average for four 80^3 crops.
 template <int NO>
-__global__ void __launch_bounds__(CR_WT) k_cr_wgrad(const unsigned short* __restrict__ in, int in_cs, int in_co,
-                                                    int cin, const unsigned short* __restrict__ dy, int dy_cs,
-                                                    int dy_co, int cout, float* __restrict__ part, CrShape s, int lo,
-                                                    int hi, int G) {
+__global__ void __launch_bounds__(CR_WT) k_cr_wgrad(CrIn in, int cin, const unsigned short* __restrict__ dy, int cout,
+                                                    float* __restrict__ part, CrShape s, int lo, int hi, int G) {
     __shared__ __align__(16) unsigned short xs[CR_WHX * CR_WHY * CR_WHZ * 16];
     __shared__ __align__(16) unsigned short ys[NO][CR_WBX * CR_WBY * CR_WBZ * 16];
     const int g = blockIdx.x, c = blockIdx.y, o0 = blockIdx.z * NO * 16;
@@ -267,6 +476,8 @@ __global__ void __launch_bounds__(CR_WT) k_cr_wgrad(const unsigned short* __rest
     const int e = hi - lo;
     const int bx_n = (e + CR_WBX - 1) / CR_WBX, by_n = (e + CR_WBY - 1) / CR_WBY, bz_n = (e + CR_WBZ - 1) / CR_WBZ;
     const int nblocks = s.n * bz_n * by_n * bx_n;
+    // the input is formed up to one voxel around the cube and no further
+    const int ilo = max(lo - 1, 0), ihi = min(hi + 1, s.w);
     cr_f4 acc[9][NO], bacc[NO];
 #pragma unroll
     for (int nb = 0; nb < NO; nb++) {
@@ -289,9 +500,8 @@ __global__ void __launch_bounds__(CR_WT) k_cr_wgrad(const unsigned short* __rest
             const int lx = v % CR_WHX, ly = (v / CR_WHX) % CR_WHY, lz = v / (CR_WHX * CR_WHY);
             const int gx = x0 - 1 + lx, gy = y0 - 1 + ly, gz = z0 - 1 + lz;
             uint4 val = {0u, 0u, 0u, 0u};
-            if (gx >= 0 && gx < s.w && gy >= 0 && gy < s.h && gz >= 0 && gz < s.d)
-                val = *reinterpret_cast<const uint4*>(in + cr_vox(s, b, gz, gy, gx) * in_cs + in_co + c * 16 +
-                                                      half * 8);
+            if (min(gx, min(gy, gz)) >= ilo && max(gx, max(gy, gz)) < ihi)
+                val = cr_load(in, s, c, half, b, gz, gy, gx);
             *reinterpret_cast<uint4*>(xs + t * 8) = val;
         }
 #pragma unroll
@@ -302,8 +512,8 @@ __global__ void __launch_bounds__(CR_WT) k_cr_wgrad(const unsigned short* __rest
                 const int gx = x0 + lx, gy = y0 + ly, gz = z0 + lz;
                 uint4 val = {0u, 0u, 0u, 0u};
                 if (gx < hi && gy < hi && gz < hi)
-                    val = *reinterpret_cast<const uint4*>(dy + cr_vox(s, b, gz, gy, gx) * dy_cs + dy_co + o0 +
-                                                          nb * 16 + half * 8);
+                    val = *reinterpret_cast<const uint4*>(dy + cr_vox(s, b, gz, gy, gx) * cout + o0 + nb * 16 +
+                                                          half * 8);
                 *reinterpret_cast<uint4*>(ys[nb] + t * 8) = val;
             }
         __syncthreads();
@@ -361,12 +571,79 @@ __global__ void __launch_bounds__(CR_WT) k_cr_wgrad(const unsigned short* __rest
     }
 }
 
+// The first layer's weight and bias gradients: one input channel, so the 27
+// taps and a row of ones (the bias) are the matrix rows and the contraction
+// over voxels runs on two row blocks instead of 27 taps.  part[g][28][16].
+__global__ void __launch_bounds__(256) k_cr_wgrad_first(CrVol V, const unsigned short* __restrict__ dy,
+                                                        float* __restrict__ part, CrShape s, int lo, int hi, int G) {
+    __shared__ unsigned short xs[10 * 6 * CR_FP];
+    __shared__ __align__(16) unsigned short ys[CR_WBX * CR_WBY * CR_WBZ * 16];
+    const int g = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m = lane & 15, kq = lane >> 4;
+    const int lrow = kq >> 1, lvx = (kq & 1) * 8 + (m >> 2), lch = (m & 3) * 4;
+    const int e = hi - lo;
+    const int bx_n = (e + CR_WBX - 1) / CR_WBX, by_n = (e + CR_WBY - 1) / CR_WBY, bz_n = (e + CR_WBZ - 1) / CR_WBZ;
+    const int nblocks = s.n * bz_n * by_n * bx_n;
+    int off[2];  // tap 16 k + m of the first voxel of this lane's eight
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int t = min(16 * k + m, 26);
+        off[k] = (t / 9 * 10 + t / 3 % 3 + lrow) * CR_FP + t % 3 + (kq & 1) * 8;
+    }
+    cr_f4 acc[2] = {cr_f4{0.f, 0.f, 0.f, 0.f}, cr_f4{0.f, 0.f, 0.f, 0.f}};
+    for (int blk0 = g; blk0 < nblocks; blk0 += G) {
+        int blk = blk0;
+        const int x0 = lo + blk % bx_n * CR_WBX; blk /= bx_n;
+        const int y0 = lo + blk % by_n * CR_WBY; blk /= by_n;
+        const int z0 = lo + blk % bz_n * CR_WBZ;
+        const int b = blk / bz_n;
+        __syncthreads();
+        cr_stage_vol(xs, V, s, b, z0, y0, x0, 0, s.w, 256);
+        for (int t = threadIdx.x; t < CR_WBX * CR_WBY * CR_WBZ * 2; t += 256) {
+            const int v = t >> 1, half = t & 1;
+            const int gx = x0 + v % CR_WBX, gy = y0 + (v / CR_WBX) % CR_WBY, gz = z0 + v / (CR_WBX * CR_WBY);
+            uint4 val = {0u, 0u, 0u, 0u};
+            if (gx < hi && gy < hi && gz < hi)
+                val = *reinterpret_cast<const uint4*>(dy + cr_vox(s, b, gz, gy, gx) * 16 + half * 8);
+            *reinterpret_cast<uint4*>(ys + t * 8) = val;
+        }
+        __syncthreads();
+        // wave = z plane of the block
+#pragma unroll
+        for (int yp = 0; yp < CR_WBY; yp += 2) {
+            const unsigned short* q = ys + ((wave * CR_WBY + yp + lrow) * CR_WBX + lvx) * 16 + lch;
+            const cr_b8 bf = cr_frag_tr(q, q + 4 * 16);
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const unsigned short* r = xs + (wave * 10 + yp) * CR_FP + off[k];
+                unsigned h[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) h[j] = 16 * k + m < 27 ? r[j] : (16 * k + m == 27 ? 0x3f80u : 0u);
+                const uint4 f = {h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
+                acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(cr_b8, f), bf, acc[k], 0, 0, 0);
+            }
+        }
+    }
+    // the four waves' sums in order
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(ys);  // [4][32][16]
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) red[(wave * 32 + 16 * k + 4 * kq + i) * 16 + m] = acc[k][i];
+    __syncthreads();
+    for (int t = threadIdx.x; t < 28 * 16; t += 256)
+        part[(size_t)g * 448 + t] = ((red[t] + red[512 + t]) + red[1024 + t]) + red[1536 + t];
+}
+
 // Sum of the G partial gradients of n values into grad.  A work-group takes
 // 64 values, four threads a value with a quarter of the partials each; every
 // quarter and the four quarters are added in order, so the sum is the same in
-// every run.
+// every run.  first: the values are [28][16] of the first layer, whose weights
+// [tap][ci][co] with ci > 0 never meet an input and keep a zero gradient.
 __global__ void __launch_bounds__(256) k_cr_reduce(const float* __restrict__ part, int G, size_t n,
-                                                   float* __restrict__ grad) {
+                                                   float* __restrict__ grad, int first) {
     __shared__ float red[4][64];
     const int l = threadIdx.x & 63, q = threadIdx.x >> 6;
     const size_t t = (size_t)blockIdx.x * 64 + l;
@@ -378,165 +655,45 @@ __global__ void __launch_bounds__(256) k_cr_reduce(const float* __restrict__ par
     }
     red[q][l] = sum;
     __syncthreads();
-    if (q == 0 && t < n) grad[t] = ((red[0][l] + red[1][l]) + red[2][l]) + red[3][l];
+    const size_t at = first ? (t >> 4) * 256 + (t & 15) : t;
+    if (q == 0 && t < n) grad[at] = ((red[0][l] + red[1][l]) + red[2][l]) + red[3][l];
 }
 
-// 2 x 2 x 2 average pooling: out (c channels) from in at half resolution.
-__global__ void k_cr_pool(const unsigned short* __restrict__ in, int in_cs, int in_co,
-                          unsigned short* __restrict__ out, int out_cs, int out_co, int c, CrShape so) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t nvox = (size_t)so.n * so.d * so.h * so.w;
-    if (t >= nvox * c) return;
-    const int ch = (int)(t % c);
-    size_t v = t / c;
-    const int x = (int)(v % so.w); v /= so.w;
-    const int y = (int)(v % so.h); v /= so.h;
-    const int z = (int)(v % so.d);
-    const int b = (int)(v / so.d);
-    const int W = 2 * so.w, H = 2 * so.h, D = 2 * so.d;
-    float sum = 0.f;
-    for (int k = 0; k < 8; k++) {
-        const int xx = 2 * x + (k & 1), yy = 2 * y + ((k >> 1) & 1), zz = 2 * z + (k >> 2);
-        sum += cr_bf2f(in[((((size_t)b * D + zz) * H + yy) * W + xx) * in_cs + in_co + ch]);
-    }
-    out[(t / c) * out_cs + out_co + ch] = cr_f2bf(0.125f * sum);
-}
-
-// Backward of the pooling added to the fine gradient, times the ReLU mask
-// of the pooled activation: g[v][c] = (g[v][c] + gc[v/2][c] / 8) * (act > 0).
-__global__ void k_cr_pool_bwd(unsigned short* __restrict__ gf, int g_cs, int g_co,
-                              const unsigned short* __restrict__ gc, int gc_cs, int gc_co,
-                              const unsigned short* __restrict__ act, int a_cs, int a_co, int c, CrShape sf) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t nvox = (size_t)sf.n * sf.d * sf.h * sf.w;
-    if (t >= nvox * c) return;
-    const int ch = (int)(t % c);
-    size_t v = t / c;
-    const size_t vf = v;
-    const int x = (int)(v % sf.w); v /= sf.w;
-    const int y = (int)(v % sf.h); v /= sf.h;
-    const int z = (int)(v % sf.d);
-    const int b = (int)(v / sf.d);
-    const size_t vc = (((size_t)b * (sf.d / 2) + z / 2) * (sf.h / 2) + y / 2) * (sf.w / 2) + x / 2;
-    const unsigned short a = act[vf * a_cs + a_co + ch];
-    float val = cr_bf2f(gf[vf * g_cs + g_co + ch]) + 0.125f * cr_bf2f(gc[vc * gc_cs + gc_co + ch]);
-    if (!(a != 0 && (a & 0x8000u) == 0)) val = 0.f;
-    gf[vf * g_cs + g_co + ch] = cr_f2bf(val);
-}
-
-// Nearest 2x upsampling: out (fine, c channels) from in (coarse).
-__global__ void k_cr_up(const unsigned short* __restrict__ in, int in_cs, int in_co,
-                        unsigned short* __restrict__ out, int out_cs, int out_co, int c, CrShape sf) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t nvox = (size_t)sf.n * sf.d * sf.h * sf.w;
-    if (t >= nvox * c) return;
-    const int ch = (int)(t % c);
-    size_t v = t / c;
-    const size_t vf = v;
-    const int x = (int)(v % sf.w); v /= sf.w;
-    const int y = (int)(v % sf.h); v /= sf.h;
-    const int z = (int)(v % sf.d);
-    const int b = (int)(v / sf.d);
-    const size_t vc = (((size_t)b * (sf.d / 2) + z / 2) * (sf.h / 2) + y / 2) * (sf.w / 2) + x / 2;
-    out[vf * out_cs + out_co + ch] = in[vc * in_cs + in_co + ch];
-}
-
-// Backward of the upsampling: gc[u][c] = sum of the 8 fine gradients.
-__global__ void k_cr_up_bwd(const unsigned short* __restrict__ gf, int g_cs, int g_co,
-                            unsigned short* __restrict__ gc, int gc_cs, int gc_co, int c, CrShape sc) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t nvox = (size_t)sc.n * sc.d * sc.h * sc.w;
-    if (t >= nvox * c) return;
-    const int ch = (int)(t % c);
-    size_t v = t / c;
-    const int x = (int)(v % sc.w); v /= sc.w;
-    const int y = (int)(v % sc.h); v /= sc.h;
-    const int z = (int)(v % sc.d);
-    const int b = (int)(v / sc.d);
-    const int W = 2 * sc.w, H = 2 * sc.h, D = 2 * sc.d;
-    float sum = 0.f;
-    for (int k = 0; k < 8; k++) {
-        const int xx = 2 * x + (k & 1), yy = 2 * y + ((k >> 1) & 1), zz = 2 * z + (k >> 2);
-        sum += cr_bf2f(gf[((((size_t)b * D + zz) * H + yy) * W + xx) * g_cs + g_co + ch]);
-    }
-    gc[(t / c) * gc_cs + gc_co + ch] = cr_f2bf(sum);
-}
-
-// Network input: FP32 crops [n][T][T][T] -> x0 (BF16, 16 channels, the value
-// times scale in channel 0) and x0f (FP32, the value times scale).
-__global__ void k_cr_input(const float* __restrict__ vol, float scale, size_t nvox,
-                           unsigned short* __restrict__ x0, float* __restrict__ x0f) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nvox) return;
-    const float v = vol[t] * scale;
-    x0f[t] = v;
-    uint4 z = {0u, 0u, 0u, 0u};
-    z.x = cr_f2bf(v);
-    *reinterpret_cast<uint4*>(x0 + t * 16) = z;
-    *reinterpret_cast<uint4*>(x0 + t * 16 + 8) = uint4{0u, 0u, 0u, 0u};
-}
-
-// Head: out = alpha * x0f + b1 + sum_c w1[c] * act[c]  (FP32); hp = {w1[16], b1, alpha}.
-__global__ void k_cr_head(const unsigned short* __restrict__ act, const float* __restrict__ x0f,
-                          const float* __restrict__ hp, size_t nvox, float* __restrict__ out) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nvox) return;
-    float s = hp[16] + hp[17] * x0f[t];
+// Gradient of an activation that is both pooled and concatenated: in the cube
+// [lo, hi)^3, g = (g inside [glo, ghi)^3, else 0, + gc at half the coordinates
+// / 8) where act > 0, else 0.  Eight channels a thread.
+__global__ void __launch_bounds__(256) k_cr_pool_bwd(unsigned short* __restrict__ g, const unsigned short* __restrict__ gc,
+                                                     const unsigned short* __restrict__ act, int c, CrShape s, int lo,
+                                                     int hi, int glo, int ghi) {
+    const int ext = hi - lo, c8 = c / 8;
+    const unsigned t = blockIdx.x * 256 + threadIdx.x;
+    const int k = (int)(t % c8);
+    unsigned v = t / c8;
+    const int x = lo + (int)(v % ext); v /= ext;
+    const int y = lo + (int)(v % ext); v /= ext;
+    const int z = lo + (int)(v % ext);
+    const int b = (int)(v / ext);
+    if (b >= s.n) return;
+    const size_t at = cr_vox(s, b, z, y, x) * c + k * 8;
+    const size_t ac = ((((size_t)b * (s.d / 2) + z / 2) * (s.h / 2) + y / 2) * (s.w / 2) + x / 2) * c + k * 8;
+    const bool have = min(x, min(y, z)) >= glo && max(x, max(y, z)) < ghi;
+    uint4 gv = {0u, 0u, 0u, 0u};
+    if (have) gv = *reinterpret_cast<const uint4*>(g + at);
+    const uint4 cv = *reinterpret_cast<const uint4*>(gc + ac), av = *reinterpret_cast<const uint4*>(act + at);
+    const unsigned gw[4] = {gv.x, gv.y, gv.z, gv.w}, cw[4] = {cv.x, cv.y, cv.z, cv.w}, aw[4] = {av.x, av.y, av.z, av.w};
+    uint2 r[2];
 #pragma unroll
-    for (int c = 0; c < 16; c++) s += hp[c] * cr_bf2f(act[t * 16 + c]);
-    out[t] = s;
-}
-
-// Loss and head backward over the central tile^3 of every T^3 crop
-// (halo h): L = sum (out - tgt)^2 / count; g = 2 (out - tgt) / count there and
-// 0 in the halo; gact[v][c] = g w1[c] (act > 0); per work-group partial sums
-// part[wg][20] = {dw1[16], db1, dalpha, loss, 0}.  Work-groups walk the voxels
-// in strides of the grid (CR_HEADG of them), each lane keeping its own sums;
-// lanes are added by a fixed shuffle tree, then the waves in order.
-constexpr int CR_HEADG = 1024;
-__global__ void __launch_bounds__(256) k_cr_head_bwd(const unsigned short* __restrict__ act,
-                                                     const float* __restrict__ x0f, const float* __restrict__ out,
-                                                     const float* __restrict__ tgt, const float* __restrict__ hp,
-                                                     int T, int halo, size_t nvox, float inv_count,
-                                                     unsigned short* __restrict__ gact, float* __restrict__ part) {
-    __shared__ float red[4][20];
-    float w1[16], loc[19];
+    for (int h = 0; h < 2; h++) {
+        float f[4];
 #pragma unroll
-    for (int c = 0; c < 16; c++) w1[c] = hp[c];
-#pragma unroll
-    for (int k = 0; k < 19; k++) loc[k] = 0.f;
-    for (size_t t = (size_t)blockIdx.x * 256 + threadIdx.x; t < nvox; t += (size_t)gridDim.x * 256) {
-        const int x = (int)(t % T), y = (int)((t / T) % T), z = (int)((t / ((size_t)T * T)) % T);
-        const bool in = x >= halo && x < T - halo && y >= halo && y < T - halo && z >= halo && z < T - halo;
-        const float d = out[t] - tgt[t];
-        const float g = in ? 2.f * d * inv_count : 0.f;
-        uint4 w[2], av4[2];
-        unsigned short* wp = reinterpret_cast<unsigned short*>(w);
-        const unsigned short* ap = reinterpret_cast<const unsigned short*>(av4);
-        av4[0] = *reinterpret_cast<const uint4*>(act + t * 16);
-        av4[1] = *reinterpret_cast<const uint4*>(act + t * 16 + 8);
-#pragma unroll
-        for (int c = 0; c < 16; c++) {
-            const unsigned short a = ap[c];
-            loc[c] += g * cr_bf2f(a);
-            wp[c] = cr_f2bf((a != 0 && (a & 0x8000u) == 0) ? g * w1[c] : 0.f);
+        for (int i = 0; i < 2; i++) {
+            f[2 * i] = cr_bflo(gw[2 * h + i]) + 0.125f * cr_bflo(cw[2 * h + i]);
+            f[2 * i + 1] = cr_bfhi(gw[2 * h + i]) + 0.125f * cr_bfhi(cw[2 * h + i]);
         }
-        *reinterpret_cast<uint4*>(gact + t * 16) = w[0];
-        *reinterpret_cast<uint4*>(gact + t * 16 + 8) = w[1];
-        loc[16] += g;
-        loc[17] += g * x0f[t];
-        loc[18] += in ? d * d * inv_count : 0.f;
+        cr_relu_mask(f, uint2{aw[2 * h], aw[2 * h + 1]});
+        r[h] = cr_pack4(f);
     }
-#pragma unroll
-    for (int k = 0; k < 19; k++) {
-        for (int o = 32; o > 0; o >>= 1) loc[k] += __shfl_xor(loc[k], o);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = loc[k];
-    }
-    __syncthreads();
-    if (threadIdx.x < 20) {
-        const int k = threadIdx.x;
-        part[(size_t)blockIdx.x * 20 + k] = k < 19 ? ((red[0][k] + red[1][k]) + red[2][k]) + red[3][k] : 0.f;
-    }
+    *reinterpret_cast<uint4*>(g + at) = uint4{r[0].x, r[0].y, r[1].x, r[1].y};
 }
 
 // Sum of nblk partial rows of width 20 in FP64 into res[20] and, of the first
@@ -602,41 +759,14 @@ __global__ void k_cr_pack(const float* __restrict__ W, int cin, int cout, int fw
     wf[t] = q;
 }
 
-// Tiles of a volume for inference: crop b of the (tz, ty, tx) tile grid
-// covers [t0 - halo, t0 + tile + halo) per axis, zeros outside the volume.
-__global__ void k_cr_gather(const float* __restrict__ vol, int nx, int ny, int nz, int tile, int halo,
-                            int ntx, int nty, int first, int nb, float* __restrict__ crops) {
-    const int T = tile + 2 * halo;
-    const size_t per = (size_t)T * T * T;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= per * nb) return;
-    const int b = (int)(t / per);
-    size_t r = t % per;
-    const int x = (int)(r % T), y = (int)((r / T) % T), z = (int)(r / ((size_t)T * T));
-    const int id = first + b;
-    const int tx = id % ntx, ty = (id / ntx) % nty, tz = id / (ntx * nty);
-    const int gx = tx * tile - halo + x, gy = ty * tile - halo + y, gz = tz * tile - halo + z;
-    float v = 0.f;
-    if (gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz) v = vol[((size_t)gz * ny + gy) * nx + gx];
-    crops[t] = v;
-}
-
-// Central tile^3 of each output crop back into the volume (divided by scale).
-__global__ void k_cr_scatter(const float* __restrict__ crops, int nx, int ny, int nz, int tile, int halo,
-                             int ntx, int nty, int first, int nb, float inv_scale, float* __restrict__ vol) {
-    const int T = tile + 2 * halo;
-    const size_t per = (size_t)tile * tile * tile;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= per * nb) return;
-    const int b = (int)(t / per);
-    size_t r = t % per;
-    const int x = (int)(r % tile), y = (int)((r / tile) % tile), z = (int)(r / ((size_t)tile * tile));
-    const int id = first + b;
-    const int tx = id % ntx, ty = (id / ntx) % nty, tz = id / (ntx * nty);
-    const int gx = tx * tile + x, gy = ty * tile + y, gz = tz * tile + z;
-    if (gx >= nx || gy >= ny || gz >= nz) return;
-    const size_t src = (size_t)b * T * T * T + ((size_t)(z + halo) * T + (y + halo)) * T + (x + halo);
-    vol[((size_t)gz * ny + gy) * nx + gx] = crops[src] * inv_scale;
+// The first layer's fragment: lane (n = lane % 16, kq = lane / 16) holds taps
+// 8 kq + j (zero from 27 on) of input channel 0, output channel n.
+__global__ void k_cr_pack_first(const float* __restrict__ W, uint4* __restrict__ wf) {
+    const int lane = threadIdx.x, n = lane & 15, kq = lane >> 4;
+    uint4 q;
+    unsigned short* h = reinterpret_cast<unsigned short*>(&q);
+    for (int j = 0; j < 8; j++) h[j] = kq * 8 + j < 27 ? cr_f2bf(W[(kq * 8 + j) * 256 + n]) : (unsigned short)0;
+    wf[lane] = q;
 }
 
 }  // namespace utr
@@ -651,14 +781,14 @@ struct CrLayerDef {
 };
 constexpr CrLayerDef kCrLayers[10] = {
     {16, 16},  // e1a  (input: the volume in channel 0 of 16)
-    {16, 16},  // e1b  -> C1[32:48]
+    {16, 16},  // e1b
     {16, 32},  // e2a  (input: pooled e1b)
-    {32, 32},  // e2b  -> C2[64:96]
+    {32, 32},  // e2b
     {32, 64},  // e3a  (input: pooled e2b)
     {64, 64},  // e3b
-    {96, 32},  // d2a  (input: C2 = up(e3b) | e2b)
+    {96, 32},  // d2a  (input: up(e3b) | e2b)
     {32, 32},  // d2b
-    {48, 16},  // d1a  (input: C1 = up(d2b) | e1b)
+    {48, 16},  // d1a  (input: up(d2b) | e1b)
     {16, 16},  // d1b
 };
 constexpr int kCrHead = 18;
@@ -681,11 +811,11 @@ struct utr_corr {
     int step = 0;
     float scale = 1.f;
     // activations (BF16, channels last) at the three resolutions
-    DevBuf<bf16_t> x0, e1a, C1, p1, e2a, C2, p2, e3a, e3b, d2a, d2b, d1a, d1b;
-    DevBuf<float> x0f, out;
+    DevBuf<bf16_t> e1a, e1b, p1, e2a, e2b, p2, e3a, e3b, d2a, d2b, d1a;
     // activation gradients
-    DevBuf<bf16_t> gd1b, gd1a, gC1, gd2b, gd2a, gC2, ge3b, ge3a, gp2, ge2a, gp1, ge1a;
-    DevBuf<float> part, hpart, crops_in, crops_out;
+    DevBuf<bf16_t> gd1b, gd1a, ge1b, gd2b, gd2a, ge2b, ge3b, ge3a, gp2, ge2a, gp1, ge1a;
+    DevBuf<uint4> wfirst;
+    DevBuf<float> part, hpart;
     hipStream_t st = nullptr;
     double last_ms = 0.0;
 };
@@ -699,43 +829,117 @@ utr::CrShape cr_shape(int n, int e) {
     return s;
 }
 
-// Blocks of 16 x 8 voxels in x and y where they make at least two work-groups
-// per CU, 8 x 8 otherwise (the coarsest level of a few crops).
-template <int PX, int PY>
+struct CrCube {
+    int lo, hi;
+};
+
+// The cubes a network pass over crops of edge T needs when only outputs in
+// [h, T - h)^3 count: each is grown by one voxel per convolution behind it,
+// halved (rounded outwards) at each coarser level, and made even where a
+// pooling or upsampling pairs voxels.  Forward, activation qN is formed on its
+// cube from inputs formed on theirs; backward, every gradient is zero outside
+// the same cubes.
+struct CrCubes {
+    CrCube d1b, d1a, c1, d2b, d2a, c2, e3b, e3a, e2b, e2a, e1b, e1a;
+};
+CrCubes cr_cubes(int T, int h) {
+    auto grow = [](CrCube q, int e) { return CrCube{std::max(0, q.lo - 1), std::min(e, q.hi + 1)}; };
+    auto half = [](CrCube q) { return CrCube{q.lo / 2, (q.hi + 1) / 2}; };
+    auto twice = [](CrCube q) { return CrCube{2 * q.lo, 2 * q.hi}; };
+    auto both = [](CrCube a, CrCube b) { return CrCube{std::min(a.lo, b.lo), std::max(a.hi, b.hi)}; };
+    CrCubes Q;
+    Q.d1b = {h, T - h};
+    Q.d1a = grow(Q.d1b, T);
+    Q.d2b = half(grow(Q.d1a, T));
+    Q.c1 = twice(Q.d2b);  // concatenated input of d1a
+    Q.d2a = grow(Q.d2b, T / 2);
+    Q.e3b = half(grow(Q.d2a, T / 2));
+    Q.c2 = twice(Q.e3b);  // concatenated input of d2a
+    Q.e3a = grow(Q.e3b, T / 4);
+    Q.e2b = both(Q.c2, twice(grow(Q.e3a, T / 4)));
+    Q.e2a = grow(Q.e2b, T / 2);
+    Q.e1b = both(Q.c1, twice(grow(Q.e2a, T / 2)));
+    Q.e1a = grow(Q.e1b, T);
+    return Q;
+}
+
+// Work-groups a convolution's cube [lo, hi)^3 of n crops splits into: blocks
+// of 16 x 8 voxels in x and y where they make at least two work-groups per CU,
+// 8 x 8 otherwise (the coarsest level of a few crops).
+long cr_conv_tiles(int px, int py, int n, CrCube q) {
+    const long e = q.hi - q.lo;
+    return n * ((e + 4 * px - 1) / (4 * px)) * ((e + 4 * py - 1) / (4 * py)) * ((e + utr::CR_Z - 1) / utr::CR_Z);
+}
+bool cr_conv_big(int n, CrCube q) { return cr_conv_tiles(4, 2, n, q) >= 512; }
+
+template <int NB, int EPI>
 int cr_conv_launch(utr_corr* c, const utr::CrConv& A) {
-    const auto& s = A.s;
-    const unsigned tiles = (unsigned)(s.n * ((s.w + 4 * PX - 1) / (4 * PX)) * ((s.h + 4 * PY - 1) / (4 * PY)) *
-                                      ((s.d + utr::CR_Z - 1) / utr::CR_Z));
-    const int nb = A.nbt % 3 == 0 ? 3 : A.nbt % 2 == 0 ? 2 : 1;
-    const unsigned grid = utr::xcd_grid(tiles * (unsigned)(A.nbt / nb));
-    if (nb == 3) utr::k_cr_conv<PX, PY, 3><<<grid, 256, 0, c->st>>>(A);
-    else if (nb == 2) utr::k_cr_conv<PX, PY, 2><<<grid, 256, 0, c->st>>>(A);
-    else utr::k_cr_conv<PX, PY, 1><<<grid, 256, 0, c->st>>>(A);
+    const CrCube q = {A.lo, A.hi};
+    if (cr_conv_big(A.s.n, q)) {
+        const unsigned grid = utr::xcd_grid((unsigned)cr_conv_tiles(4, 2, A.s.n, q) * (unsigned)(A.nbt / NB));
+        utr::k_cr_conv<4, 2, NB, EPI><<<grid, 512, 0, c->st>>>(A);
+    } else {
+        const unsigned grid = utr::xcd_grid((unsigned)cr_conv_tiles(2, 2, A.s.n, q) * (unsigned)(A.nbt / NB));
+        utr::k_cr_conv<2, 2, NB, EPI><<<grid, 256, 0, c->st>>>(A);
+    }
     UTR_HIP_TRY(hipGetLastError());
     return UTR_OK;
 }
 
-int cr_conv(utr_corr* c, int layer, bool fwd, const bf16_t* in, int in_cs, int in_co, bf16_t* out, int out_cs,
-            int out_co, const bf16_t* mask, int mask_cs, int mask_co, utr::CrShape s) {
+// A layer's convolution (forward) or input gradient; the caller fills in what
+// its epilogue needs.
+utr::CrConv cr_conv_args(const utr_corr* c, int layer, bool fwd, utr::CrIn in, utr::CrShape s, CrCube q, CrCube iq) {
     const CrLayer& Ly = c->L[layer];
-    utr::CrConv A;
+    utr::CrConv A{};
     A.in = in;
-    A.in_cs = in_cs;
-    A.in_co = in_co;
     A.cin = fwd ? Ly.cin : Ly.cout;
     A.nbt = (fwd ? Ly.cout : Ly.cin) / 16;
     A.wf = fwd ? Ly.wf.p : Ly.wb.p;
-    A.bias = fwd ? c->w.p + Ly.boff : nullptr;
-    A.relu = fwd ? 1 : 0;
-    A.mask = mask;
-    A.mask_cs = mask_cs;
-    A.mask_co = mask_co;
-    A.out = out;
-    A.out_cs = out_cs;
-    A.out_co = out_co;
+    A.bias = c->w.p + Ly.boff;
     A.s = s;
-    const long big = (long)s.n * ((s.w + 15) / 16) * ((s.h + 7) / 8) * ((s.d + 3) / 4);
-    return big >= 512 ? cr_conv_launch<4, 2>(c, A) : cr_conv_launch<2, 2>(c, A);
+    A.lo = q.lo;
+    A.hi = q.hi;
+    A.ilo = iq.lo;
+    A.ihi = iq.hi;
+    return A;
+}
+utr::CrIn cr_in(const DevBuf<bf16_t>& p, int ch) { return utr::CrIn{nullptr, 0, 0, p.p, ch}; }
+utr::CrIn cr_in(const DevBuf<bf16_t>& up, int upc, const DevBuf<bf16_t>& p, int ch) {
+    return utr::CrIn{up.p, upc, upc / 16, p.p, ch};
+}
+
+int cr_act(utr_corr* c, int layer, utr::CrIn in, bf16_t* out, utr::CrShape s, CrCube q, bf16_t* pooled = nullptr) {
+    utr::CrConv A = cr_conv_args(c, layer, true, in, s, q, {0, s.w});
+    A.out = out;
+    A.out_c = A.out2_c = 16 * A.nbt;
+    A.out2 = pooled;
+    if (pooled) return A.nbt == 1 ? cr_conv_launch<1, utr::CR_POOL>(c, A) : cr_conv_launch<2, utr::CR_POOL>(c, A);
+    return A.nbt == 1 ? cr_conv_launch<1, utr::CR_ACT>(c, A) : cr_conv_launch<2, utr::CR_ACT>(c, A);
+}
+
+// Input gradient on cube q of an output gradient that is zero outside gq.
+int cr_grad(utr_corr* c, int layer, const DevBuf<bf16_t>& dy, CrCube gq, bf16_t* out, const bf16_t* mask, utr::CrShape s,
+            CrCube q) {
+    utr::CrConv A = cr_conv_args(c, layer, false, cr_in(dy, c->L[layer].cout), s, q, gq);
+    A.out = out;
+    A.out_c = 16 * A.nbt;
+    A.mask = mask;
+    return A.nbt == 1 ? cr_conv_launch<1, utr::CR_GRAD>(c, A) : cr_conv_launch<2, utr::CR_GRAD>(c, A);
+}
+
+// The same for a layer whose input is an upsampled tensor of upc channels
+// beside one at its own resolution.
+int cr_grad_split(utr_corr* c, int layer, const DevBuf<bf16_t>& dy, CrCube gq, bf16_t* gup, const bf16_t* up, int upc,
+                  bf16_t* out, const bf16_t* mask, utr::CrShape s, CrCube q) {
+    utr::CrConv A = cr_conv_args(c, layer, false, cr_in(dy, c->L[layer].cout), s, q, gq);
+    A.nup = upc / 16;
+    A.out = out;
+    A.out_c = 16 * A.nbt - upc;
+    A.mask = mask;
+    A.out2 = gup;
+    A.out2_c = upc;
+    A.mask2 = up;
+    return cr_conv_launch<3, utr::CR_SPLIT>(c, A);
 }
 
 // Weight-gradient launch of a layer over n cubes [0, e)^3: output blocks per
@@ -752,23 +956,29 @@ int cr_wgrad_groups(int cin, int cout, int n, int e) {
     return (nb + each - 1) / each;
 }
 
-// dy is zero outside [lo, hi)^3.
-int cr_wgrad(utr_corr* c, int layer, const bf16_t* in, int in_cs, int in_co, const bf16_t* dy, int dy_cs,
-             int dy_co, utr::CrShape s, int lo, int hi) {
+// dy is zero outside q^3.
+int cr_wgrad(utr_corr* c, int layer, utr::CrIn in, const DevBuf<bf16_t>& dy, utr::CrShape s, CrCube q) {
     const CrLayer& Ly = c->L[layer];
     const size_t nw = (size_t)27 * Ly.cin * Ly.cout + Ly.cout;
-    const int no = cr_wgrad_no(Ly.cout), G = cr_wgrad_groups(Ly.cin, Ly.cout, s.n, hi - lo);
+    const int no = cr_wgrad_no(Ly.cout), G = cr_wgrad_groups(Ly.cin, Ly.cout, s.n, q.hi - q.lo);
     if ((size_t)G * nw > c->part.n) return set_err(UTR_E_STATE, "corrector: gradient workspace too small");
     const dim3 grid(G, Ly.cin / 16, Ly.cout / 16 / no);
     if (no == 2)
-        utr::k_cr_wgrad<2><<<grid, utr::CR_WT, 0, c->st>>>(in, in_cs, in_co, Ly.cin, dy, dy_cs, dy_co, Ly.cout,
-                                                           c->part.p, s, lo, hi, G);
+        utr::k_cr_wgrad<2><<<grid, utr::CR_WT, 0, c->st>>>(in, Ly.cin, dy.p, Ly.cout, c->part.p, s, q.lo, q.hi, G);
     else
-        utr::k_cr_wgrad<1><<<grid, utr::CR_WT, 0, c->st>>>(in, in_cs, in_co, Ly.cin, dy, dy_cs, dy_co, Ly.cout,
-                                                           c->part.p, s, lo, hi, G);
+        utr::k_cr_wgrad<1><<<grid, utr::CR_WT, 0, c->st>>>(in, Ly.cin, dy.p, Ly.cout, c->part.p, s, q.lo, q.hi, G);
     UTR_HIP_TRY(hipGetLastError());
     // weights and bias of a layer are contiguous in the gradient vector
-    utr::k_cr_reduce<<<(unsigned)((nw + 63) / 64), 256, 0, c->st>>>(c->part.p, G, nw, c->g.p + Ly.woff);
+    utr::k_cr_reduce<<<(unsigned)((nw + 63) / 64), 256, 0, c->st>>>(c->part.p, G, nw, c->g.p + Ly.woff, 0);
+    UTR_HIP_TRY(hipGetLastError());
+    return UTR_OK;
+}
+
+int cr_wgrad_first(utr_corr* c, const utr::CrVol& V, const DevBuf<bf16_t>& dy, utr::CrShape s, CrCube q) {
+    const int G = cr_wgrad_groups(16, 16, s.n, q.hi - q.lo);
+    utr::k_cr_wgrad_first<<<G, 256, 0, c->st>>>(V, dy.p, c->part.p, s, q.lo, q.hi, G);
+    UTR_HIP_TRY(hipGetLastError());
+    utr::k_cr_reduce<<<7, 256, 0, c->st>>>(c->part.p, G, 448, c->g.p + c->L[0].woff, 1);
     UTR_HIP_TRY(hipGetLastError());
     return UTR_OK;
 }
@@ -790,16 +1000,17 @@ size_t cr_part_size() {
 int cr_alloc(utr_corr* c) {
     const size_t n1 = (size_t)c->batch * c->T * c->T * c->T;
     const size_t n2 = n1 / 8, n3 = n1 / 64;
+    // the loss's partial sums: one row per work-group of the last convolution
+    const CrCube q = {c->halo, c->T - c->halo};
+    const size_t hp = (size_t)std::max(cr_conv_tiles(4, 2, c->batch, q), cr_conv_tiles(2, 2, c->batch, q)) * 20;
     const hipError_t e[] = {
-        c->x0.alloc(n1 * 16), c->e1a.alloc(n1 * 16), c->C1.alloc(n1 * 48), c->p1.alloc(n2 * 16),
-        c->e2a.alloc(n2 * 32), c->C2.alloc(n2 * 96), c->p2.alloc(n3 * 32), c->e3a.alloc(n3 * 64),
-        c->e3b.alloc(n3 * 64), c->d2a.alloc(n2 * 32), c->d2b.alloc(n2 * 32), c->d1a.alloc(n1 * 16),
-        c->d1b.alloc(n1 * 16), c->x0f.alloc(n1), c->out.alloc(n1),
-        c->gd1b.alloc(n1 * 16), c->gd1a.alloc(n1 * 16), c->gC1.alloc(n1 * 48), c->gd2b.alloc(n2 * 32),
-        c->gd2a.alloc(n2 * 32), c->gC2.alloc(n2 * 96), c->ge3b.alloc(n3 * 64), c->ge3a.alloc(n3 * 64),
+        c->e1a.alloc(n1 * 16), c->e1b.alloc(n1 * 16), c->p1.alloc(n2 * 16), c->e2a.alloc(n2 * 32),
+        c->e2b.alloc(n2 * 32), c->p2.alloc(n3 * 32), c->e3a.alloc(n3 * 64), c->e3b.alloc(n3 * 64),
+        c->d2a.alloc(n2 * 32), c->d2b.alloc(n2 * 32), c->d1a.alloc(n1 * 16),
+        c->gd1b.alloc(n1 * 16), c->gd1a.alloc(n1 * 16), c->ge1b.alloc(n1 * 16), c->gd2b.alloc(n2 * 32),
+        c->gd2a.alloc(n2 * 32), c->ge2b.alloc(n2 * 32), c->ge3b.alloc(n3 * 64), c->ge3a.alloc(n3 * 64),
         c->gp2.alloc(n3 * 32), c->ge2a.alloc(n2 * 32), c->gp1.alloc(n2 * 16), c->ge1a.alloc(n1 * 16),
-        c->part.alloc(cr_part_size()), c->hpart.alloc((size_t)utr::CR_HEADG * 20), c->res.alloc(32),
-        c->crops_in.alloc(n1), c->crops_out.alloc(n1)};
+        c->wfirst.alloc(64), c->part.alloc(cr_part_size()), c->hpart.alloc(hp), c->res.alloc(32)};
     for (hipError_t x : e)
         if (x != hipSuccess)
             return set_err(x == hipErrorOutOfMemory ? UTR_E_NOMEM : UTR_E_DEVICE,
@@ -808,7 +1019,9 @@ int cr_alloc(utr_corr* c) {
 }
 
 int cr_repack(utr_corr* c) {
-    for (int l = 0; l < 10; l++) {
+    utr::k_cr_pack_first<<<1, 64, 0, c->st>>>(c->w.p + c->L[0].woff, c->wfirst.p);
+    UTR_HIP_TRY(hipGetLastError());
+    for (int l = 1; l < 10; l++) {
         CrLayer& Ly = c->L[l];
         const size_t nf = (size_t)(Ly.cin / 16) * utr::CR_STEPS * (Ly.cout / 16) * 64;
         utr::k_cr_pack<<<cr_blocks(nf), 256, 0, c->st>>>(c->w.p + Ly.woff, Ly.cin, Ly.cout, 1, Ly.wf.p);
@@ -819,105 +1032,96 @@ int cr_repack(utr_corr* c) {
     return UTR_OK;
 }
 
-// Forward pass of nb crops already in x0 / x0f; result in c->out.
-int cr_forward(utr_corr* c, int nb) {
+// Forward pass of nb crops of V up to d1a, on the cubes Q.
+int cr_forward(utr_corr* c, int nb, const utr::CrVol& V, const CrCubes& Q) {
     const int T = c->T;
     const utr::CrShape s1 = cr_shape(nb, T), s2 = cr_shape(nb, T / 2), s3 = cr_shape(nb, T / 4);
-    const size_t n1 = (size_t)nb * T * T * T, n2 = n1 / 8, n3 = n1 / 64;
     int rc;
-    if ((rc = cr_conv(c, 0, true, c->x0.p, 16, 0, c->e1a.p, 16, 0, nullptr, 0, 0, s1))) return rc;
-    if ((rc = cr_conv(c, 1, true, c->e1a.p, 16, 0, c->C1.p, 48, 32, nullptr, 0, 0, s1))) return rc;
-    utr::k_cr_pool<<<cr_blocks(n2 * 16), 256, 0, c->st>>>(c->C1.p, 48, 32, c->p1.p, 16, 0, 16, s2);
-    if ((rc = cr_conv(c, 2, true, c->p1.p, 16, 0, c->e2a.p, 32, 0, nullptr, 0, 0, s2))) return rc;
-    if ((rc = cr_conv(c, 3, true, c->e2a.p, 32, 0, c->C2.p, 96, 64, nullptr, 0, 0, s2))) return rc;
-    utr::k_cr_pool<<<cr_blocks(n3 * 32), 256, 0, c->st>>>(c->C2.p, 96, 64, c->p2.p, 32, 0, 32, s3);
-    if ((rc = cr_conv(c, 4, true, c->p2.p, 32, 0, c->e3a.p, 64, 0, nullptr, 0, 0, s3))) return rc;
-    if ((rc = cr_conv(c, 5, true, c->e3a.p, 64, 0, c->e3b.p, 64, 0, nullptr, 0, 0, s3))) return rc;
-    utr::k_cr_up<<<cr_blocks(n2 * 64), 256, 0, c->st>>>(c->e3b.p, 64, 0, c->C2.p, 96, 0, 64, s2);
-    if ((rc = cr_conv(c, 6, true, c->C2.p, 96, 0, c->d2a.p, 32, 0, nullptr, 0, 0, s2))) return rc;
-    if ((rc = cr_conv(c, 7, true, c->d2a.p, 32, 0, c->d2b.p, 32, 0, nullptr, 0, 0, s2))) return rc;
-    utr::k_cr_up<<<cr_blocks(n1 * 32), 256, 0, c->st>>>(c->d2b.p, 32, 0, c->C1.p, 48, 0, 32, s1);
-    if ((rc = cr_conv(c, 8, true, c->C1.p, 48, 0, c->d1a.p, 16, 0, nullptr, 0, 0, s1))) return rc;
-    if ((rc = cr_conv(c, 9, true, c->d1a.p, 16, 0, c->d1b.p, 16, 0, nullptr, 0, 0, s1))) return rc;
-    utr::k_cr_head<<<cr_blocks(n1), 256, 0, c->st>>>(c->d1b.p, c->x0f.p, c->w.p + c->headoff, n1, c->out.p);
+    utr::k_cr_first<<<utr::xcd_grid((unsigned)cr_conv_tiles(4, 2, nb, Q.e1a)), 256, 0, c->st>>>(
+        V, c->wfirst.p, c->w.p + c->L[0].boff, c->e1a.p, s1, Q.e1a.lo, Q.e1a.hi);
     UTR_HIP_TRY(hipGetLastError());
-    return UTR_OK;
+    if ((rc = cr_act(c, 1, cr_in(c->e1a, 16), c->e1b.p, s1, Q.e1b, c->p1.p))) return rc;
+    if ((rc = cr_act(c, 2, cr_in(c->p1, 16), c->e2a.p, s2, Q.e2a))) return rc;
+    if ((rc = cr_act(c, 3, cr_in(c->e2a, 32), c->e2b.p, s2, Q.e2b, c->p2.p))) return rc;
+    if ((rc = cr_act(c, 4, cr_in(c->p2, 32), c->e3a.p, s3, Q.e3a))) return rc;
+    if ((rc = cr_act(c, 5, cr_in(c->e3a, 64), c->e3b.p, s3, Q.e3b))) return rc;
+    if ((rc = cr_act(c, 6, cr_in(c->e3b, 64, c->e2b, 32), c->d2a.p, s2, Q.d2a))) return rc;
+    if ((rc = cr_act(c, 7, cr_in(c->d2a, 32), c->d2b.p, s2, Q.d2b))) return rc;
+    return cr_act(c, 8, cr_in(c->d2b, 32, c->e1b, 16), c->d1a.p, s1, Q.d1a);
 }
 
-// Loss and gradients of nb crops after cr_forward, targets in tgt (FP32,
-// already scaled); gradient vector in c->g, {dw1, db1, dalpha, loss} in res.
-int cr_backward(utr_corr* c, int nb, const float* tgt) {
+// The last convolution with the head: out (laid out like V) = oscale * (alpha x
+// + b1 + w1 . d1b) on the cube Q.d1b of each crop.
+int cr_head(utr_corr* c, int nb, const utr::CrVol& V, const CrCubes& Q, float* out, float oscale) {
+    utr::CrConv A = cr_conv_args(c, 9, true, cr_in(c->d1a, 16), cr_shape(nb, c->T), Q.d1b, {0, c->T});
+    A.vol = V;
+    A.hp = c->w.p + c->headoff;
+    A.vout = out;
+    A.oscale = oscale;
+    return cr_conv_launch<1, utr::CR_HEAD>(c, A);
+}
+
+// Loss and gradients of nb crops V after cr_forward against the targets tgt
+// (unscaled): gradient vector in c->g, {dw1, db1, dalpha, loss} in res.
+int cr_backward(utr_corr* c, int nb, const utr::CrVol& V, const CrCubes& Q, const float* tgt) {
     const int T = c->T;
     const utr::CrShape s1 = cr_shape(nb, T), s2 = cr_shape(nb, T / 2), s3 = cr_shape(nb, T / 4);
-    const size_t n1 = (size_t)nb * T * T * T, n2 = n1 / 8, n3 = n1 / 64;
     const double cnt = (double)nb * c->tile * c->tile * c->tile;
-    const unsigned hb = std::min(cr_blocks(n1), (unsigned)utr::CR_HEADG);
     int rc;
-    utr::k_cr_head_bwd<<<hb, 256, 0, c->st>>>(c->d1b.p, c->x0f.p, c->out.p, tgt, c->w.p + c->headoff, T, c->halo, n1,
-                                              (float)(1.0 / cnt), c->gd1b.p, c->hpart.p);
+    utr::CrConv A = cr_conv_args(c, 9, true, cr_in(c->d1a, 16), s1, Q.d1b, {0, T});
+    A.vol = V;
+    A.hp = c->w.p + c->headoff;
+    A.out = c->gd1b.p;
+    A.tgt = tgt;
+    A.tscale = c->scale;
+    A.inv_count = (float)(1.0 / cnt);
+    A.part = c->hpart.p;
+    const long nwg = cr_conv_big(nb, Q.d1b) ? cr_conv_tiles(4, 2, nb, Q.d1b) : cr_conv_tiles(2, 2, nb, Q.d1b);
+    if ((size_t)nwg * 20 > c->hpart.n) return set_err(UTR_E_STATE, "corrector: loss workspace too small");
+    if ((rc = cr_conv_launch<1, utr::CR_LOSS>(c, A))) return rc;
+    utr::k_cr_head_reduce<<<1, 640, 0, c->st>>>(c->hpart.p, (int)nwg, kCrHead, c->res.p, c->g.p + c->headoff);
     UTR_HIP_TRY(hipGetLastError());
-    utr::k_cr_head_reduce<<<1, 640, 0, c->st>>>(c->hpart.p, (int)hb, kCrHead, c->res.p, c->g.p + c->headoff);
-    UTR_HIP_TRY(hipGetLastError());
-    // The loss covers [halo, T - halo)^3, so each layer's output gradient is
-    // zero outside that cube grown by one voxel per convolution behind it
-    // (halved, rounded outwards, at each coarser level); its weight gradient
-    // contracts over that cube only.
-    struct Cube {
-        int lo, hi;
+    auto pool_bwd = [&](DevBuf<bf16_t>& g, const DevBuf<bf16_t>& gc, const DevBuf<bf16_t>& act, int ch, utr::CrShape s,
+                        CrCube q, CrCube have) -> int {
+        const size_t e = (size_t)(q.hi - q.lo), n = (size_t)nb * e * e * e * (ch / 8);
+        utr::k_cr_pool_bwd<<<cr_blocks(n), 256, 0, c->st>>>(g.p, gc.p, act.p, ch, s, q.lo, q.hi, have.lo, have.hi);
+        UTR_HIP_TRY(hipGetLastError());
+        return UTR_OK;
     };
-    auto grow = [](Cube q, int e) { return Cube{std::max(0, q.lo - 1), std::min(e, q.hi + 1)}; };
-    auto half = [](Cube q) { return Cube{q.lo / 2, (q.hi + 1) / 2}; };
-    const Cube q9 = {c->halo, T - c->halo}, q8 = grow(q9, T), qC1 = grow(q8, T);
-    const Cube q7 = half(qC1), q6 = grow(q7, T / 2), qC2 = grow(q6, T / 2);
-    const Cube q5 = half(qC2), q4 = grow(q5, T / 4), qp2 = grow(q4, T / 4);
-    const Cube q3 = {std::min(qC2.lo, 2 * qp2.lo), std::max(qC2.hi, 2 * qp2.hi)};
-    const Cube q2 = grow(q3, T / 2), qp1 = grow(q2, T / 2);
-    const Cube q1 = {std::min(qC1.lo, 2 * qp1.lo), std::max(qC1.hi, 2 * qp1.hi)}, q0 = grow(q1, T);
     // d1b, d1a
-    if ((rc = cr_wgrad(c, 9, c->d1a.p, 16, 0, c->gd1b.p, 16, 0, s1, q9.lo, q9.hi))) return rc;
-    if ((rc = cr_conv(c, 9, false, c->gd1b.p, 16, 0, c->gd1a.p, 16, 0, c->d1a.p, 16, 0, s1))) return rc;
-    if ((rc = cr_wgrad(c, 8, c->C1.p, 48, 0, c->gd1a.p, 16, 0, s1, q8.lo, q8.hi))) return rc;
-    if ((rc = cr_conv(c, 8, false, c->gd1a.p, 16, 0, c->gC1.p, 48, 0, c->C1.p, 48, 0, s1))) return rc;
-    // up(d2b) -> d2b, d2a
-    utr::k_cr_up_bwd<<<cr_blocks(n2 * 32), 256, 0, c->st>>>(c->gC1.p, 48, 0, c->gd2b.p, 32, 0, 32, s2);
-    if ((rc = cr_wgrad(c, 7, c->d2a.p, 32, 0, c->gd2b.p, 32, 0, s2, q7.lo, q7.hi))) return rc;
-    if ((rc = cr_conv(c, 7, false, c->gd2b.p, 32, 0, c->gd2a.p, 32, 0, c->d2a.p, 32, 0, s2))) return rc;
-    if ((rc = cr_wgrad(c, 6, c->C2.p, 96, 0, c->gd2a.p, 32, 0, s2, q6.lo, q6.hi))) return rc;
-    if ((rc = cr_conv(c, 6, false, c->gd2a.p, 32, 0, c->gC2.p, 96, 0, c->C2.p, 96, 0, s2))) return rc;
-    // up(e3b) -> e3b, e3a
-    utr::k_cr_up_bwd<<<cr_blocks(n3 * 64), 256, 0, c->st>>>(c->gC2.p, 96, 0, c->ge3b.p, 64, 0, 64, s3);
-    if ((rc = cr_wgrad(c, 5, c->e3a.p, 64, 0, c->ge3b.p, 64, 0, s3, q5.lo, q5.hi))) return rc;
-    if ((rc = cr_conv(c, 5, false, c->ge3b.p, 64, 0, c->ge3a.p, 64, 0, c->e3a.p, 64, 0, s3))) return rc;
-    if ((rc = cr_wgrad(c, 4, c->p2.p, 32, 0, c->ge3a.p, 64, 0, s3, q4.lo, q4.hi))) return rc;
-    if ((rc = cr_conv(c, 4, false, c->ge3a.p, 64, 0, c->gp2.p, 32, 0, nullptr, 0, 0, s3))) return rc;
-    // pool(e2b) -> e2b (skip and pooled paths), e2a
-    utr::k_cr_pool_bwd<<<cr_blocks(n2 * 32), 256, 0, c->st>>>(c->gC2.p, 96, 64, c->gp2.p, 32, 0, c->C2.p, 96, 64, 32,
-                                                               s2);
-    if ((rc = cr_wgrad(c, 3, c->e2a.p, 32, 0, c->gC2.p, 96, 64, s2, q3.lo, q3.hi))) return rc;
-    if ((rc = cr_conv(c, 3, false, c->gC2.p, 96, 64, c->ge2a.p, 32, 0, c->e2a.p, 32, 0, s2))) return rc;
-    if ((rc = cr_wgrad(c, 2, c->p1.p, 16, 0, c->ge2a.p, 32, 0, s2, q2.lo, q2.hi))) return rc;
-    if ((rc = cr_conv(c, 2, false, c->ge2a.p, 32, 0, c->gp1.p, 16, 0, nullptr, 0, 0, s2))) return rc;
-    // pool(e1b) -> e1b, e1a
-    utr::k_cr_pool_bwd<<<cr_blocks(n1 * 16), 256, 0, c->st>>>(c->gC1.p, 48, 32, c->gp1.p, 16, 0, c->C1.p, 48, 32, 16,
-                                                               s1);
-    if ((rc = cr_wgrad(c, 1, c->e1a.p, 16, 0, c->gC1.p, 48, 32, s1, q1.lo, q1.hi))) return rc;
-    if ((rc = cr_conv(c, 1, false, c->gC1.p, 48, 32, c->ge1a.p, 16, 0, c->e1a.p, 16, 0, s1))) return rc;
-    if ((rc = cr_wgrad(c, 0, c->x0.p, 16, 0, c->ge1a.p, 16, 0, s1, q0.lo, q0.hi))) return rc;
-    UTR_HIP_TRY(hipGetLastError());
-    return UTR_OK;
+    if ((rc = cr_wgrad(c, 9, cr_in(c->d1a, 16), c->gd1b, s1, Q.d1b))) return rc;
+    if ((rc = cr_grad(c, 9, c->gd1b, Q.d1b, c->gd1a.p, c->d1a.p, s1, Q.d1a))) return rc;
+    if ((rc = cr_wgrad(c, 8, cr_in(c->d2b, 32, c->e1b, 16), c->gd1a, s1, Q.d1a))) return rc;
+    if ((rc = cr_grad_split(c, 8, c->gd1a, Q.d1a, c->gd2b.p, c->d2b.p, 32, c->ge1b.p, c->e1b.p, s1, Q.c1))) return rc;
+    // d2b, d2a
+    if ((rc = cr_wgrad(c, 7, cr_in(c->d2a, 32), c->gd2b, s2, Q.d2b))) return rc;
+    if ((rc = cr_grad(c, 7, c->gd2b, Q.d2b, c->gd2a.p, c->d2a.p, s2, Q.d2a))) return rc;
+    if ((rc = cr_wgrad(c, 6, cr_in(c->e3b, 64, c->e2b, 32), c->gd2a, s2, Q.d2a))) return rc;
+    if ((rc = cr_grad_split(c, 6, c->gd2a, Q.d2a, c->ge3b.p, c->e3b.p, 64, c->ge2b.p, c->e2b.p, s2, Q.c2))) return rc;
+    // e3b, e3a
+    const CrCube p2 = {Q.e2b.lo / 2, Q.e2b.hi / 2}, p1 = {Q.e1b.lo / 2, Q.e1b.hi / 2};
+    if ((rc = cr_wgrad(c, 5, cr_in(c->e3a, 64), c->ge3b, s3, Q.e3b))) return rc;
+    if ((rc = cr_grad(c, 5, c->ge3b, Q.e3b, c->ge3a.p, c->e3a.p, s3, Q.e3a))) return rc;
+    if ((rc = cr_wgrad(c, 4, cr_in(c->p2, 32), c->ge3a, s3, Q.e3a))) return rc;
+    if ((rc = cr_grad(c, 4, c->ge3a, Q.e3a, c->gp2.p, nullptr, s3, p2))) return rc;
+    // e2b (skip and pooled paths), e2a
+    if ((rc = pool_bwd(c->ge2b, c->gp2, c->e2b, 32, s2, Q.e2b, Q.c2))) return rc;
+    if ((rc = cr_wgrad(c, 3, cr_in(c->e2a, 32), c->ge2b, s2, Q.e2b))) return rc;
+    if ((rc = cr_grad(c, 3, c->ge2b, Q.e2b, c->ge2a.p, c->e2a.p, s2, Q.e2a))) return rc;
+    if ((rc = cr_wgrad(c, 2, cr_in(c->p1, 16), c->ge2a, s2, Q.e2a))) return rc;
+    if ((rc = cr_grad(c, 2, c->ge2a, Q.e2a, c->gp1.p, nullptr, s2, p1))) return rc;
+    // e1b, e1a
+    if ((rc = pool_bwd(c->ge1b, c->gp1, c->e1b, 16, s1, Q.e1b, Q.c1))) return rc;
+    if ((rc = cr_wgrad(c, 1, cr_in(c->e1a, 16), c->ge1b, s1, Q.e1b))) return rc;
+    if ((rc = cr_grad(c, 1, c->ge1b, Q.e1b, c->ge1a.p, c->e1a.p, s1, Q.e1a))) return rc;
+    return cr_wgrad_first(c, V, c->ge1a, s1, Q.e1a);
 }
 
-int cr_load_crops(utr_corr* c, const float* d_in, int nb) {
-    const size_t n1 = (size_t)nb * c->T * c->T * c->T;
-    utr::k_cr_input<<<cr_blocks(n1), 256, 0, c->st>>>(d_in, c->scale, n1, c->x0.p, c->x0f.p);
-    UTR_HIP_TRY(hipGetLastError());
-    return UTR_OK;
-}
-
-// Target crops scaled like the input, into crops_out (reused as scratch).
-__global__ void k_cr_scale_copy(const float* __restrict__ src, float s, size_t n, float* __restrict__ dst) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) dst[t] = src[t] * s;
+utr::CrVol cr_crops(const utr_corr* c, const float* d_in) {
+    utr::CrVol V{};
+    V.p = d_in;
+    V.scale = c->scale;
+    return V;
 }
 
 int cr_check(utr_corr* c) {
@@ -1037,11 +1241,10 @@ int utr_corr_set_params(utr_corr* c, const float* host, float scale) {
 int utr_corr_forward(utr_corr* c, const float* d_in, int nb, float* d_out) {
     if (int rc = cr_check(c)) return rc;
     if (!d_in || !d_out || nb < 1 || nb > c->batch) return set_err(UTR_E_INVALID, "utr_corr_forward: 1 <= nb <= batch crops");
-    if (int rc = cr_load_crops(c, d_in, nb)) return rc;
-    if (int rc = cr_forward(c, nb)) return rc;
-    const size_t n1 = (size_t)nb * c->T * c->T * c->T;
-    k_cr_scale_copy<<<cr_blocks(n1), 256, 0, c->st>>>(c->out.p, 1.f / c->scale, n1, d_out);
-    UTR_HIP_TRY(hipGetLastError());
+    const utr::CrVol V = cr_crops(c, d_in);
+    const CrCubes Q = cr_cubes(c->T, 0);  // the whole crop is returned
+    if (int rc = cr_forward(c, nb, V, Q)) return rc;
+    if (int rc = cr_head(c, nb, V, Q, d_out, 1.f / c->scale)) return rc;
     UTR_HIP_TRY(hipStreamSynchronize(c->st));
     return UTR_OK;
 }
@@ -1050,12 +1253,10 @@ int utr_corr_gradient(utr_corr* c, const float* d_in, const float* d_tgt, int nb
     if (int rc = cr_check(c)) return rc;
     if (!d_in || !d_tgt || nb < 1 || nb > c->batch)
         return set_err(UTR_E_INVALID, "utr_corr_gradient: 1 <= nb <= batch crops");
-    const size_t n1 = (size_t)nb * c->T * c->T * c->T;
-    if (int rc = cr_load_crops(c, d_in, nb)) return rc;
-    k_cr_scale_copy<<<cr_blocks(n1), 256, 0, c->st>>>(d_tgt, c->scale, n1, c->crops_out.p);
-    UTR_HIP_TRY(hipGetLastError());
-    if (int rc = cr_forward(c, nb)) return rc;
-    if (int rc = cr_backward(c, nb, c->crops_out.p)) return rc;
+    const utr::CrVol V = cr_crops(c, d_in);
+    const CrCubes Q = cr_cubes(c->T, c->halo);
+    if (int rc = cr_forward(c, nb, V, Q)) return rc;
+    if (int rc = cr_backward(c, nb, V, Q, d_tgt)) return rc;
     float res[20];
     UTR_HIP_TRY(hipMemcpyAsync(res, c->res.p, sizeof(res), hipMemcpyDeviceToHost, c->st));
     UTR_HIP_TRY(hipStreamSynchronize(c->st));
@@ -1069,12 +1270,10 @@ int utr_corr_train_step(utr_corr* c, const float* d_in, const float* d_tgt, int 
     if (!d_in || !d_tgt || nb < 1 || nb > c->batch)
         return set_err(UTR_E_INVALID, "utr_corr_train_step: 1 <= nb <= batch crops");
     if (!(lr > 0) || !std::isfinite(lr)) return set_err(UTR_E_INVALID, "utr_corr_train_step: lr must be positive");
-    const size_t n1 = (size_t)nb * c->T * c->T * c->T;
-    if (int rc = cr_load_crops(c, d_in, nb)) return rc;
-    k_cr_scale_copy<<<cr_blocks(n1), 256, 0, c->st>>>(d_tgt, c->scale, n1, c->crops_out.p);
-    UTR_HIP_TRY(hipGetLastError());
-    if (int rc = cr_forward(c, nb)) return rc;
-    if (int rc = cr_backward(c, nb, c->crops_out.p)) return rc;
+    const utr::CrVol V = cr_crops(c, d_in);
+    const CrCubes Q = cr_cubes(c->T, c->halo);
+    if (int rc = cr_forward(c, nb, V, Q)) return rc;
+    if (int rc = cr_backward(c, nb, V, Q, d_tgt)) return rc;
     c->step++;
     const double b1 = 0.9, b2 = 0.999;
     const double lr_t = lr * std::sqrt(1.0 - std::pow(b2, c->step)) / (1.0 - std::pow(b1, c->step));
@@ -1096,18 +1295,20 @@ int utr_corr_apply(utr_corr* c, const float* d_vol, float* d_out, int nx, int ny
     if (nx < 1 || ny < 1 || nz < 1) return set_err(UTR_E_INVALID, "utr_corr_apply: sizes must be positive");
     const int ntx = (nx + c->tile - 1) / c->tile, nty = (ny + c->tile - 1) / c->tile, ntz = (nz + c->tile - 1) / c->tile;
     const int ntiles = ntx * nty * ntz;
-    const size_t per = (size_t)c->T * c->T * c->T;
+    const CrCubes Q = cr_cubes(c->T, c->halo);
+    utr::CrVol V = cr_crops(c, d_vol);
+    V.nx = nx;
+    V.ny = ny;
+    V.nz = nz;
+    V.tile = c->tile;
+    V.halo = c->halo;
+    V.ntx = ntx;
+    V.nty = nty;
     for (int first = 0; first < ntiles; first += c->batch) {
         const int nb = std::min(c->batch, ntiles - first);
-        utr::k_cr_gather<<<cr_blocks(per * nb), 256, 0, c->st>>>(d_vol, nx, ny, nz, c->tile, c->halo, ntx, nty, first,
-                                                                 nb, c->crops_in.p);
-        UTR_HIP_TRY(hipGetLastError());
-        if (int rc = cr_load_crops(c, c->crops_in.p, nb)) return rc;
-        if (int rc = cr_forward(c, nb)) return rc;
-        const size_t pt = (size_t)c->tile * c->tile * c->tile;
-        utr::k_cr_scatter<<<cr_blocks(pt * nb), 256, 0, c->st>>>(c->out.p, nx, ny, nz, c->tile, c->halo, ntx, nty,
-                                                                 first, nb, 1.f / c->scale, d_out);
-        UTR_HIP_TRY(hipGetLastError());
+        V.first = first;
+        if (int rc = cr_forward(c, nb, V, Q)) return rc;
+        if (int rc = cr_head(c, nb, V, Q, d_out, 1.f / c->scale)) return rc;
     }
     UTR_HIP_TRY(hipStreamSynchronize(c->st));
     return UTR_OK;
@@ -1124,13 +1325,13 @@ int utr_corr_destroy(utr_corr* c) {
         Ly.wf.release();
         Ly.wb.release();
     }
-    DevBuf<bf16_t>* bb[] = {&c->x0, &c->e1a, &c->C1, &c->p1, &c->e2a, &c->C2, &c->p2, &c->e3a, &c->e3b,
-                            &c->d2a, &c->d2b, &c->d1a, &c->d1b, &c->gd1b, &c->gd1a, &c->gC1, &c->gd2b,
-                            &c->gd2a, &c->gC2, &c->ge3b, &c->ge3a, &c->gp2, &c->ge2a, &c->gp1, &c->ge1a};
+    DevBuf<bf16_t>* bb[] = {&c->e1a, &c->e1b, &c->p1, &c->e2a, &c->e2b, &c->p2, &c->e3a, &c->e3b, &c->d2a, &c->d2b,
+                            &c->d1a, &c->gd1b, &c->gd1a, &c->ge1b, &c->gd2b, &c->gd2a, &c->ge2b, &c->ge3b, &c->ge3a,
+                            &c->gp2, &c->ge2a, &c->gp1, &c->ge1a};
     for (auto* b : bb) b->release();
-    DevBuf<float>* fb[] = {&c->w, &c->g, &c->m, &c->v, &c->res, &c->x0f, &c->out, &c->part, &c->hpart,
-                           &c->crops_in, &c->crops_out};
+    DevBuf<float>* fb[] = {&c->w, &c->g, &c->m, &c->v, &c->res, &c->part, &c->hpart};
     for (auto* b : fb) b->release();
+    c->wfirst.release();
     delete c;
     return UTR_OK;
 }

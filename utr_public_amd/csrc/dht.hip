@@ -35,6 +35,7 @@ struct DhtGeom {
     double xlo, ylo, xc, yc, zc;
     int nx2, ny2, nz2;
     int use_ap;  // aperture or Cs terms present: filters read the table ap
+    double rxst;  // 1 / xst (dht_quot)
 };
 
 // One orientation of the DHT path.
@@ -63,8 +64,17 @@ struct SerAng {
 };
 
 constexpr int DHT_BX = 16, DHT_BY = 8, DHT_BZ = 8;
-constexpr int DHT_PY = DHT_BX + 1, DHT_PZ = DHT_PY * (DHT_BY + 1), DHT_PAD = DHT_PZ * DHT_BZ;
+// LDS sums with a one-cell halo on every side: cell (x, y, z) of [-1, B]^3 at
+// dht_lds; the halo cells of neighbouring rows and planes share slots (they
+// are written and never read)
+constexpr int DHT_PY = DHT_BX + 1, DHT_PZ = DHT_PY * (DHT_BY + 1);
+constexpr int DHT_PAD = (DHT_BX + 1) + DHT_PY * (DHT_BY + 1) + DHT_PZ * (DHT_BZ + 1) + 1;
 constexpr int DHT_VOX = DHT_BX * DHT_BY * DHT_BZ;
+constexpr int DHT_LINES = 512;    // source lines listed together (two a thread)
+// and their samples: the map to grid positions is a rotation, so the unit
+// cubes about the samples of a 17.1 x 9.1 x 9.1 box lie in that box grown by
+// sqrt(3)/2 on every side, whose volume is 2214
+constexpr int DHT_POINTS = 2304;
 
 __device__ __forceinline__ double dht_freq(int k, int n, double xst) {
     return (double)(k <= n / 2 ? k : k - n) / ((double)n * xst);
@@ -344,12 +354,35 @@ __global__ void __launch_bounds__(256) k_dht_prop_cols(const cplx<float>* __rest
         atomicMax(pmax, __float_as_uint(fmaxf(fmaxf(s_wmax[0], s_wmax[1]), fmaxf(s_wmax[2], s_wmax[3]))));
 }
 
-__device__ __forceinline__ int dht_lds(int lx, int ly, int lz) { return lx + DHT_PY * ly + DHT_PZ * lz; }
+__device__ __forceinline__ int dht_lds(int lx, int ly, int lz) {
+    return (lx + 1) + DHT_PY * (ly + 1) + DHT_PZ * (lz + 1);
+}
+
+// a / b with r = 1 / b rounded to nearest: the quotient a r corrected once by
+// its exact remainder (P. Markstein, IBM J. Res. Dev. 34 (1990) 111) is the
+// rounded quotient, in three operations instead of the dozen of a division.
+__device__ __forceinline__ double dht_quot(double a, double b, double r) {
+    const double q = __dmul_rn(a, r);
+    return __fma_rn(__fma_rn(-q, b, a), r, q);
+}
 
 // Splat of the batch's plane stacks (orientations a0 .. a0+na-1) into one
 // brick, added to the FP64 volume acc3 (the brick's own voxels only).
 // xs/ys/zs: per orientation (x_i - xc) sinY, (x_i - xc) cosY; (y_j - yc) sinZ,
 // (y_j - yc) cosZ; (z_n - zc) sinY, (z_n - zc) cosY, as DHT.cpp:1083-1107.
+//
+// Per orientation the threads clip the source lines (n, j) that can reach the
+// brick to it (about 400 lines of 4 samples on average, 1.34 times the brick's
+// voxels in all), give each line a run of the brick's point list (a wave
+// prefix sum and one LDS add per wave) and write the line's number into its
+// run; then every thread takes points, one sample each, so all lanes work
+// (with a line per lane they waited for the wave's longest line).  The order
+// of the points does not matter: the sums are exact.  Lists are double
+// buffered, so one barrier separates a list's writing from its reading.  A
+// sample's eight corners go to LDS without bounds tests (the halo takes those
+// outside).  Bound by the FP64 instructions of a sample.  Measured with 108
+// random orientations of 256 x 128 x 151 samples: 5.26 ms, against 11.75 ms
+// with a line per lane and IEEE divisions.
 __global__ void __launch_bounds__(256) k_dht_splat(const float* __restrict__ P, DhtGeom g,
                                                    const DhtRow* __restrict__ rows,
                                                    const double* __restrict__ xs,
@@ -358,12 +391,16 @@ __global__ void __launch_bounds__(256) k_dht_splat(const float* __restrict__ P, 
                                                    const unsigned* __restrict__ pmax,
                                                    double* __restrict__ acc3) {
     __shared__ unsigned long long acc[DHT_PAD];
-    const int tid = threadIdx.x;
+    __shared__ int2 s_line[2][DHT_LINES];  // i - point number, j | n << 10 (j < 2^10)
+    __shared__ unsigned short s_pt[2][DHT_POINTS];
+    __shared__ int s_tot[3];
+    const int tid = threadIdx.x, lane = tid & 63;
     const int nbx = (g.nx + DHT_BX - 1) / DHT_BX, nby = (g.ny + DHT_BY - 1) / DHT_BY;
     const int bid = blockIdx.x;
     const int bx = bid % nbx, by = (bid / nbx) % nby, bz = bid / (nbx * nby);
     const int x0 = bx * DHT_BX, y0 = by * DHT_BY, z0 = bz * DHT_BZ;
     for (int t = tid; t < DHT_PAD; t += 256) acc[t] = 0ull;
+    if (tid < 3) s_tot[tid] = 0;
     // fixed-point scale: per orientation a voxel takes at most 27 samples with
     // |weight| <= 8 (truncation allows dz1 in (-1, 0)), so |sum| < 2^8 na max|P|
     int ek = 0, ea = 0;
@@ -376,94 +413,118 @@ __global__ void __launch_bounds__(256) k_dht_splat(const float* __restrict__ P, 
 
     const int np_stride = g.nplanes;
     const size_t n2 = (size_t)g.nx * g.ny;
+    // samples whose truncated cell can touch the brick lie in the open box
+    // (x0-1, x0+BX) etc.; 0.05 of margin covers the FP32 error of the maps
+    // below (coordinates up to 2^10, a few units of 2^-24 relative)
+    const float bl[3] = {(float)x0 - 1.05f, (float)y0 - 1.05f, (float)z0 - 1.05f};
+    const float bh[3] = {(float)(x0 + DHT_BX) + 0.05f, (float)(y0 + DHT_BY) + 0.05f, (float)(z0 + DHT_BZ) + 0.05f};
+    int round = 0;
     for (int ab = 0; ab < na; ab++) {
         const DhtRow& R = rows[a0 + ab];
-        // source-index box of the brick's preimage: samples whose truncated
-        // cell can touch the brick lie in the open box (x0-1, x0+BX) etc.
-        float lo[3] = {1e30f, 1e30f, 1e30f}, hi[3] = {-1e30f, -1e30f, -1e30f};
-        const float bl[3] = {(float)x0 - 1.f, (float)y0 - 1.f, (float)z0 - 1.f};
-        const float bh[3] = {(float)(x0 + DHT_BX), (float)(y0 + DHT_BY), (float)(z0 + DHT_BZ)};
+        // source-index box (i, j, n) of the brick's preimage
+        int slo[3], shi[3];
+        const int smax[3] = {g.nx - 1, g.ny - 1, g.nz - 1};
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const float q[3] = {((c & 1) ? bh[0] : bl[0]) - R.c0[0], ((c & 2) ? bh[1] : bl[1]) - R.c0[1],
-                                ((c & 4) ? bh[2] : bl[2]) - R.c0[2]};
+        for (int d = 0; d < 3; d++) {
+            float ctr = 0.f, half = 0.f;
 #pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const float v = R.inv[3 * d] * q[0] + R.inv[3 * d + 1] * q[1] + R.inv[3 * d + 2] * q[2];
-                lo[d] = fminf(lo[d], v);
-                hi[d] = fmaxf(hi[d], v);
+            for (int c = 0; c < 3; c++) {
+                ctr += R.inv[3 * d + c] * (0.5f * (bl[c] + bh[c]) - R.c0[c]);
+                half += fabsf(R.inv[3 * d + c]) * (0.5f * (bh[c] - bl[c]));
             }
+            slo[d] = (int)fmaxf(ceilf(ctr - half), 0.f);
+            shi[d] = (int)fminf(floorf(ctr + half), (float)smax[d]);
         }
-        // lo/hi over (i, j, n); one sample of margin
-        const int jlo = max((int)floorf(lo[1]) - 1, 0), jhi = min((int)ceilf(hi[1]) + 1, g.ny - 1);
-        const int nlo = max((int)floorf(lo[2]) - 1, 0), nhi = min((int)ceilf(hi[2]) + 1, g.nz - 1);
-        const int ilo0 = max((int)floorf(lo[0]) - 1, 0), ihi0 = min((int)ceilf(hi[0]) + 1, g.nx - 1);
-        if (jlo > jhi || nlo > nhi || ilo0 > ihi0) continue;
-        const int nj = jhi - jlo + 1;
-        const int nlines = nj * (nhi - nlo + 1);
-        const double* X = xs + (size_t)(a0 + ab) * 2 * g.nx;
-        const double* Y = ys + (size_t)(a0 + ab) * 2 * g.ny;
-        const double* Z = zs + (size_t)(a0 + ab) * 2 * g.nz;
-        for (int L = tid; L < nlines; L += 256) {
-            const int n = nlo + L / nj, j = jlo + L % nj;
-            // i-interval of this line inside the box (slab test, one sample of margin)
-            float ilo = (float)ilo0, ihi = (float)ihi0;
+        const int jlo = slo[1], nj = shi[1] - jlo + 1, nlo = slo[2];
+        if (slo[0] > shi[0] || nj <= 0 || nlo > shi[2]) continue;
+        const int nlines = nj * (shi[2] - nlo + 1);
+        const double2* X = reinterpret_cast<const double2*>(xs) + (size_t)(a0 + ab) * g.nx;
+        const double2* Y = reinterpret_cast<const double2*>(ys) + (size_t)(a0 + ab) * g.ny;
+        const double2* Z = reinterpret_cast<const double2*>(zs) + (size_t)(a0 + ab) * g.nz;
+        const float* Pab = P + (size_t)ab * np_stride * n2;
+        for (int L0 = 0; L0 < nlines; L0 += DHT_LINES, round++) {
+            const int buf = round & 1;
+            int pos[2], cnt[2];
+            if (tid == 0) s_tot[(round + 1) % 3] = 0;
 #pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const float base = R.c0[d] + R.uj[d] * j + R.un[d] * n;
-                const float u = R.ui[d];
-                const float l = bl[d] - 0.05f - base, h = bh[d] + 0.05f - base;
-                if (fabsf(u) < 1e-6f) {
-                    if (l > 0.f || h < 0.f) ihi = ilo - 1.f;
-                } else {
-                    float t0 = l / u, t1 = h / u;
-                    if (u < 0.f) { const float tt = t0; t0 = t1; t1 = tt; }
-                    ilo = fmaxf(ilo, floorf(t0) - 1.f);
-                    ihi = fminf(ihi, ceilf(t1) + 1.f);
+            for (int h = 0; h < 2; h++) {
+                const int Lc = h * 256 + tid, L = L0 + Lc;
+                cnt[h] = 0;
+                int i0 = 0, j = 0, n = 0;
+                if (L < nlines) {
+                    n = nlo + L / nj;
+                    j = jlo + L % nj;
+                    // i-interval of this line inside the box
+                    float ilo = (float)slo[0], ihi = (float)shi[0];
+#pragma unroll
+                    for (int d = 0; d < 3; d++) {
+                        const float base = R.c0[d] + R.uj[d] * j + R.un[d] * n;
+                        const float u = R.ui[d];
+                        const float l = bl[d] - base, hh = bh[d] - base;
+                        if (fabsf(u) < 1e-6f) {
+                            if (l > 0.f || hh < 0.f) ihi = ilo - 1.f;
+                        } else {
+                            const float r = 1.f / u, t0 = l * r, t1 = hh * r;
+                            ilo = fmaxf(ilo, ceilf(fminf(t0, t1)));
+                            ihi = fminf(ihi, floorf(fmaxf(t0, t1)));
+                        }
+                    }
+                    if (ilo <= ihi) {
+                        i0 = (int)ilo;
+                        cnt[h] = (int)ihi - i0 + 1;
+                    }
                 }
+                int incl = cnt[h];
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int v = __shfl_up(incl, o);
+                    if (lane >= o) incl += v;
+                }
+                int base = 0;
+                if (lane == 63) base = atomicAdd(&s_tot[round % 3], incl);
+                base = __shfl(base, 63);
+                pos[h] = base + incl - cnt[h];
+                s_line[buf][Lc] = int2{i0 - pos[h], j | (n << 10)};
+                for (int q = 0; q < cnt[h] && pos[h] + q < DHT_POINTS; q++)
+                    s_pt[buf][pos[h] + q] = (unsigned short)Lc;
             }
-            ilo = fminf(ilo, (float)ihi0 + 1.f);  // keep the conversions in range
-            ihi = fmaxf(ihi, (float)ilo0 - 1.f);
-            const int i0 = (int)ilo, i1 = (int)ihi;
-            const float* Kp = P + ((size_t)ab * np_stride + (g.escc ? n : 0)) * n2 + (size_t)j * g.nx;
-            const double zsin = Z[2 * n], zcos = Z[2 * n + 1];
-            const double ysin = Y[2 * j], ycos = Y[2 * j + 1];
-            for (int i = i0; i <= i1; i++) {
+            __syncthreads();
+            const int total = min(s_tot[round % 3], DHT_POINTS);
+            for (int p = tid; p < total; p += 256) {
+                const int2 ln = s_line[buf][s_pt[buf][p]];
+                const int i = ln.x + p, j = ln.y & 0x3ff, n = (int)((unsigned)ln.y >> 10);
+                const float kraw = Pab[(size_t)(g.escc ? n : 0) * n2 + (size_t)j * g.nx + i];
+                const double2 xv = X[i], yv = Y[j], zv = Z[n];
                 // DHT.cpp:1119-1150, operation by operation
-                const double zzz = __dadd_rn(__dadd_rn(g.zc, zcos), X[2 * i]);
-                double dz1 = __ddiv_rn(__dsub_rn(zzz, g.zlodz), g.xst);
+                const double zzz = __dadd_rn(__dadd_rn(g.zc, zv.y), xv.x);
+                double dz1 = dht_quot(__dsub_rn(zzz, g.zlodz), g.xst, g.rxst);
                 const int nn = (int)dz1;
-                if (nn < 0 || nn > g.nz2) continue;
                 dz1 = __dsub_rn(dz1, (double)nn);
                 const double dz0 = __dsub_rn(1.0, dz1);
-                const double xx = __dadd_rn(-zsin, X[2 * i + 1]);
+                const double xx = __dadd_rn(-zv.x, xv.y);
                 const double xx_sinZ = __dmul_rn(xx, R.sinZ), xx_cosZ = __dmul_rn(xx, R.cosZ);
-                const double xxx = __dadd_rn(__dadd_rn(g.xc, ysin), xx_cosZ);
-                double dx1 = __ddiv_rn(__dsub_rn(xxx, g.xlo), g.xst);
+                const double xxx = __dadd_rn(__dadd_rn(g.xc, yv.x), xx_cosZ);
+                double dx1 = dht_quot(__dsub_rn(xxx, g.xlo), g.xst, g.rxst);
                 const int ii = (int)dx1;
-                if (ii < 0 || ii > g.nx2) continue;
                 dx1 = __dsub_rn(dx1, (double)ii);
                 const double dx0 = __dsub_rn(1.0, dx1);
-                const double yyy = __dsub_rn(__dadd_rn(g.yc, ycos), xx_sinZ);
-                double dy1 = __ddiv_rn(__dsub_rn(yyy, g.ylo), g.xst);
+                const double yyy = __dsub_rn(__dadd_rn(g.yc, yv.y), xx_sinZ);
+                double dy1 = dht_quot(__dsub_rn(yyy, g.ylo), g.xst, g.rxst);
                 const int jj = (int)dy1;
-                if (jj < 0 || jj > g.ny2) continue;
                 dy1 = __dsub_rn(dy1, (double)jj);
                 const double dy0 = __dsub_rn(1.0, dy1);
+                if (nn < 0 || nn > g.nz2 || ii < 0 || ii > g.nx2 || jj < 0 || jj > g.ny2) continue;
                 const int lx = ii - x0, ly = jj - y0, lz = nn - z0;
                 if (lx < -1 || lx >= DHT_BX || ly < -1 || ly >= DHT_BY || lz < -1 || lz >= DHT_BZ) continue;
-                const double k = (double)Kp[i];
+                const double k = (double)kraw;
                 const double dz0K = dz0 * k, dz1K = dz1 * k;
                 const double wx[2] = {dx0, dx1}, wy[2] = {dy0, dy1}, wz[2] = {dz0K, dz1K};
+                unsigned long long* A = acc + dht_lds(lx, ly, lz);
 #pragma unroll
                 for (int c = 0; c < 8; c++) {
                     const int cx = c & 1, cy = (c >> 1) & 1, cz = c >> 2;
-                    const int vx = lx + cx, vy = ly + cy, vz = lz + cz;
-                    if ((unsigned)vx >= (unsigned)DHT_BX || (unsigned)vy >= (unsigned)DHT_BY ||
-                        (unsigned)vz >= (unsigned)DHT_BZ)
-                        continue;
                     const double w = wx[cx] * wy[cy] * wz[cz];
-                    atomicAdd(&acc[dht_lds(vx, vy, vz)], (unsigned long long)dround_i64(w * scale));
+                    atomicAdd(&A[cx + DHT_PY * cy + DHT_PZ * cz], (unsigned long long)dround_i64(w * scale));
                 }
             }
         }
@@ -1034,7 +1095,7 @@ int dht_setup(dht_ctx* c, const dht_params* p, int nang, const double* angZ_deg,
     g.nx = p->nx; g.ny = p->ny; g.method = p->method; g.escc = p->escc;
     g.use_f1 = p->norm_f1 != 1.0; g.use_f2 = p->norm_f2 != 0.0;
     g.f1 = (float)p->norm_f1; g.f2 = (float)p->norm_f2;
-    g.xst = p->xst; g.wl = p->wl;
+    g.xst = p->xst; g.rxst = 1.0 / p->xst; g.wl = p->wl;
     g.k2maxo = std::pow(p->aobj_mrad * (double)0.001f / p->wl, 2.0);  // DHT.cpp:250
     const double cs3 = p->cs3_mm * 1.e+7, cs5 = p->cs5_mm * 1.e+7;
     g.c3 = p->method != 4 ? -cs3 : cs3;  // iSign = -1 reverts the aberrations (DHT.cpp:962)

@@ -646,8 +646,12 @@ int launch_grid32(utr_ctx* c, float* d_S, hipEvent_t ev_start) {
                              ((g.ny + utr::SBY - 1) / utr::SBY) * ((g.nz + utr::SBZ - 1) / utr::SBZ);
         if (nblocks <= 0 || nblocks > 0x7fffffffL) return set_err(UTR_E_INVALID, "volume too large");
         if (ev_start) UTR_HIP_TRY(hipEventRecord(ev_start, c->stream));
-        utr::k_grid_fx<<<(unsigned)nblocks, 256, 0, c->stream>>>(c->spec32.p, c->rows.p, c->plan.nrows,
-                                                                 c->rowmax.p, g, c->V32.p, d_S);
+        if (g.rot_centre_shift)
+            utr::k_grid_fx<true><<<(unsigned)nblocks, 256, 0, c->stream>>>(c->spec32.p, c->rows.p, c->plan.nrows,
+                                                                          c->rowmax.p, g, c->V32.p, d_S);
+        else
+            utr::k_grid_fx<false><<<(unsigned)nblocks, 256, 0, c->stream>>>(c->spec32.p, c->rows.p, c->plan.nrows,
+                                                                           c->rowmax.p, g, c->V32.p, d_S);
     }
     UTR_HIP_TRY(hipGetLastError());
     return UTR_OK;

@@ -685,28 +685,44 @@ __global__ void __launch_bounds__(256) k_gather(const cplx<float>* __restrict__ 
 // One workgroup owns a brick of SBX x SBY x SBZ voxels.  It lists the rows
 // whose Ewald sheet can reach the brick (in row order) and, for each listed
 // row, the detector lines b whose points can splat into it.  Lines are
-// processed 256 at a time, one per thread: the thread bounds the a-interval
-// of its line that can land in the brick, evaluates each point's grid
-// position in FP64 (the same expressions as the CPU restatement), and adds
-// w*K (FP32 products) for the point's corners inside the brick.
+// clipped 256 at a time, one per thread, to the a-interval that can land in
+// the brick; each line gets a run of the brick's point list (a wave prefix
+// sum and one LDS add per wave) and writes its number into it.  Then every
+// thread takes points of the list: it evaluates the point's grid position in
+// FP64 (the same expressions as the CPU restatement) and adds w*K for the
+// point's eight corners.  With a line per lane (the form before) a wave
+// waited for its longest line and lanes loaded distant spectrum values; the
+// list keeps all lanes on consecutive values of a few lines.  The lists are
+// double buffered, so one barrier separates writing from reading.
 //
 // The sums are kept in LDS as 64-bit fixed-point integers, added with integer
 // LDS atomics (on gfx950 these cost no more than plain stores, while float
 // LDS atomics are several times slower).  Integer addition is associative, so
 // the sums are exact, independent of the order in which points arrive, and
 // the result is deterministic; the only rounding is that of each w*K product
-// and of its conversion to the fixed-point grid.  The scales come from the
-// largest spectrum component and the row count so that no sum can overflow:
-// V3 is resolved to about 1e-11 (in units of K), Samp3 to about 1e-15.
+// to the fixed-point grid.  The scales come from the largest spectrum
+// component and the row count so that no sum can overflow: V3 is resolved to
+// about 1e-11 (in units of K), Samp3 to about 1e-15.  A one-cell halo takes
+// the corners outside the brick, so corners need no bounds tests.
 // Weights below 2^-20 (rare: cells crossed within a millionth of a grid
-// plane, mostly at exact grid alignments) go instead to float accumulators,
+// plane, mostly at exact grid alignments) stay out of the fixed-point sums,
 // so a voxel reached only by such weights keeps the relative precision that
-// V3/Samp3 needs there and counts as sampled exactly as in the reference.
-// Corners of weight exactly zero are skipped (adding them changes nothing).
+// V3/Samp3 needs there and counts as sampled exactly as in the reference:
+// their points are recorded, the sums converted to FP64 in place and just
+// those corners' FP32 terms added in FP64 (in a second pass over all points
+// when more were met than the record holds).  Corners of weight exactly zero
+// add nothing.
 //
-// The fixed-point accumulators use odd strides (17 along y, 153 along z) so
-// that lanes walking along x, y or z, as the points of a detector line do for
-// any orientation, address distinct LDS banks.
+// The strides are odd (17 along y, 153 along z) so that points along x, y or
+// z address distinct LDS banks.  Bricks start from the volume's centre
+// outwards: every row's sheet passes it, so the central bricks hold 25 times
+// the points of an average one and would set the tail.
+// Of 553 us for 216 random rows of 256^2 into 256^3 (764 us before), the
+// points take about 230, listing the lines 180 (latency of a few rounds a
+// brick), zeroing, row tests and the V3 write 112, the CTF epilogue 70.  One
+// row per wave without barriers (rows in scalar registers) measured 523 us
+// there but 192 against 118 us for 108 rows of 192 x 160 into 192 x 160 x 96,
+// where a brick has fewer rows than waves.
 
 constexpr int SBX = 16, SBY = 8, SBZ = 8;
 constexpr int SVOX = SBX * SBY * SBZ;
@@ -714,12 +730,41 @@ constexpr int SOWN = SVOX / 256;  // voxels finalised per thread
 static_assert(SVOX % 256 == 0, "brick must be a multiple of the workgroup");
 constexpr int SPY = SBX + 1;           // LDS stride along y
 constexpr int SPZ = SPY * (SBY + 1);   // LDS stride along z
-constexpr int SPAD = SPZ * SBZ;        // LDS entries per component
+// LDS entries per component: cells of [-1, SBX] x [-1, SBY] x [-1, SBZ] (the
+// halo cells of neighbouring rows and planes share slots; they are not read)
+constexpr int SPAD = (SBX + 1) + SPY * (SBY + 1) + SPZ * (SBZ + 1) + 1;
 constexpr int S_LIST = 256;            // rows tested per chunk
+constexpr int S_POINTS = 3072;         // points listed at a time
+constexpr int S_TQ = 256;              // points with tiny corner weights recorded (one per thread)
 constexpr double S_TINY_D = 9.5367431640625e-07;  // 2^-20
 constexpr double S_TINY_1D = 9.765625e-04;         // 2^-10
 
-__device__ __forceinline__ int lds_idx(int lx, int ly, int lz) { return lx + SPY * ly + SPZ * lz; }
+__device__ __forceinline__ int lds_idx(int lx, int ly, int lz) { return (lx + 1) + SPY * (ly + 1) + SPZ * (lz + 1); }
+
+// Inclusive prefix sum over the wave's lanes in the vector unit (DPP row
+// shifts and broadcasts; through LDS permutes the six steps cost their
+// latency six times).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_or0(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+    v += dpp_or0<0x111, 0xf>(v);  // row_shr:1
+    v += dpp_or0<0x112, 0xf>(v);
+    v += dpp_or0<0x114, 0xf>(v);
+    v += dpp_or0<0x118, 0xf>(v);
+    v += dpp_or0<0x142, 0xa>(v);  // row_bcast:15
+    v += dpp_or0<0x143, 0xc>(v);  // row_bcast:31
+    return v;
+}
+
+// k-th index of 0 .. n-1 from the centre outwards
+__device__ __forceinline__ int centre_out(int k, int n) { return n / 2 + ((k & 1) ? -((k + 1) >> 1) : (k >> 1)); }
+
+template <bool B>
+struct PassKind {
+    static constexpr bool value = B;
+};
 
 // round(d) as a 64-bit integer for |d| < 2^51 (1.5 * 2^52 aligns the units
 // digit with the last mantissa bit; round to nearest even)
@@ -735,27 +780,37 @@ __device__ __forceinline__ long long fx_term(double w, double k) {
     return (long long)(__double_as_longlong(y) - 0x4338000000000000LL);
 }
 
-__global__ void __launch_bounds__(256, 3) k_grid_fx(const cplx<float>* __restrict__ spec,
+// ROT: rows carry the centre-shift phase (compiled separately: its FP64
+// sincos would otherwise set the register budget of the common case).
+template <bool ROT>
+__global__ void __launch_bounds__(256, ROT ? 2 : 3) k_grid_fx(const cplx<float>* __restrict__ spec,
                                                  const RowParams* __restrict__ rows, int nrows,
                                                  const unsigned* __restrict__ rowmax, GeomDev g,
                                                  cplx<float>* __restrict__ Vout,
                                                  float* __restrict__ Sout) {
-    __shared__ unsigned long long acc[3 * SPAD];
-    __shared__ float tiny[3 * SVOX];
+    __shared__ unsigned long long acc[3 * SPAD];  // fixed-point sums (FP64 after a tiny-weight pass)
     __shared__ float s_red[4];
     __shared__ int s_list[S_LIST];     // rows reaching the brick, in row order
     __shared__ int s_lo[S_LIST];       // first detector line of each listed row
     __shared__ int s_pre[S_LIST + 1];  // line counts, then their exclusive prefix
     __shared__ int s_cnt[4], s_wsum[4];
     __shared__ int s_n;
+    __shared__ int2 s_line[2][256];                  // row; b << 16 | (a - point number) & 0xffff
+    __shared__ unsigned char s_pt[2][S_POINTS];      // line of each listed point
+    __shared__ int s_tot[3];                         // points of a round
+    __shared__ int2 s_tq[S_TQ];                      // points with a corner weight below 2^-20 (row; b << 16 | a)
+    __shared__ int s_tn;                             // their count (may exceed S_TQ)
+    double* const accd = reinterpret_cast<double*>(acc);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nbx = (g.nx + SBX - 1) / SBX, nby = (g.ny + SBY - 1) / SBY;
+    const int nbx = (g.nx + SBX - 1) / SBX, nby = (g.ny + SBY - 1) / SBY, nbz = (g.nz + SBZ - 1) / SBZ;
     const int bid = blockIdx.x;
-    const int bx = bid % nbx, by = (bid / nbx) % nby, bz = bid / (nbx * nby);
+    const int bx = centre_out(bid % nbx, nbx), by = centre_out((bid / nbx) % nby, nby),
+              bz = centre_out(bid / (nbx * nby), nbz);
     const int x0 = bx * SBX, y0 = by * SBY, z0 = bz * SBZ;
     for (int t = tid; t < 3 * SPAD; t += 256) acc[t] = 0ull;
-    for (int t = tid; t < 3 * SVOX; t += 256) tiny[t] = 0.f;
+    if (tid < 3) s_tot[tid] = 0;
+    if (tid == 0) s_tn = 0;
     // fixed-point scales: 2^sv for V3, 2^sw for Samp3.  Per row a voxel
     // receives a total weight below 8, so |sum| < 8 nrows max|K| 2^sv < 2^62;
     // each term stays below 2^51 for fx_term.
@@ -771,6 +826,7 @@ __global__ void __launch_bounds__(256, 3) k_grid_fx(const cplx<float>* __restric
     const int sv = min(61 - ek - ea, 50 - ek);
     const int sw = min(61 - ea, 50);
     const double vscale = ldexp(1.0, sv), wscale = ldexp(1.0, sw);
+    const double vinv = ldexp(1.0, -sv), winv = ldexp(1.0, -sw);
 
     const float fx2 = (float)(g.fxst * g.fxst), fy2 = (float)(g.fyst * g.fyst);
     const float wl2f = (float)g.wl2;
@@ -782,19 +838,106 @@ __global__ void __launch_bounds__(256, 3) k_grid_fx(const cplx<float>* __restric
     const float bmax[3] = {(float)(x0 + SBX - 1), (float)(y0 + SBY - 1), (float)(z0 + SBZ - 1)};
     const float cgrid[3] = {(float)g.nxd2, (float)g.nyd2, (float)g.nzd2};
 
-    for (int base = 0; base < nrows; base += S_LIST) {
-        const int nchunk = min(S_LIST, nrows - base);
-        if (tid == 0) s_n = 0;
-        __syncthreads();
-        // rows whose sheet can reach the brick, with their detector lines
-        for (int r0 = 0; r0 < nchunk; r0 += 256) {
-            const int r = r0 + tid;
-            bool pass = false;
+    // One point (a, b) of row r.  FIX false: the fixed-point terms of every
+    // corner of weight >= 2^-20, and the point recorded when a smaller nonzero
+    // one is in the brick.  FIX true: only those small corners, their FP32
+    // terms added in FP64 to the converted sums.
+    struct Point {
+        int r, a, b;
+        cplx<float> k;
+        double m[9];
+    };
+    auto load = [&](const int r, const int a, const int b) {
+        Point q;
+        q.r = r;
+        q.a = a;
+        q.b = b;
+        q.k = spec[((size_t)r * g.ny + (b + g.nyd2)) * g.nx + (a + g.nxd2)];
+#pragma unroll
+        for (int t = 0; t < 9; t++) q.m[t] = t == 7 ? 0.0 : rows[r].m[t];
+        return q;
+    };
+    auto splat = [&](auto kind, const Point& q) {
+        constexpr bool FIX = decltype(kind)::value;
+        const int r = q.r, a = q.a, b = q.b;
+        const RowParams& R = rows[r];
+        const cplx<float> kraw = q.k;
+        const GridPos P = grid_pos(g, q.m, a, b);
+        const double fnn = floor(P.dz1), fii = floor(P.dx1), fjj = floor(P.dy1);
+        if (fnn < 0.0 || fnn > (double)(g.nz - 2)) return;
+        if (fii < 0.0 || fii > (double)(g.nx - 2)) return;
+        if (fjj < 0.0 || fjj > (double)(g.ny - 2)) return;
+        const int ii = (int)fii - x0, jj = (int)fjj - y0, nn = (int)fnn - z0;
+        if (ii < -1 || ii >= SBX || jj < -1 || jj >= SBY || nn < -1 || nn >= SBZ) return;
+        const double fx = P.dx1 - fii, fy = P.dy1 - fjj, fz = P.dz1 - fnn;
+        const double wxs[2] = {1.0 - fx, fx}, wys[2] = {1.0 - fy, fy}, wzs[2] = {1.0 - fz, fz};
+        // the smallest nonzero corner weight (a fraction of 0 has one corner)
+        const double mx = fx == 0.0 ? 1.0 : fmin(wxs[0], wxs[1]), my = fy == 0.0 ? 1.0 : fmin(wys[0], wys[1]),
+                     mz = fz == 0.0 ? 1.0 : fmin(wzs[0], wzs[1]);
+        const bool near = mx * my * mz < S_TINY_D;
+        if (FIX && !near) return;
+        cplx<float> kv = kraw;
+        if (ROT) {
+            const double phs = -(R.ph[0] * P.ox + R.ph[1] * P.oy + R.ph[2] * P.oz);
+            double sn, c;
+            sincos(phs, &sn, &c);
+            const float cf = (float)c, sf = (float)sn;
+            kv = {kraw.x * cf - kraw.y * sf, kraw.x * sf + kraw.y * cf};
+        }
+        const int li0 = lds_idx(ii, jj, nn);
+        double wds[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) wds[c] = wxs[c & 1] * wys[(c >> 1) & 1] * wzs[c >> 2];
+        if (near) {
+            bool any_tiny = false;
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                const bool tny = wds[c] != 0.0 && wds[c] < S_TINY_D;
+                const bool inb = (unsigned)(ii + (c & 1)) < (unsigned)SBX &&
+                                 (unsigned)(jj + ((c >> 1) & 1)) < (unsigned)SBY &&
+                                 (unsigned)(nn + (c >> 2)) < (unsigned)SBZ;
+                if (FIX) {
+                    if (!(tny && inb)) continue;
+                    const int li = li0 + (c & 1) + SPY * ((c >> 1) & 1) + SPZ * (c >> 2);
+                    const float w = (float)wds[c];
+                    atomicAdd(&accd[li], (double)(w * kv.x));
+                    atomicAdd(&accd[SPAD + li], (double)(w * kv.y));
+                    atomicAdd(&accd[2 * SPAD + li], (double)w);
+                } else {
+                    any_tiny |= tny && inb;
+                    if (tny) wds[c] = 0.0;
+                }
+            }
+            if (!FIX && any_tiny) {
+                const int slot = atomicAdd(&s_tn, 1);
+                if (slot < S_TQ) s_tq[slot] = int2{r, (int)((unsigned)b << 16 | ((unsigned)a & 0xffffu))};
+            }
+        }
+        if (FIX) return;
+        // the spectrum value on the V3 fixed-point grid (exact: a power of two)
+        const double kxs = (double)kv.x * vscale, kys = (double)kv.y * vscale;
+        unsigned long long* A = acc + li0;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const int li = (c & 1) + SPY * ((c >> 1) & 1) + SPZ * (c >> 2);
+            atomicAdd(&A[li], (unsigned long long)fx_term(wds[c], kxs));
+            atomicAdd(&A[SPAD + li], (unsigned long long)fx_term(wds[c], kys));
+            atomicAdd(&A[2 * SPAD + li], (unsigned long long)fx_term(wds[c], wscale));
+        }
+    };
+
+    int round = 0;
+    // one pass of splat over all points that can reach the brick
+    auto pass = [&](auto kind) {
+        for (int base = 0; base < nrows; base += S_LIST) {
+            const int nchunk = min(S_LIST, nrows - base);
+            // rows whose sheet can reach the brick, with their detector lines
+            bool touch = false;
             int blo = 0, nl = 0;
-            if (r < nchunk) {
-                const RowParams& R = rows[base + r];
-                pass = brick_touch(g, R, bcx, bcy, bcz, ex, ey, ez, fx2, fy2, wl2f);
-                if (pass) {
+            if (tid < nchunk) {
+                const RowParams& R = rows[base + tid];
+                touch = brick_touch(g, R, bcx, bcy, bcz, ex, ey, ez, fx2, fy2, wl2f);
+                if (touch) {
                     int bhi;
                     if (R.y_exact) {
                         // y grid coordinate is ny/2 + b exactly: lines outside the
@@ -808,274 +951,142 @@ __global__ void __launch_bounds__(256, 3) k_grid_fx(const cplx<float>* __restric
                         blo = max((int)ceilf(t - Wb), -g.nyd2);
                         bhi = min((int)floorf(t + Wb), g.ny - 1 - g.nyd2);
                     }
-                    nl = bhi - blo + 1;
-                    pass = nl > 0;
+                    nl = max(bhi - blo + 1, 0);
+                    touch = nl > 0;
                 }
             }
-            const unsigned long long mask = __ballot(pass);
+            // list them in row order with the exclusive prefix of their lines
+            const unsigned long long mask = __ballot(touch);
             const int pre = __popcll(mask & ((1ull << lane) - 1ull));
-            if (lane == 0) s_cnt[wave] = __popcll(mask);
-            __syncthreads();
-            int off = s_n;
-            for (int w = 0; w < wave; w++) off += s_cnt[w];
-            if (pass) {
-                s_list[off + pre] = base + r;
-                s_lo[off + pre] = blo;
-                s_pre[off + pre] = nl;
+            const int incl = wave_prefix_sum(nl);
+            __syncthreads();  // the previous chunk's list is no longer read
+            if (lane == 63) {
+                s_cnt[wave] = __popcll(mask);
+                s_wsum[wave] = incl;
             }
             __syncthreads();
-            if (tid == 0) s_n += s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
-            __syncthreads();
-        }
-        const int n = s_n;
-        // exclusive prefix of the line counts (two entries per thread)
-        {
-            const int c0 = (2 * tid < n) ? s_pre[2 * tid] : 0;
-            const int c1 = (2 * tid + 1 < n) ? s_pre[2 * tid + 1] : 0;
-            const int pair = c0 + c1;
-            int incl = pair;
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(incl, o);
-                if (lane >= o) incl += v;
+            int off = pre, loff = incl - nl;
+            for (int w = 0; w < wave; w++) {
+                off += s_cnt[w];
+                loff += s_wsum[w];
             }
-            if (lane == 63) s_wsum[wave] = incl;
+            if (touch) {
+                s_list[off] = base + tid;
+                s_lo[off] = blo;
+                s_pre[off] = loff;
+            }
+            const int n = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
+            const int total = s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3];
             __syncthreads();
-            int woff = 0;
-            for (int w = 0; w < wave; w++) woff += s_wsum[w];
-            const int excl = woff + incl - pair;
-            if (2 * tid < n) s_pre[2 * tid] = excl;
-            if (2 * tid + 1 < n) s_pre[2 * tid + 1] = excl + c0;
-            if (tid == 0) s_pre[n] = s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3];
-            __syncthreads();
-        }
-        const int total = s_pre[n];
-        for (int G = 0; G < total; G += 256) {
-            const int gl = G + tid;
-            if (gl < total) {
-                // listed row q holding global line gl: last q with s_pre[q] <= gl
-                int lo = 0, hi = n - 1;
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (s_pre[mid] <= gl) lo = mid;
-                    else hi = mid - 1;
-                }
-                const int r = s_list[lo];
-                const int b = s_lo[lo] + (gl - s_pre[lo]);
-                const RowParams& R = rows[r];
-                const float* mi = R.minv;
-                // a-interval of this line whose points can land in the brick
-                const float s = mi[0] * bcx + mi[1] * bcy + mi[2] * bcz;
-                const float Wa = fabsf(mi[0]) * ex + fabsf(mi[1]) * ey + fabsf(mi[2]) * ez + 0.01f;
-                float alo = fmaxf(s - Wa, (float)(-g.nxd2));
-                float ahi = fminf(s + Wa, (float)(g.nx - 1 - g.nxd2));
-                double m[9];
+            for (int G = 0; G < total; G += 256, round++) {
+                const int gl = G + tid, buf = round & 1;
+                int cnt = 0, a0 = 0, r = 0, b = 0;
+                if (tid == 0) s_tot[(round + 1) % 3] = 0;
+                if (gl < total) {
+                    // listed row q holding line gl: last q with s_pre[q] <= gl
+                    int lo = 0, hi = n - 1;
+                    while (lo < hi) {
+                        const int mid = (lo + hi + 1) >> 1;
+                        if (s_pre[mid] <= gl) lo = mid;
+                        else hi = mid - 1;
+                    }
+                    r = s_list[lo];
+                    b = s_lo[lo] + (gl - s_pre[lo]);
+                    const RowParams& R = rows[r];
+                    const float* mi = R.minv;
+                    // a-interval of this line whose points can land in the brick
+                    const float s = mi[0] * bcx + mi[1] * bcy + mi[2] * bcz;
+                    const float Wa = fabsf(mi[0]) * ex + fabsf(mi[1]) * ey + fabsf(mi[2]) * ez + 0.01f;
+                    float alo = fmaxf(s - Wa, (float)(-g.nxd2));
+                    float ahi = fminf(s + Wa, (float)(g.nx - 1 - g.nxd2));
+                    if (alo <= ahi) {
+                        const float ac = 0.5f * (alo + ahi), W = 0.5f * (ahi - alo);
+                        const float fb = (float)b;
+                        const float zz0 = g.escc ? -wl2f * (fx2 * ac * ac + fy2 * fb * fb) : 0.f;
+                        const float dzz = g.escc ? -2.f * wl2f * fx2 * ac : 0.f;
+                        const float curv = g.escc ? wl2f * fx2 * W * W : 0.f;
 #pragma unroll
-                for (int t = 0; t < 9; t++) m[t] = R.m[t];
-                if (alo <= ahi) {
-                    const float ac = 0.5f * (alo + ahi), W = 0.5f * (ahi - alo);
-                    const float fb = (float)b;
-                    const float zz0 = g.escc ? -wl2f * (fx2 * ac * ac + fy2 * fb * fb) : 0.f;
-                    const float dzz = g.escc ? -2.f * wl2f * fx2 * ac : 0.f;
-                    const float curv = g.escc ? wl2f * fx2 * W * W : 0.f;
-#pragma unroll
-                    for (int d = 0; d < 3; d++) {
-                        const float m0 = (float)m[3 * d], m1 = (float)m[3 * d + 1], m2 = (float)m[3 * d + 2];
-                        const float Pc = cgrid[d] + m0 * ac + m1 * fb + m2 * zz0;
-                        const float Pd = m0 + m2 * dzz;
-                        const float mg = fabsf(m2) * curv * 1.01f + 2e-4f * (1.f + fabsf(Pc)) + 0.01f;
-                        const float lo_d = bmin[d] - 1.f - mg - Pc, hi_d = bmax[d] + 1.f + mg - Pc;
-                        if (fabsf(Pd) < 1e-6f) {
-                            if (lo_d > 0.f || hi_d < 0.f) alo = ahi + 1.f;
-                        } else {
-                            // the margins above exceed the 1-ulp error of the reciprocal
-                            const float rp = __builtin_amdgcn_rcpf(Pd);
-                            float t0 = lo_d * rp, t1 = hi_d * rp;
-                            if (Pd < 0.f) { const float tt = t0; t0 = t1; t1 = tt; }
-                            alo = fmaxf(alo, ac + t0);
-                            ahi = fminf(ahi, ac + t1);
+                        for (int d = 0; d < 3; d++) {
+                            const float m0 = (float)R.m[3 * d], m1 = (float)R.m[3 * d + 1], m2 = (float)R.m[3 * d + 2];
+                            const float Pc = cgrid[d] + m0 * ac + m1 * fb + m2 * zz0;
+                            const float Pd = m0 + m2 * dzz;
+                            const float mg = fabsf(m2) * curv * 1.01f + 2e-4f * (1.f + fabsf(Pc)) + 0.01f;
+                            const float lo_d = bmin[d] - 1.f - mg - Pc, hi_d = bmax[d] + 1.f + mg - Pc;
+                            if (fabsf(Pd) < 1e-6f) {
+                                if (lo_d > 0.f || hi_d < 0.f) alo = ahi + 1.f;
+                            } else {
+                                // the margins above exceed the 1-ulp error of the reciprocal
+                                const float rp = __builtin_amdgcn_rcpf(Pd);
+                                const float t0 = lo_d * rp, t1 = hi_d * rp;
+                                alo = fmaxf(alo, ac + fminf(t0, t1));
+                                ahi = fminf(ahi, ac + fmaxf(t0, t1));
+                            }
                         }
                     }
+                    if (alo <= ahi) {
+                        a0 = max((int)ceilf(alo - 1e-3f), -g.nxd2);
+                        cnt = max(min((int)floorf(ahi + 1e-3f), g.nx - 1 - g.nxd2) - a0 + 1, 0);
+                    }
                 }
-                int a0 = 0, a1 = -1;
-                if (alo <= ahi) {
-                    a0 = max((int)ceilf(alo - 1e-3f), -g.nxd2);
-                    a1 = min((int)floorf(ahi + 1e-3f), g.nx - 1 - g.nxd2);
-                }
-                const cplx<float>* Kline = spec + ((size_t)r * g.ny + (b + g.nyd2)) * g.nx + g.nxd2;
-                double ph[3] = {0.0, 0.0, 0.0};
-                if (g.rot_centre_shift) {
-                    ph[0] = R.ph[0];
-                    ph[1] = R.ph[1];
-                    ph[2] = R.ph[2];
-                }
-                if (R.y_exact) {
-                    // No rotation about Z: the point's y grid coordinate is ny/2 + b
-                    // exactly (weight 1 on its own plane, 0 on the next), so only the
-                    // four (x, z) corners can receive weight.  Same expressions as
-                    // grid_pos, so the result is bit-identical to the general path.
-                    const int jjg = b + g.nyd2;
-                    const int ly = jjg - y0;
-                    if (jjg <= g.ny - 2 && ly >= 0 && ly < SBY) {
-                        const double bd = (double)b;
-                        const double qy = __dmul_rn(g.fyst, bd);
-                        const double qy2 = __dmul_rn(qy, qy);
-                        // one detector point: position, corner terms, LDS adds
-                        auto splat = [&](const int a, const cplx<float> kraw) {
-                            const double ad = (double)a;
-                            const double qx = __dmul_rn(g.fxst, ad);
-                            const double zz = g.escc ? __dmul_rn(-g.wl2, __fma_rn(qx, qx, qy2)) : 0.0;
-                            const double ox = __fma_rn(ad, m[0], __fma_rn(bd, m[1], __dmul_rn(zz, m[2])));
-                            const double oz = __fma_rn(ad, m[6], __dmul_rn(zz, m[8]));
-                            const double dx1 = __dadd_rn((double)g.nxd2, ox);
-                            const double dz1 = __dadd_rn((double)g.nzd2, oz);
-                            const double fnn = floor(dz1), fii = floor(dx1);
-                            if (fnn < 0.0 || fnn > (double)(g.nz - 2)) return;
-                            if (fii < 0.0 || fii > (double)(g.nx - 2)) return;
-                            const int ii = (int)fii - x0, nn = (int)fnn - z0;
-                            if (ii < -1 || ii >= SBX || nn < -1 || nn >= SBZ) return;
-                            const double fx = dx1 - fii, fz = dz1 - fnn;
-                            const double wxs[2] = {1.0 - fx, fx}, wzs[2] = {1.0 - fz, fz};
-                            cplx<float> kv = kraw;
-                            if (g.rot_centre_shift) {
-                                const double phs = -(ph[0] * ox + ph[1] * bd + ph[2] * oz);
-                                double sn, c;
-                                sincos(phs, &sn, &c);
-                                const float cf = (float)c, sf = (float)sn;
-                                kv = {kraw.x * cf - kraw.y * sf, kraw.x * sf + kraw.y * cf};
-                            }
-                            // the spectrum value on the V3 fixed-point grid (exact: a power of two)
-                            const double kxs = (double)kv.x * vscale, kys = (double)kv.y * vscale;
-                            long long tr[4], ti[4], tw[4];
-                            float wc[4];
-                            bool big[4], tny[4];
-                            bool any_tiny = false;
-#pragma unroll
-                            for (int c = 0; c < 4; c++) {
-                                const int cx = c & 1, cz = c >> 1;
-                                const bool inb = (unsigned)(ii + cx) < (unsigned)SBX &&
-                                                 (unsigned)(nn + cz) < (unsigned)SBZ;
-                                const double wd = wxs[cx] * 1.0 * wzs[cz];
-                                big[c] = inb && wd >= S_TINY_D;
-                                tny[c] = inb && wd != 0.0 && wd < S_TINY_D;
-                                any_tiny |= tny[c];
-                                wc[c] = (float)wd;
-                                tr[c] = fx_term(wd, kxs);
-                                ti[c] = fx_term(wd, kys);
-                                tw[c] = fx_term(wd, wscale);
-                            }
-                            const int li0 = lds_idx(ii, ly, nn);
-#pragma unroll
-                            for (int c = 0; c < 4; c++) {
-                                if (!big[c]) continue;
-                                const int li = li0 + (c & 1) + SPZ * (c >> 1);
-                                atomicAdd(&acc[li], (unsigned long long)tr[c]);
-                                atomicAdd(&acc[SPAD + li], (unsigned long long)ti[c]);
-                                atomicAdd(&acc[2 * SPAD + li], (unsigned long long)tw[c]);
-                            }
-                            if (any_tiny) {
-#pragma unroll
-                                for (int c = 0; c < 4; c++) {
-                                    const int lx = ii + (c & 1), lz = nn + (c >> 1);
-                                    const float w = wc[c];
-                                    if (!tny[c]) continue;
-                                    const int v = lx + SBX * (ly + SBY * lz);
-                                    atomicAdd(&tiny[v], w * kv.x);
-                                    atomicAdd(&tiny[SVOX + v], w * kv.y);
-                                    atomicAdd(&tiny[2 * SVOX + v], w);
-                                }
-                            }
-                        };
-                        // two points in flight without register moves between the
-                        // loads and their use (clamped indices keep loads in the line)
-                        cplx<float> kA = {0.f, 0.f}, kB = {0.f, 0.f};
-                        if (a0 <= a1) {
-                            kA = Kline[a0];
-                            kB = Kline[min(a0 + 1, a1)];
-                        }
-                        for (int a = a0; a <= a1; a += 2) {
-                            splat(a, kA);
-                            kA = Kline[min(a + 2, a1)];
-                            if (a + 1 <= a1) splat(a + 1, kB);
-                            kB = Kline[min(a + 3, a1)];
+                const int inc = wave_prefix_sum(cnt);
+                int first = 0;
+                if (lane == 63) first = atomicAdd(&s_tot[round % 3], inc);
+                const int pos = __builtin_amdgcn_readlane(first, 63) + inc - cnt;
+                s_line[buf][tid] = int2{r, (int)((unsigned)b << 16 | ((unsigned)(a0 - pos) & 0xffffu))};
+                for (int q = 0; q < cnt && pos + q < S_POINTS; q++) s_pt[buf][pos + q] = (unsigned char)tid;
+                __syncthreads();
+                const int np = s_tot[round % 3];
+                for (int w0 = 0;;) {
+                    const int wn = min(np - w0, S_POINTS);
+                    // the next point's loads are in flight while one is splatted
+                    auto fetch = [&](const int p) {
+                        const int2 ln = s_line[buf][s_pt[buf][p]];
+                        return load(ln.x, (int)(short)((ln.y & 0xffff) + w0 + p), ln.y >> 16);
+                    };
+                    if (tid < wn) {
+                        Point cur = fetch(tid);
+                        for (int p = tid; p < wn; p += 256) {
+                            const Point nxt = fetch(min(p + 256, wn - 1));
+                            splat(kind, cur);
+                            cur = nxt;
                         }
                     }
-                } else {
-                // the next point's value is loaded while this one is splatted
-                cplx<float> knext = {0.f, 0.f};
-                if (a0 <= a1) knext = Kline[a0];
-                for (int a = a0; a <= a1; a++) {
-                    const cplx<float> kraw = knext;
-                    if (a < a1) knext = Kline[a + 1];
-                    const GridPos P = grid_pos(g, m, a, b);
-                    const double fnn = floor(P.dz1), fii = floor(P.dx1), fjj = floor(P.dy1);
-                    if (fnn < 0.0 || fnn > (double)(g.nz - 2)) continue;
-                    if (fii < 0.0 || fii > (double)(g.nx - 2)) continue;
-                    if (fjj < 0.0 || fjj > (double)(g.ny - 2)) continue;
-                    const int ii = (int)fii - x0, jj = (int)fjj - y0, nn = (int)fnn - z0;
-                    if (ii < -1 || ii >= SBX || jj < -1 || jj >= SBY || nn < -1 || nn >= SBZ) continue;
-                    const double fx = P.dx1 - fii, fy = P.dy1 - fjj, fz = P.dz1 - fnn;
-                    const double wxs[2] = {1.0 - fx, fx}, wys[2] = {1.0 - fy, fy}, wzs[2] = {1.0 - fz, fz};
-                    cplx<float> kv = kraw;
-                    if (g.rot_centre_shift) {
-                        const double phs = -(ph[0] * P.ox + ph[1] * P.oy + ph[2] * P.oz);
-                        double sn, c;
-                        sincos(phs, &sn, &c);
-                        const float cf = (float)c, sf = (float)sn;
-                        kv = {kraw.x * cf - kraw.y * sf, kraw.x * sf + kraw.y * cf};
-                    }
-                    // the eight corners' terms are formed first, without branches, so
-                    // that their independent chains overlap; then each corner inside
-                    // the brick adds its terms
-                    // the spectrum value on the V3 fixed-point grid (exact: a power of two)
-                    const double kxs = (double)kv.x * vscale, kys = (double)kv.y * vscale;
-                    long long tr[8], ti[8], tw[8];
-                    float wc[8];
-                    bool big[8], tny[8];
-                    bool any_tiny = false;
-#pragma unroll
-                    for (int c = 0; c < 8; c++) {
-                        const int cx = c & 1, cy = (c >> 1) & 1, cz = c >> 2;
-                        const bool inb = (unsigned)(ii + cx) < (unsigned)SBX &&
-                                         (unsigned)(jj + cy) < (unsigned)SBY &&
-                                         (unsigned)(nn + cz) < (unsigned)SBZ;
-                        const double wd = wxs[cx] * wys[cy] * wzs[cz];
-                        big[c] = inb && wd >= S_TINY_D;
-                        tny[c] = inb && wd != 0.0 && wd < S_TINY_D;
-                        any_tiny |= tny[c];
-                        wc[c] = (float)wd;
-                        tr[c] = fx_term(wd, kxs);
-                        ti[c] = fx_term(wd, kys);
-                        tw[c] = fx_term(wd, wscale);
-                    }
-                    const int li0 = lds_idx(ii, jj, nn);
-#pragma unroll
-                    for (int c = 0; c < 8; c++) {
-                        if (!big[c]) continue;
-                        const int li = li0 + (c & 1) + SPY * ((c >> 1) & 1) + SPZ * (c >> 2);
-                        atomicAdd(&acc[li], (unsigned long long)tr[c]);
-                        atomicAdd(&acc[SPAD + li], (unsigned long long)ti[c]);
-                        atomicAdd(&acc[2 * SPAD + li], (unsigned long long)tw[c]);
-                    }
-                    if (any_tiny) {
-                        // weights below 2^-20: float accumulators (rare)
-#pragma unroll
-                        for (int c = 0; c < 8; c++) {
-                            const int lx = ii + (c & 1), ly = jj + ((c >> 1) & 1), lz = nn + (c >> 2);
-                            const float w = wc[c];
-                            if (!tny[c]) continue;
-                            const int v = lx + SBX * (ly + SBY * lz);
-                            atomicAdd(&tiny[v], w * kv.x);
-                            atomicAdd(&tiny[SVOX + v], w * kv.y);
-                            atomicAdd(&tiny[2 * SVOX + v], w);
-                        }
-                    }
-                }
+                    w0 += S_POINTS;
+                    if (w0 >= np) break;
+                    // the list's next part (steps along the line shorter than a
+                    // voxel: volumes thinner than the images)
+                    __syncthreads();
+                    for (int q = max(0, w0 - pos); q < cnt && pos + q < w0 + S_POINTS; q++)
+                        s_pt[buf][pos + q - w0] = (unsigned char)tid;
+                    __syncthreads();
                 }
             }
         }
         __syncthreads();
+    };
+    pass(PassKind<false>{});
+    const int tn = s_tn;  // same in all threads
+    const bool fixd = tn != 0;
+    if (fixd) {
+#pragma unroll
+        for (int k = 0; k < SOWN; k++) {
+            const int v = tid + 256 * k;
+            const int li = lds_idx(v % SBX, (v / SBX) % SBY, v / (SBX * SBY));
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const double d = (double)(long long)acc[c * SPAD + li] * (c < 2 ? vinv : winv);
+                accd[c * SPAD + li] = d;
+            }
+        }
+        __syncthreads();
+        if (tn <= S_TQ) {
+            if (tid < tn)
+                splat(PassKind<true>{}, load(s_tq[tid].x, (int)(short)(s_tq[tid].y & 0xffff), s_tq[tid].y >> 16));
+        } else {
+            pass(PassKind<true>{});
+        }
+        __syncthreads();
     }
-    const double vinv = ldexp(1.0, -sv), winv = ldexp(1.0, -sw);
 #pragma unroll
     for (int k = 0; k < SOWN; k++) {
         const int v = tid + 256 * k;
@@ -1083,9 +1094,16 @@ __global__ void __launch_bounds__(256, 3) k_grid_fx(const cplx<float>* __restric
         const int vx = x0 + lx, vy = y0 + ly, vz = z0 + lz;
         if (vx >= g.nx || vy >= g.ny || vz >= g.nz) continue;
         const int li = lds_idx(lx, ly, lz);
-        const float vr = (float)((double)(long long)acc[li] * vinv + (double)tiny[v]);
-        const float vi = (float)((double)(long long)acc[SPAD + li] * vinv + (double)tiny[SVOX + v]);
-        const float S = (float)((double)(long long)acc[2 * SPAD + li] * winv + (double)tiny[2 * SVOX + v]);
+        float vr, vi, S;
+        if (fixd) {
+            vr = (float)accd[li];
+            vi = (float)accd[SPAD + li];
+            S = (float)accd[2 * SPAD + li];
+        } else {
+            vr = (float)((double)(long long)acc[li] * vinv);
+            vi = (float)((double)(long long)acc[SPAD + li] * vinv);
+            S = (float)((double)(long long)acc[2 * SPAD + li] * winv);
+        }
         const size_t vidx = ((size_t)vz * g.ny + vy) * g.nx + vx;
         if (Sout) Sout[vidx] = S;
         Vout[vidx] = voxel_epilogue<float>(g, vx, vy, vz, cplx<float>{vr, vi}, S);
@@ -1227,11 +1245,6 @@ __host__ __device__ constexpr unsigned yp_grid(int ntiles, int ngroups) {
 // LDS then holds only the fixed-point sums (with their halo), the list and
 // the record (31 KB), and the noise-gate instantiation fits 96 VGPRs: 5
 // workgroups per CU.
-template <bool B>
-struct PassKind {
-    static constexpr bool value = B;
-};
-
 template <bool ROT, bool GATE, int PL>
 __global__ void __launch_bounds__(256, ROT ? 1 : (GATE && PL <= P_LIST_S ? 5 : 4)) k_grid_yp(const cplx<float>* __restrict__ spec,
                                                  const RowParams* __restrict__ rows,

@@ -10,11 +10,11 @@
 //
 // All orientations of a batch advance through the slices together, so
 // every launch covers B images.  Per slice:
-//   k_ms_potential    projected potential of the slice's atoms, summed per
+//   k_ms_potential_rows  projected potential of the slice's atoms, summed per
 //                     pixel (atom order, float) and turned into the
 //                     transmission function exp(i sigma V)
 //                     (autoslic.cpp:917-990)
-//   k_post_lines      x FFT (exponent +1, cfpix::fft) of the transmission
+//                     and its x FFT (exponent +1, cfpix::fft)
 //   k_ms_cols<0>      y FFT, bandwidth limit k^2 < k2max, y inverse FFT
 //                     (autoslic.cpp:992-1006)
 //   k_ms_mul          x inverse FFTs of transmission and wave, product, x FFT
@@ -31,11 +31,20 @@
 namespace utr {
 
 constexpr int MS_NR = 100;  // radii of the potential look-up table (slicelib.cpp:2818-2820)
-// LDS budget (bytes of one buffer) of the column and product kernels.
-// 8192 (4 columns of 256 per workgroup) measured faster than 16384 (8
-// columns, fewer resident workgroups): 96 against 124 us per column pass
-// over 360 images of 256^2.
-constexpr int MS_LDS = 8192;
+// Columns kept by the bandwidth limit: kx < lim or kx > nx - lim (lim is the
+// first kx with kx2 >= k2max; nx: all).  The transmission after its limit and
+// the wave after every propagation are zero in the others, a third of a square
+// image's, so no kernel reads or writes them: they hold stale values.
+__device__ __forceinline__ bool ms_kept(int kx, int nx, int lim) { return kx < lim || kx > nx - lim; }
+// Column tiles of w columns with a kept column, and the t-th of them.
+__host__ __device__ inline int ms_tiles(int nx, int w, int lim) {
+    const int all = (nx + w - 1) / w, left = (lim + w - 1) / w, right = (nx - lim + 1) / w;
+    return left >= right ? all : left + (all - right);
+}
+__device__ __forceinline__ int ms_tile(int t, int nx, int w, int lim) {
+    const int left = (lim + w - 1) / w, right = (nx - lim + 1) / w;
+    return left >= right || t < left ? t : right + (t - left);
+}
 
 struct alignas(16) MsAtom {
     float x, y, occ;
@@ -54,6 +63,9 @@ __device__ __forceinline__ int ms_pmod(int a, int n) {
     const int r = a % n;
     return r < 0 ? r + n : r;
 }
+
+// rx^2 + ry^2 with the rounding fixed, so that every kernel forms the same
+__device__ __forceinline__ double ms_r2(double rx, double ry) { return __fma_rn(rx, rx, __dmul_rn(ry, ry)); }
 
 // vzatomLUT (slicelib.cpp:2868-2886): interval of seval (below the first
 // knot 0, at or above the next-to-last n-2, else x[i] <= r2 < x[i+1]) and the
@@ -132,7 +144,7 @@ __global__ void __launch_bounds__(256) k_ms_potential(const MsAtom* __restrict__
             if (iy > t.iyo + g.idy) continue;
             const double rx = (double)t.x - (double)ix * g.sx;
             const double ry = (double)t.y - (double)iy * g.sy;
-            double r2 = rx * rx + ry * ry;
+            double r2 = ms_r2(rx, ry);
             if (r2 > 9.0) continue;
             if (r2 < g.rminsq) r2 = g.rminsq;
             acc += (float)((double)t.occ * ms_lut(knots, coef + (size_t)t.zi * MS_NR, r2, g));
@@ -143,41 +155,44 @@ __global__ void __launch_bounds__(256) k_ms_potential(const MsAtom* __restrict__
     trans[((size_t)o * g.ny + py) * g.nx + px] = {cs, sn};
 }
 
-// The same potential for NB whole rows of one orientation, followed by the
-// rows' x FFT (exponent +1) in LDS, so the transmission function reaches
-// HBM once, already x-transformed (k_ms_potential + k_post_lines in one
-// pass; the sums, the FFT and so the result are the same bit for bit).
-// grid (row groups, orientation).
+// The same potential for whole rows of one orientation, followed by the rows'
+// x FFT (exponent +1), so the transmission function reaches HBM once, already
+// x-transformed (k_ms_potential + k_ms_lines in one pass; the sums, the FFT and
+// so the result are the same bit for bit), kept columns only unless raw.
+// A thread holds pixels i + M r of one row (Fft), M pixels apart: where that is
+// wider than an atom's window at most one of them meets it, found without a
+// test per pixel.  grid (row groups, orientation).
 template <int N>
-__global__ void __launch_bounds__(256) k_ms_potential_rows(const MsAtom* __restrict__ atoms,
+__global__ void __launch_bounds__(Fft<N>::NT) k_ms_potential_rows(const MsAtom* __restrict__ atoms,
                                                            const int* __restrict__ off, int natom, int s,
                                                            MsGeom g, const double* __restrict__ knots,
                                                            const double4* __restrict__ coef, double scale,
                                                            cplx<float>* __restrict__ trans,
-                                                           const cplx<float>* __restrict__ tw, int raw) {
-    constexpr int NB = lds_batch(N, sizeof(cplx<float>), LDS_POST);
-    constexpr int PER = (NB * N + 255) / 256;
-    __shared__ cplx<float> sm[2 * lds_len(NB * N)];
-    __shared__ MsAtom sa[256];
-    __shared__ int wcount[4];
+                                                           const cplx<float>* __restrict__ tw, int raw, int lim) {
+    using F = Fft<N>;
+    constexpr int NT = F::NT, NB = F::NB, M = F::M, NW = (NT + 63) / 64;
+    __shared__ cplx<float> sm[F::LDS];
+    __shared__ MsAtom sa[NT];
+    __shared__ int wcount[NW];
     const int o = blockIdx.y;
     const int a0 = off[o * g.nsl1 + s], a1 = off[o * g.nsl1 + s + 1];
     if (a0 == a1) return;  // empty slice: the wave is not transmitted
     const int y0 = blockIdx.x * NB;
     const int nb = min(NB, g.ny - y0);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int row = F::Q::row_c(tid), i = F::Q::row_i(tid), py = y0 + row;
     const MsAtom* A = atoms + (size_t)o * natom;
-    float acc[PER];
+    float acc[8];
 #pragma unroll
-    for (int q = 0; q < PER; q++) acc[q] = 0.f;
-    for (int c0 = a0; c0 < a1; c0 += 256) {
-        const int n = min(256, a1 - c0);
+    for (int r = 0; r < 8; r++) acc[r] = 0.f;
+    for (int c0 = a0; c0 < a1; c0 += NT) {
+        const int n = min(NT, a1 - c0);
         bool hit = false;
         // the record travels as two 16-byte vectors (a local MsAtom
         // aggregate was given a scratch slot by the compiler)
         float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f), r1 = r0;
-        if ((int)threadIdx.x < n) {
-            const float4* src = reinterpret_cast<const float4*>(A + c0 + threadIdx.x);
+        if (tid < n) {
+            const float4* src = reinterpret_cast<const float4*>(A + c0 + tid);
             r0 = src[0];
             r1 = src[1];
             // rows y0 .. y0+nb-1 meet some image of the atom's y window
@@ -190,9 +205,12 @@ __global__ void __launch_bounds__(256) k_ms_potential_rows(const MsAtom* __restr
         __syncthreads();
         if (lane == 0) wcount[wv] = __popcll(m);
         __syncthreads();
-        int base = 0;
-        for (int k = 0; k < wv; k++) base += wcount[k];
-        const int total = wcount[0] + wcount[1] + wcount[2] + wcount[3];
+        int base = 0, total = 0;
+#pragma unroll
+        for (int k = 0; k < NW; k++) {
+            if (k < wv) base += wcount[k];
+            total += wcount[k];
+        }
         if (hit) {
             float4* dstv = reinterpret_cast<float4*>(sa + base + pre);
             dstv[0] = r0;
@@ -201,45 +219,62 @@ __global__ void __launch_bounds__(256) k_ms_potential_rows(const MsAtom* __restr
         __syncthreads();
         for (int k = 0; k < total; k++) {
             const MsAtom t = sa[k];
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int p = (int)threadIdx.x + q * 256;
-                if (p >= nb * N) break;
-                const int r = p / N, px = p - r * N, py = y0 + r;
-                const int x0 = t.ixo - g.idx;
-                const int ix = x0 + ms_pmod(px - x0, g.nx);
-                if (ix > t.ixo + g.idx) continue;
-                const int yw = t.iyo - g.idy;
-                const int iy = yw + ms_pmod(py - yw, g.ny);
-                if (iy > t.iyo + g.idy) continue;
+            const int yw = t.iyo - g.idy, xw = t.ixo - g.idx;
+            const int iy = yw + ms_pmod(py - yw, g.ny);
+            if (iy > t.iyo + g.idy || row >= nb) continue;
+            const double ry = (double)t.y - (double)iy * g.sy;
+            for (int d = ms_pmod(i - xw, M); d <= 2 * g.idx; d += M) {
+                const int ix = xw + d;
                 const double rx = (double)t.x - (double)ix * g.sx;
-                const double ry = (double)t.y - (double)iy * g.sy;
-                double r2 = rx * rx + ry * ry;
+                double r2 = ms_r2(rx, ry);
                 if (r2 > 9.0) continue;
                 if (r2 < g.rminsq) r2 = g.rminsq;
-                acc[q] += (float)((double)t.occ * ms_lut(knots, coef + (size_t)t.zi * MS_NR, r2, g));
-            }
-        }
-    }
-    cplx<float>* a = sm;
-    cplx<float>* b = sm + lds_len(NB * N);
+                const float v = (float)((double)t.occ * ms_lut(knots, coef + (size_t)t.zi * MS_NR, r2, g));
+                const int rr = ms_pmod(ix, N) / M;
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-        const int p = (int)threadIdx.x + q * 256;
-        if (p < nb * N) {
-            if (raw) {  // the potential itself, for the Debye-Waller filter
-                a[lx(p)] = {acc[q], 0.f};
-            } else {
-                float sn, cs;
-                sincosf((float)(scale * (double)acc[q]), &sn, &cs);
-                a[lx(p)] = {cs, sn};
+                for (int r = 0; r < 8; r++)
+                    if (r == rr) acc[r] += v;
             }
         }
     }
-    __syncthreads();
-    fft_lds<float, N>(a, b, nb, tw, +1, threadIdx.x, blockDim.x);
-    cplx<float>* out = trans + ((size_t)o * g.ny + y0) * N;
-    for (int p = threadIdx.x; p < nb * N; p += blockDim.x) out[p] = a[lx(p)];
+    cplx<float> u[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+        if (raw) {  // the potential itself, for the Debye-Waller filter
+            u[r] = {acc[r], 0.f};
+        } else {
+            float sn, cs;
+            sincosf((float)(scale * (double)acc[r]), &sn, &cs);
+            // rounded before the FFT's additions (the compiler would fuse the
+            // last product of sincosf into them), as the two-kernel form stores them
+            asm volatile("" : "+v"(cs), "+v"(sn));
+            u[r] = {cs, sn};
+        }
+    }
+    F::rows(u, sm, tw, +1, tid, true);
+    if (row >= nb) return;
+    cplx<float>* out = trans + ((size_t)o * g.ny + py) * N;
+#pragma unroll
+    for (int r = 0; r < 8; r++)
+        if (raw || ms_kept(i + M * r, N, lim)) out[i + M * r] = u[r];
+}
+
+// x FFT (exponent +1) of lines of [B][ny][nx], in place.
+template <int N>
+__global__ void __launch_bounds__(Fft<N>::NT) k_ms_lines(cplx<float>* __restrict__ data, int nlines,
+                                                         const cplx<float>* __restrict__ tw) {
+    using F = Fft<N>;
+    __shared__ cplx<float> sm[F::LDS];
+    const int tid = threadIdx.x, i = F::Q::row_i(tid), l = blockIdx.x * F::NB + F::Q::row_c(tid);
+    cplx<float>* line = data + (size_t)l * N + i;
+    cplx<float> u[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++) u[r] = l < nlines ? line[F::M * r] : cplx<float>{0.f, 0.f};
+    F::rows(u, sm, tw, +1, tid, true);
+    if (l < nlines) {
+#pragma unroll
+        for (int r = 0; r < 8; r++) line[F::M * r] = u[r];
+    }
 }
 
 // 3D electrostatic potential of the atoms on a plane at height zp, per
@@ -298,150 +333,152 @@ __global__ void __launch_bounds__(256) k_ms_vatom(const MsAtom* __restrict__ ato
 // same limit times the propagator py * px (slicelib.cpp:827-835); the two
 // vectors stay in cache where a full (ky, kx) table is read once per image
 // (measured 154 against 180 us per pass over 360 images of 256^2).  MODE 2:
-// the Fresnel table F[ky][kx] times scale.
+// the Fresnel table F[ky][kx] times scale.  MODE 3: the Debye-Waller factor.
+// Bound by HBM: the product is formed between the two transforms in registers
+// (Fft), and only tiles with a column below lim are formed (ms_kept; every
+// mode leaves zeros or nothing in the others).
 template <int N, int MODE>
-__global__ void __launch_bounds__(256) k_ms_cols(const cplx<float>* __restrict__ src, cplx<float>* __restrict__ dst,
-                                                 int nx, int gx, int gy, const cplx<float>* __restrict__ tw,
+__global__ void __launch_bounds__(Fft<N>::NT) k_ms_cols(const cplx<float>* __restrict__ src, cplx<float>* __restrict__ dst,
+                                                 int nx, int gx, int gy, int lim, const cplx<float>* __restrict__ tw,
                                                  const float* __restrict__ kx2, const float* __restrict__ ky2,
                                                  float k2max, const cplx<float>* __restrict__ px,
                                                  const cplx<float>* __restrict__ py,
-                                                 const cplx<float>* __restrict__ F, float scale,
+                                                 const cplx<float>* __restrict__ F2, float scale,
                                                  const int* __restrict__ off, int nsl1, int s,
                                                  const float* __restrict__ dwm) {
-    constexpr int NB = lds_batch(N, sizeof(cplx<float>), MS_LDS);
-    __shared__ cplx<float> sm[2 * lds_len(NB * N)];
-    cplx<float>* a = sm;
-    cplx<float>* b = sm + lds_len(NB * N);
+    using F = Fft<N>;
+    __shared__ cplx<float> sm[F::LDS];
     int tx, o;
     if (!xcd_tile(gx, gy, tx, o)) return;
     if ((MODE == 0 || MODE == 3) && off[o * nsl1 + s] == off[o * nsl1 + s + 1]) return;
-    const int c0 = tx * NB;
-    const int nb = min(NB, nx - c0);
-    const size_t base = (size_t)o * N * nx + c0;
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) {
-        const int y = t / nb, c = t - y * nb;
-        a[lx(c * N + y)] = src[base + (size_t)y * nx + c];
-    }
-    __syncthreads();
-    fft_lds<float, N>(a, b, nb, tw, +1, threadIdx.x, blockDim.x);
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) {
-        const int c = t / N, y = t - c * N;
-        const int kx = c0 + c;
-        cplx<float> v = a[lx(t)];
+    const int tid = threadIdx.x, i = F::Q::col_i(tid);
+    const int kx = ms_tile(tx, nx, F::NB, lim) * F::NB + F::Q::col_c(tid);
+    const bool have = kx < nx && ms_kept(kx, nx, lim);
+    const size_t base = ((size_t)o * N + i) * nx + kx, step = (size_t)F::M * nx;
+    cplx<float> u[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++) u[r] = have ? src[base + r * step] : cplx<float>{0.f, 0.f};
+    F::cols(u, sm, tw, +1, tid, true);
+    const float kxv = have ? kx2[kx] : 0.f;
+    cplx<float> pxv = {1.f, 0.f};
+    if (MODE == 1 && have) pxv = px[kx];
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+        const int y = i + F::M * r;
+        cplx<float> v = u[r];
         if (MODE == 3) {
             // exp(-M) of trlayerDW (autoslic.cpp:1080-1088): every frequency
-            const float e = (float)exp((double)dwm[o * nsl1 + s] * (double)(ky2[y] + kx2[kx]));
+            const float e = (float)exp((double)dwm[o * nsl1 + s] * (double)(ky2[y] + kxv));
             v = {v.x * e * scale, v.y * e * scale};
         } else if (MODE == 2) {
-            v = cmul(v, F[(size_t)y * nx + kx]);
+            if (have) v = cmul(v, F2[(size_t)y * nx + kx]);
             v = {v.x * scale, v.y * scale};
-        } else if (kx2[kx] + ky2[y] < k2max) {
-            if (MODE == 1) v = cmul(cmul(v, py[y]), px[kx]);
+        } else if (have && kxv + ky2[y] < k2max) {
+            if (MODE == 1) v = cmul(cmul(v, py[y]), pxv);
             v = {v.x * scale, v.y * scale};
         } else {
             v = {0.f, 0.f};
         }
-        a[lx(t)] = v;
+        u[r] = v;
     }
-    __syncthreads();
-    fft_lds<float, N>(a, b, nb, tw, -1, threadIdx.x, blockDim.x);
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) {
-        const int y = t / nb, c = t - y * nb;
-        dst[base + (size_t)y * nx + c] = a[lx(c * N + y)];
+    F::cols(u, sm, tw, -1, tid, false);
+    if (have) {
+#pragma unroll
+        for (int r = 0; r < 8; r++) dst[base + r * step] = u[r];
     }
 }
 
-// Lines of [B][ny][nx]: NB lines per workgroup.  Multislice (PROJ false):
-// the wave W and the transmission T are both x-transformed; inverse x FFT of
+// Lines of [B][ny][nx].  Multislice (PROJ false): the wave W and the
+// transmission T are both x-transformed and zero above lim; inverse x FFT of
 // both, W * T where the slice holds atoms for this orientation, x FFT of the
-// product back into W.  Projection (PROJ true): W is real-space; inverse x
-// FFT of T only and W *= T.
+// product back into W (kept columns).  Projection (PROJ true): W is real-space;
+// inverse x FFT of T only and W *= T.
 template <int N, bool PROJ>
-__global__ void __launch_bounds__(256) k_ms_mul(cplx<float>* __restrict__ W, const cplx<float>* __restrict__ T,
-                                                int ny, int nlines, const cplx<float>* __restrict__ tw,
+__global__ void __launch_bounds__(Fft<N>::NT) k_ms_mul(cplx<float>* __restrict__ W, const cplx<float>* __restrict__ T,
+                                                int ny, int nlines, int lim, const cplx<float>* __restrict__ tw,
                                                 const int* __restrict__ off, int nsl1, int s) {
-    constexpr int NB = lds_batch(N, sizeof(cplx<float>), MS_LDS) / 2;
-    static_assert(NB >= 1, "two sequences per line must fit");
-    __shared__ cplx<float> sm[2 * lds_len(2 * NB * N)];
-    cplx<float>* a = sm;
-    cplx<float>* b = sm + lds_len(2 * NB * N);
-    const int l0 = blockIdx.x * NB;
-    const int nb = min(NB, nlines - l0);
-    const size_t base = (size_t)l0 * N;
-    // lines of one workgroup may straddle two orientations: flag per line
-    if (PROJ) {
-        for (int t = threadIdx.x; t < nb * N; t += blockDim.x) a[lx(t)] = T[base + t];
-        __syncthreads();
-        fft_lds<float, N>(a, b, nb, tw, -1, threadIdx.x, blockDim.x);
-        for (int t = threadIdx.x; t < nb * N; t += blockDim.x) {
-            const int o = (l0 + t / N) / ny;
-            if (off[o * nsl1 + s] == off[o * nsl1 + s + 1]) continue;
-            W[base + t] = cmul(W[base + t], a[lx(t)]);
-        }
-        return;
+    using F = Fft<N>;
+    constexpr int M = F::M;
+    __shared__ cplx<float> sm[F::LDS];
+    const int tid = threadIdx.x, i = F::Q::row_i(tid), l = blockIdx.x * F::NB + F::Q::row_c(tid);
+    const bool line = l < nlines;
+    const int o = line ? l / ny : 0;
+    const bool full = line && off[o * nsl1 + s] != off[o * nsl1 + s + 1];
+    const size_t base = (size_t)l * N + i;
+    cplx<float> w[8], t[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+        const bool kept = ms_kept(i + M * r, N, lim);
+        w[r] = t[r] = {0.f, 0.f};
+        if (line && (PROJ || kept)) w[r] = W[base + M * r];
+        if (full && kept) t[r] = T[base + M * r];
     }
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) {
-        a[lx(t)] = W[base + t];
-        a[lx(nb * N + t)] = T[base + t];
+    F::rows(t, sm, tw, -1, tid, true);
+    if constexpr (!PROJ) F::rows(w, sm, tw, -1, tid, false);
+    if (full) {
+#pragma unroll
+        for (int r = 0; r < 8; r++) w[r] = cmul(w[r], t[r]);
     }
-    __syncthreads();
-    fft_lds<float, N>(a, b, 2 * nb, tw, -1, threadIdx.x, blockDim.x);
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) {
-        const int o = (l0 + t / N) / ny;
-        if (off[o * nsl1 + s] != off[o * nsl1 + s + 1]) a[lx(t)] = cmul(a[lx(t)], a[lx(nb * N + t)]);
-    }
-    __syncthreads();
-    fft_lds<float, N>(a, b, nb, tw, +1, threadIdx.x, blockDim.x);
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) W[base + t] = a[lx(t)];
+    if constexpr (!PROJ) F::rows(w, sm, tw, +1, tid, false);
+    if (!line || (PROJ && !full)) return;
+#pragma unroll
+    for (int r = 0; r < 8; r++)
+        if (PROJ || ms_kept(i + M * r, N, lim)) W[base + M * r] = w[r];
 }
 
 // Debye-Waller branch, after the filter: lines of T (the filtered potential,
 // x-transformed and normalised): inverse x FFT, the transmission
-// exp(i sigma Re V) (autoslic.cpp:1091-1097), x FFT back into T.
+// exp(i sigma Re V) (autoslic.cpp:1091-1097), x FFT back into T (kept columns).
 template <int N>
-__global__ void __launch_bounds__(256) k_ms_dwexp(cplx<float>* __restrict__ T, int nlines, double scale,
+__global__ void __launch_bounds__(Fft<N>::NT) k_ms_dwexp(cplx<float>* __restrict__ T, int nlines, double scale, int lim,
                                                   const cplx<float>* __restrict__ tw) {
-    constexpr int NB = lds_batch(N, sizeof(cplx<float>), LDS_POST);
-    __shared__ cplx<float> sm[2 * lds_len(NB * N)];
-    cplx<float>* a = sm;
-    cplx<float>* b = sm + lds_len(NB * N);
-    const int l0 = blockIdx.x * NB;
-    const int nb = min(NB, nlines - l0);
-    cplx<float>* base = T + (size_t)l0 * N;
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) a[lx(t)] = base[t];
-    __syncthreads();
-    fft_lds<float, N>(a, b, nb, tw, -1, threadIdx.x, blockDim.x);
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) {
+    using F = Fft<N>;
+    constexpr int M = F::M;
+    __shared__ cplx<float> sm[F::LDS];
+    const int tid = threadIdx.x, i = F::Q::row_i(tid), l = blockIdx.x * F::NB + F::Q::row_c(tid);
+    cplx<float>* line = T + (size_t)l * N + i;
+    cplx<float> u[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++) u[r] = l < nlines ? line[M * r] : cplx<float>{0.f, 0.f};
+    F::rows(u, sm, tw, -1, tid, true);
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
         float sn, cs;
-        sincosf((float)(scale * (double)a[lx(t)].x), &sn, &cs);
-        a[lx(t)] = {cs, sn};
+        sincosf((float)(scale * (double)u[r].x), &sn, &cs);
+        u[r] = {cs, sn};
     }
-    __syncthreads();
-    fft_lds<float, N>(a, b, nb, tw, +1, threadIdx.x, blockDim.x);
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) base[t] = a[lx(t)];
+    F::rows(u, sm, tw, +1, tid, false);
+    if (l < nlines) {
+#pragma unroll
+        for (int r = 0; r < 8; r++)
+            if (ms_kept(i + M * r, N, lim)) line[M * r] = u[r];
+    }
 }
 
-// Lines of E [B][ny][nx] (x-transformed, normalised): inverse x FFT, then
-// |psi|^2 (what 0), arg psi (what 1, CArg) or psi (what 2) into
+// Lines of E [B][ny][nx] (x-transformed, normalised, zero above lim): inverse
+// x FFT, then |psi|^2 (what 0), arg psi (what 1, CArg) or psi (what 2) into
 // out[(o * ndef + d) * ny + y] (autosliccmd.cpp:1196-1239).
 template <int N>
-__global__ void __launch_bounds__(256) k_ms_out(const cplx<float>* __restrict__ E, float* __restrict__ out,
-                                                int ny, int nlines, int ndef, int d, int what,
+__global__ void __launch_bounds__(Fft<N>::NT) k_ms_out(const cplx<float>* __restrict__ E, float* __restrict__ out,
+                                                int ny, int nlines, int lim, int ndef, int d, int what,
                                                 const cplx<float>* __restrict__ tw, int accum, float div) {
-    constexpr int NB = lds_batch(N, sizeof(cplx<float>), LDS_POST);
-    __shared__ cplx<float> sm[2 * lds_len(NB * N)];
-    cplx<float>* a = sm;
-    cplx<float>* b = sm + lds_len(NB * N);
-    const int l0 = blockIdx.x * NB;
-    const int nb = min(NB, nlines - l0);
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) a[lx(t)] = E[(size_t)l0 * N + t];
-    __syncthreads();
-    fft_lds<float, N>(a, b, nb, tw, -1, threadIdx.x, blockDim.x);
-    for (int t = threadIdx.x; t < nb * N; t += blockDim.x) {
-        const int l = l0 + t / N, x = t % N;
-        const int o = l / ny, y = l - o * ny;
-        const size_t row = ((size_t)o * ndef + d) * ny + y;
-        const cplx<float> v = a[lx(t)];
+    using F = Fft<N>;
+    constexpr int M = F::M;
+    __shared__ cplx<float> sm[F::LDS];
+    const int tid = threadIdx.x, i = F::Q::row_i(tid), l = blockIdx.x * F::NB + F::Q::row_c(tid);
+    const bool line = l < nlines;
+    cplx<float> u[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++)
+        u[r] = line && ms_kept(i + M * r, N, lim) ? E[(size_t)l * N + i + M * r] : cplx<float>{0.f, 0.f};
+    F::rows(u, sm, tw, -1, tid, true);
+    if (!line) return;
+    const int o = l / ny, y = l - o * ny;
+    const size_t row = ((size_t)o * ndef + d) * ny + y;
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+        const int x = i + M * r;
+        const cplx<float> v = u[r];
         if (what == 2) {
             out[2 * (row * N + x)] = v.x;
             out[2 * (row * N + x) + 1] = v.y;
@@ -577,6 +614,7 @@ struct msct_ctx {
     std::vector<float> dwm_h;
     int nsl = 0;          // slices per orientation
     float ctbf = 0.f, k2max = 0.f, wavlen = 0.f, aobj = 0.f;
+    int lim = 0;          // first kx at or above the bandwidth limit (utr::ms_kept)
     utr::MsGeom g{};
     double scale = 0.0;   // sigma(kev) / 1000
     DevBuf<double> knots, fe_el;  // fe_el: the 12 fe parameters per element row
@@ -635,35 +673,32 @@ __global__ void k_ms_fresnel(cplx<float>* __restrict__ F, int nx, int ny, double
     F[t] = {(float)c, (float)-s};
 }
 
+// Columns the wave keeps (msct_ctx::lim; all in projection mode, whose wave is
+// never limited).
+int ms_wave_lim(const msct_ctx* c) { return c->p.mode != 0 ? c->g.nx : c->lim; }
+
 int ms_run_cols(int mode, msct_ctx* c, const cplx<float>* src, cplx<float>* dst, int B, float scale, int s,
                 const cplx<float>* F, hipStream_t st) {
     const int nx = c->g.nx, ny = c->g.ny;
+    const int lim = mode < 2 ? c->lim : mode == 2 ? ms_wave_lim(c) : nx;
     bool ok = false;
+#define MS_COLS_M(N, MODE)                                                                          \
+    utr::k_ms_cols<N, MODE><<<grid, utr::Fft<N>::NT, 0, st>>>(src, dst, nx, gx, B, lim, c->twy.p, c->kx2.p, \
+                                                              c->ky2.p, c->k2max, c->px.p, c->py.p, F, \
+                                                              scale, c->off.p, c->g.nsl1, s, c->dwm.p)
 #define MS_COLS(N)                                                                                  \
     {                                                                                               \
-        constexpr int NB = utr::lds_batch(N, sizeof(cplx<float>), utr::MS_LDS);                    \
-        const int gx = (nx + NB - 1) / NB;                                                          \
+        const int gx = utr::ms_tiles(nx, utr::Fft<N>::NB, lim);                                     \
         const unsigned grid = utr::xcd_grid((unsigned)(gx * B));                                    \
-        if (mode == 0)                                                                              \
-            utr::k_ms_cols<N, 0><<<grid, 256, 0, st>>>(src, dst, nx, gx, B, c->twy.p, c->kx2.p,     \
-                                                       c->ky2.p, c->k2max, c->px.p, c->py.p,        \
-                                                       F, scale, c->off.p, c->g.nsl1, s, c->dwm.p); \
-        else if (mode == 1)                                                                         \
-            utr::k_ms_cols<N, 1><<<grid, 256, 0, st>>>(src, dst, nx, gx, B, c->twy.p, c->kx2.p,     \
-                                                       c->ky2.p, c->k2max, c->px.p, c->py.p,        \
-                                                       F, scale, c->off.p, c->g.nsl1, s, c->dwm.p); \
-        else if (mode == 2)                                                                         \
-            utr::k_ms_cols<N, 2><<<grid, 256, 0, st>>>(src, dst, nx, gx, B, c->twy.p, c->kx2.p,     \
-                                                       c->ky2.p, c->k2max, c->px.p, c->py.p,        \
-                                                       F, scale, c->off.p, c->g.nsl1, s, c->dwm.p); \
-        else                                                                                        \
-            utr::k_ms_cols<N, 3><<<grid, 256, 0, st>>>(src, dst, nx, gx, B, c->twy.p, c->kx2.p,     \
-                                                       c->ky2.p, c->k2max, c->px.p, c->py.p,        \
-                                                       F, scale, c->off.p, c->g.nsl1, s, c->dwm.p); \
+        if (mode == 0) MS_COLS_M(N, 0);                                                             \
+        else if (mode == 1) MS_COLS_M(N, 1);                                                        \
+        else if (mode == 2) MS_COLS_M(N, 2);                                                        \
+        else MS_COLS_M(N, 3);                                                                       \
         ok = true;                                                                                  \
     }
     UTR_DISPATCH_N(ny, MS_COLS)
 #undef MS_COLS
+#undef MS_COLS_M
     if (!ok) return set_err(UTR_E_UNSUPPORTED, "msct: unsupported image height for the FFT");
     UTR_HIP_TRY(hipGetLastError());
     return UTR_OK;
@@ -674,33 +709,31 @@ int ms_run_lines(msct_ctx* c, int what, int B, int s, int ndef, int d, float* ou
     const int nx = c->g.nx, ny = c->g.ny, nlines = B * ny;
     const bool proj = c->p.mode != 0;
     bool ok = false;
+    const int wlim = ms_wave_lim(c);
 #define MS_LINES(N)                                                                                 \
     {                                                                                               \
-        constexpr int NB = utr::lds_batch(N, sizeof(cplx<float>), utr::LDS_POST);                   \
-        constexpr int NB2 = utr::lds_batch(N, sizeof(cplx<float>), utr::MS_LDS) / 2;               \
+        constexpr int NB = utr::Fft<N>::NB, NT = utr::Fft<N>::NT;                                   \
+        const unsigned groups = (unsigned)((nlines + NB - 1) / NB);                                 \
         if (what == 0) {                                                                            \
-            utr::k_post_lines<float, N><<<(nlines + NB - 1) / NB, 256, 0, st>>>(c->T.p, nlines, +1, \
-                                                                               c->twx.p);           \
+            utr::k_ms_lines<N><<<groups, NT, 0, st>>>(c->T.p, nlines, c->twx.p);                    \
         } else if (what == 1) {                                                                     \
             if (proj)                                                                               \
-                utr::k_ms_mul<N, true><<<(nlines + NB2 - 1) / NB2, 256, 0, st>>>(                   \
-                    c->W.p, c->T.p, ny, nlines, c->twx.p, c->off.p, c->g.nsl1, s);                  \
+                utr::k_ms_mul<N, true><<<groups, NT, 0, st>>>(c->W.p, c->T.p, ny, nlines, c->lim, c->twx.p, \
+                                                              c->off.p, c->g.nsl1, s);              \
             else                                                                                    \
-                utr::k_ms_mul<N, false><<<(nlines + NB2 - 1) / NB2, 256, 0, st>>>(                  \
-                    c->W.p, c->T.p, ny, nlines, c->twx.p, c->off.p, c->g.nsl1, s);                  \
+                utr::k_ms_mul<N, false><<<groups, NT, 0, st>>>(c->W.p, c->T.p, ny, nlines, c->lim, c->twx.p, \
+                                                               c->off.p, c->g.nsl1, s);             \
         } else if (what == 4) {                                                                     \
-            utr::k_ms_potential_rows<N><<<dim3((ny + NB - 1) / NB, B), 256, 0, st>>>(                  \
-                c->atoms.p, c->off.p, c->natom, s, c->g, c->knots.p, c->coef.p, c->scale, c->T.p,    \
-                c->twx.p, c->p.nwobble == 1 ? 1 : 0);                                               \
+            utr::k_ms_potential_rows<N><<<dim3((ny + NB - 1) / NB, B), NT, 0, st>>>(                \
+                c->atoms.p, c->off.p, c->natom, s, c->g, c->knots.p, c->coef.p, c->scale, c->T.p,   \
+                c->twx.p, c->p.nwobble == 1 ? 1 : 0, c->lim);                                       \
         } else if (what == 5) {                                                                     \
-            utr::k_ms_dwexp<N><<<(nlines + NB - 1) / NB, 256, 0, st>>>(c->T.p, nlines, c->scale,       \
-                                                                      c->twx.p);                    \
+            utr::k_ms_dwexp<N><<<groups, NT, 0, st>>>(c->T.p, nlines, c->scale, c->lim, c->twx.p);  \
         } else if (what == 2) {                                                                     \
-            utr::k_post_lines<float, N><<<(nlines + NB - 1) / NB, 256, 0, st>>>(c->W.p, nlines, +1, \
-                                                                               c->twx.p);           \
+            utr::k_ms_lines<N><<<groups, NT, 0, st>>>(c->W.p, nlines, c->twx.p);                    \
         } else {                                                                                    \
-            utr::k_ms_out<N><<<(nlines + NB - 1) / NB, 256, 0, st>>>(c->E.p, out, ny, nlines, ndef, \
-                                                                    d, c->p.output, c->twx.p, accum, div); \
+            utr::k_ms_out<N><<<groups, NT, 0, st>>>(c->E.p, out, ny, nlines, wlim, ndef, d, c->p.output, \
+                                                    c->twx.p, accum, div);                          \
         }                                                                                           \
         ok = true;                                                                                  \
     }
@@ -1066,6 +1099,9 @@ int msct_create(const msct_params* p, const double* fe_params, int natom, const 
         const float t = pscale * (kx2[i] * c->wavlen);
         px[i] = {(float)std::cos((double)t), (float)-std::sin((double)t)};
     }
+    c->lim = nx;
+    for (int i = nx / 2; i >= 0; i--)
+        if (!(kx2[i] < c->k2max)) c->lim = i;
     for (int i = 0; i < ny; i++) {
         const float k = ms_freq(i, ny, ax);
         ky2[i] = k * k;

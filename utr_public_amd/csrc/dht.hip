@@ -157,41 +157,43 @@ __host__ __device__ inline int dht_slots(const DhtGeom& g) {
     return g.method == 4 ? (g.nplanes + 1) / 2 : g.nplanes;
 }
 
-template <int N>
-__global__ void __launch_bounds__(256) k_dht_prop_rows(const cplx<float>* __restrict__ S,
+// A workgroup takes PROP_RG groups of NB rows of one slot, so that the N + rows
+// phases are formed once for all of them; the next group's spectrum is loaded
+// while one is transformed (Fft, in registers).  Bound by the T it writes.
+constexpr int PROP_RG = 4;
+template <int N, bool PACK, bool AP>
+__global__ void __launch_bounds__(Fft<N>::NT) k_dht_prop_rows(const cplx<float>* __restrict__ S,
                                                        cplx<float>* __restrict__ T, DhtGeom g,
                                                        const DhtRow* __restrict__ rows, int a0,
                                                        const cplx<float>* __restrict__ tw,
                                                        const cplx<float>* __restrict__ ap) {
-    constexpr int NB = lds_batch(N, sizeof(cplx<float>), LDS_DHT_ROWS);
-    constexpr int PER = (NB * N + 255) / 256;  // elements per thread
-    __shared__ cplx<float> sm[2 * lds_len(NB * N)];
-    __shared__ cplx<float> s_ex[2][N], s_ey[2][NB];
-    cplx<float>* a = sm;
-    cplx<float>* b = sm + lds_len(NB * N);
+    using F = Fft<N>;
+    constexpr int NB = F::NB, M = F::M, NT = F::NT, NR = PROP_RG * NB;
+    __shared__ cplx<float> sm[F::LDS];
+    __shared__ cplx<float> s_ex[PACK ? 2 : 1][N], s_ey[PACK ? 2 : 1][NR];
     const int ny = g.ny;
-    const int slot = blockIdx.y, ab = blockIdx.z;
-    const bool pack = g.method == 4;
-    const int p0 = pack ? 2 * slot : slot;
-    const int np = pack && p0 + 1 < g.nplanes ? 2 : 1;  // planes in this slot
-    const int k0 = blockIdx.x * NB;
-    const int nb = min(NB, ny - k0);
-    const int tid = threadIdx.x;
-    const DhtRow& R = rows[a0 + ab];
+    const int slot = blockIdx.y;
+    const int p0 = PACK ? 2 * slot : slot;
+    const int np = PACK && p0 + 1 < g.nplanes ? 2 : 1;  // planes in this slot
+    const int k0 = blockIdx.x * NR;
+    const int nr = min(NR, ny - k0);
+    const int tid = threadIdx.x, i = F::Q::row_i(tid), rc = F::Q::row_c(tid);
+    const DhtRow& R = rows[a0];
     const double pi = 3.14159265358979323846, twopi = 2.0 * pi;
-    const cplx<float>* src = S + ((size_t)(a0 + ab) * ny + k0) * N;
-    const cplx<float>* aps = ap + (size_t)k0 * N;
-    cplx<float> v[PER], h[PER];
+    const cplx<float>* src = S + ((size_t)a0 * ny + k0) * N + i;
+    const cplx<float>* aps = ap + (size_t)k0 * N + i;
+    cplx<float> vn[8], hn[8];
+    auto fetch = [&](int row) {
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-        const int t = tid + 256 * q;
-        if (t < nb * N) {
-            v[q] = src[t];
-            h[q] = g.use_ap ? aps[t] : cplx<float>{1.f, 0.f};
+        for (int r = 0; r < 8; r++) {
+            vn[r] = row < nr ? src[(size_t)row * N + M * r] : cplx<float>{0.f, 0.f};
+            hn[r] = {1.f, 0.f};
+            if (AP && row < nr) hn[r] = aps[(size_t)row * N + M * r];
         }
-    }
-    for (int k = tid; k < np * (N + nb); k += 256) {
-        const int m = k >= N + nb ? 1 : 0, kk = k - m * (N + nb);
+    };
+    fetch(rc);
+    for (int k = tid; k < np * (N + nr); k += NT) {
+        const int m = k >= N + nr ? 1 : 0, kk = k - m * (N + nr);
         const int n = g.escc ? p0 + m : g.nz / 2;
         const double zn = g.zlodz + g.xst * n;  // voutdefocus[n], DHT.cpp:388
         const double d = g.method != 4 ? zn - R.zout : R.zout - zn;  // 1-3: back-propagation
@@ -208,37 +210,52 @@ __global__ void __launch_bounds__(256) k_dht_prop_rows(const cplx<float>* __rest
         else s_ey[m][kk - N] = e;
     }
     __syncthreads();
+    cplx<float> ex[PACK ? 2 : 1][8];
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-        const int t = tid + 256 * q;
-        if (t < nb * N) {
-            const int r = t / N, kx = t - r * N;
-            const bool in = h[q].x != 0.f || h[q].y != 0.f;  // |ap| = 1 inside the aperture, 0 outside
-            if (!pack) {
+    for (int m = 0; m < (PACK ? 2 : 1); m++)
+#pragma unroll
+        for (int r = 0; r < 8; r++) ex[m][r] = m < np ? s_ex[m][i + M * r] : cplx<float>{0.f, 0.f};
+    cplx<float>* dst = T + ((size_t)slot * ny + k0) * N + i;
+    for (int r0 = 0; r0 < nr; r0 += NB) {
+        const int row = r0 + rc;
+        cplx<float> u[8], h[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            u[r] = vn[r];
+            h[r] = hn[r];
+        }
+        if (r0 + NB < nr) fetch(row + NB);
+        const cplx<float> ey[2] = {s_ey[0][row], PACK ? s_ey[1][row] : cplx<float>{0.f, 0.f}};
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const cplx<float> v = u[r];
+            [[maybe_unused]] const bool in = h[r].x != 0.f || h[r].y != 0.f;  // |ap| = 1 inside the aperture, 0 outside
+            if constexpr (!PACK) {
                 // cos chi - i sin chi (the aperture table only when present)
-                cplx<float> H = cmul(s_ex[0][kx], s_ey[0][r]);
-                if (g.use_ap) H = cmul(H, h[q]);
-                const float fr = H.x, fi = H.y;
-                a[lx(t)] = {v[q].x * fr - v[q].y * fi, v[q].x * fi + v[q].y * fr};
+                cplx<float> H = cmul(ex[0][r], ey[0]);
+                if (AP) H = cmul(H, h[r]);
+                u[r] = cmul(v, H);
             } else {
                 float f[2] = {0.f, 0.f};
 #pragma unroll
                 for (int m = 0; m < 2; m++) {
                     if (m < np && in) {
-                        const cplx<float> H = cmul(cmul(s_ex[m][kx], s_ey[m][r]), h[q]);
+                        cplx<float> H = cmul(ex[m][r], ey[m]);
+                        if (AP) H = cmul(H, h[r]);
                         const float tt = -H.y - (float)g.asigma * H.x;  // sin chi - asigma cos chi
                         f[m] = tt / (2.f * (tt * tt + (float)g.epsilon));
                     }
                 }
                 // plane p0 times f[0] plus i times plane p0+1 times f[1]
-                a[lx(t)] = {v[q].x * f[0] - v[q].y * f[1], v[q].y * f[0] + v[q].x * f[1]};
+                u[r] = {v.x * f[0] - v.y * f[1], v.y * f[0] + v.x * f[1]};
             }
         }
+        F::rows(u, sm, tw, +1, tid, r0 == 0);
+        if (row < nr) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) dst[(size_t)row * N + M * r] = u[r];
+        }
     }
-    __syncthreads();
-    fft_lds<float, N>(a, b, nb, tw, +1, tid, blockDim.x);
-    cplx<float>* dst = T + (((size_t)ab * dht_slots(g) + slot) * ny + k0) * N;
-    for (int t = tid; t < nb * N; t += blockDim.x) dst[t] = a[lx(t)];
 }
 
 // Inverse FFT along y of each slot, then 1 - |psi|^2 = -2 Re u - |u|^2
@@ -255,103 +272,70 @@ __global__ void __launch_bounds__(256) k_dht_prop_rows(const cplx<float>* __rest
 // COL: the planes are stored column-major ([plane][x][y], y fastest) for
 // the column splat; otherwise row-major ([plane][y][x]).
 template <int N, bool COL>
-__global__ void __launch_bounds__(256) k_dht_prop_cols(const cplx<float>* __restrict__ T,
+__global__ void __launch_bounds__(Fft<N>::NT) k_dht_prop_cols(const cplx<float>* __restrict__ T,
                                                        float* __restrict__ P, DhtGeom g,
                                                        const DhtRow* __restrict__ rows, int a0,
                                                        const cplx<float>* __restrict__ tw,
                                                        unsigned* __restrict__ pmax, int gx, int total) {
-    constexpr int NB = lds_batch(N, sizeof(cplx<float>), LDS_DHT);
-    constexpr int PER = (NB * N + 255) / 256;  // elements per thread
-    __shared__ cplx<float> sm[2 * lds_len(NB * N)];
-    __shared__ float s_wmax[4];
+    using F = Fft<N>;
+    constexpr int NB = F::NB, M = F::M, NT = F::NT, NW = (NT + 63) / 64;
+    __shared__ cplx<float> sm[F::LDS];
+    __shared__ float s_wmax[NW];
     const int nx = g.nx;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, ci = F::Q::col_c(tid), ii = F::Q::col_i(tid);
+    // columns in; column-major planes leave with neighbouring lanes along y
+    const int co = COL ? F::Q::row_c(tid) : ci, io = COL ? F::Q::row_i(tid) : ii;
     const unsigned L = blockIdx.x, G = gridDim.x;
     auto tile_of = [&](int k) { return (int)(k * G + (L & 7u) * (G >> 3) + (L >> 3)); };
-    // element t of a tile is (row t / cols, column t % cols); a full tile
-    // (the common case) divides by the constant NB
-    cplx<float> vn[PER];
-    auto fetch_cols = [&](const cplx<float>* base, const int cols) {
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int t = tid + 256 * q;
-            if (t < cols * N) {
-                const int y = t / cols, c = t - y * cols;
-                vn[q] = base[(size_t)y * nx + c];
-            }
-        }
-    };
+    cplx<float> vn[8];
     auto fetch = [&](int w) {
-        const int pa = w / gx, x0 = (w - pa * gx) * NB, nb = min(NB, nx - x0);
-        const cplx<float>* base = T + (size_t)pa * N * nx + x0;
-        if (nb == NB) fetch_cols(base, NB);
-        else fetch_cols(base, nb);
+        const int pa = w / gx, x = (w - pa * gx) * NB + ci;
+        const cplx<float>* base = T + ((size_t)pa * N + ii) * nx + x;
+#pragma unroll
+        for (int r = 0; r < 8; r++) vn[r] = x < nx ? base[(size_t)(M * r) * nx] : cplx<float>{0.f, 0.f};
     };
     float vmax = 0.f;
     const int rounds = (total + (int)G - 1) / (int)G;
+    const float inv = (float)(1.0 / ((double)nx * N)), w = rows[a0].weight;
+    // method 4: the slot's real part is plane 2 slot, its imaginary part plane 2 slot + 1
+    const bool pack = g.method == 4;
     if (tile_of(0) < total) fetch(tile_of(0));
     for (int rk = 0; rk < rounds; rk++) {
         const int wt = tile_of(rk);
-        cplx<float> vc[PER];
+        cplx<float> u[8];
 #pragma unroll
-        for (int q = 0; q < PER; q++) vc[q] = vn[q];
+        for (int r = 0; r < 8; r++) u[r] = vn[r];
         if (rk + 1 < rounds && tile_of(rk + 1) < total) fetch(tile_of(rk + 1));
         if (wt >= total) continue;  // uniform over the workgroup
-        cplx<float>* a = sm;
-        cplx<float>* b = sm + lds_len(NB * N);
-        const int pa = wt / gx, x0 = (wt - pa * gx) * NB, nb = min(NB, nx - x0);
-        const int nslots = dht_slots(g), ab = pa / nslots, slot = pa - ab * nslots;
-        // method 4: the slot's real part is plane 2 slot, its imaginary part plane 2 slot + 1
-        const bool pack = g.method == 4;
-        const int pl0 = ab * g.nplanes + (pack ? 2 * slot : slot);
-        const bool second = pack && (pack ? 2 * slot : slot) + 1 < g.nplanes;
-        const size_t plane = (size_t)pl0 * N * nx;
-        auto put = [&](const int cols) {
+        const int slot = wt / gx, x = (wt - slot * gx) * NB + co;
+        const int pl0 = pack ? 2 * slot : slot;
+        const bool second = pack && pl0 + 1 < g.nplanes;
+        if constexpr (COL) F::cols_to_rows(u, sm, tw, +1, tid, rk == 0);
+        else F::cols(u, sm, tw, +1, tid, rk == 0);
+        if (x < nx) {
+            float* dst = P + (size_t)pl0 * N * nx + (COL ? (size_t)x * N + io : (size_t)io * nx + x);
+            const size_t step = COL ? M : (size_t)M * nx;
 #pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int t = tid + 256 * q;
-                if (t < cols * N) {
-                    const int y = t / cols, c = t - y * cols;
-                    a[lx(c * N + y)] = vc[q];
+            for (int r = 0; r < 8; r++) {
+                const float re = u[r].x * inv, im = u[r].y * inv;
+                const float v = (pack ? re : -2.f * re - (re * re + im * im)) * w;
+                dst[r * step] = v;
+                vmax = fmaxf(vmax, fabsf(v));
+                if (second) {
+                    const float v2 = im * w;
+                    dst[(size_t)N * nx + r * step] = v2;
+                    vmax = fmaxf(vmax, fabsf(v2));
                 }
             }
-        };
-        if (nb == NB) put(NB);
-        else put(nb);
-        __syncthreads();
-        fft_lds<float, N>(a, b, nb, tw, +1, tid, blockDim.x);
-        const float inv = (float)(1.0 / ((double)nx * N));
-        const float w = rows[a0 + ab].weight;
-        auto store = [&](const int cols) {
-#pragma unroll
-            for (int q = 0; q < PER; q++) {
-                const int t = tid + 256 * q;
-                if (t < cols * N) {
-                    // column-major: consecutive threads take consecutive y
-                    const int y = COL ? t % N : t / cols, c = COL ? t / N : t - y * cols;
-                    const cplx<float> z = a[lx(c * N + y)];
-                    const float re = z.x * inv, im = z.y * inv;
-                    const float v = (pack ? re : -2.f * re - (re * re + im * im)) * w;
-                    const size_t o = COL ? (size_t)(x0 + c) * N + y : (size_t)y * nx + x0 + c;
-                    P[plane + o] = v;
-                    vmax = fmaxf(vmax, fabsf(v));
-                    if (second) {
-                        const float v2 = im * w;
-                        P[plane + (size_t)N * nx + o] = v2;
-                        vmax = fmaxf(vmax, fabsf(v2));
-                    }
-                }
-            }
-        };
-        if (nb == NB) store(NB);
-        else store(nb);
-        __syncthreads();  // the next tile overwrites both buffers
+        }
     }
     for (int off = 32; off > 0; off >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, off));
     if ((tid & 63) == 0) s_wmax[tid >> 6] = vmax;
     __syncthreads();
-    if (tid == 0)
-        atomicMax(pmax, __float_as_uint(fmaxf(fmaxf(s_wmax[0], s_wmax[1]), fmaxf(s_wmax[2], s_wmax[3]))));
+    if (tid == 0) {
+        for (int k = 1; k < NW; k++) vmax = fmaxf(vmax, s_wmax[k]);
+        atomicMax(pmax, __float_as_uint(vmax));
+    }
 }
 
 __device__ __forceinline__ int dht_lds(int lx, int ly, int lz) {
@@ -1018,31 +1002,37 @@ int dht_run(dht_ctx* c, float* d_vol) {
         bool ok = false;
         for (int ab = 0; ab < na; ab++) {
             ok = false;
+#define DHT_PR1(N, PACK, AP)                                                                     \
+    utr::k_dht_prop_rows<N, PACK, AP><<<grid, utr::Fft<N>::NT, 0, c->stream>>>(                  \
+        c->spec.p, c->T.p, g, c->rows.p, a0 + ab, c->twx.p, c->ap.p)
 #define DHT_PR(N)                                                                                \
     {                                                                                            \
-        constexpr int NB = utr::lds_batch(N, sizeof(cplx<float>), utr::LDS_DHT_ROWS);                 \
-        utr::k_dht_prop_rows<N><<<dim3((g.ny + NB - 1) / NB, utr::dht_slots(g), 1), 256, 0,       \
-                                  c->stream>>>(                                                  \
-            c->spec.p, c->T.p, g, c->rows.p, a0 + ab, c->twx.p, c->ap.p);                        \
+        constexpr int NR = utr::PROP_RG * utr::Fft<N>::NB;                                       \
+        const dim3 grid((g.ny + NR - 1) / NR, utr::dht_slots(g), 1);                             \
+        if (g.method == 4 && g.use_ap) DHT_PR1(N, true, true);                                   \
+        else if (g.method == 4) DHT_PR1(N, true, false);                                         \
+        else if (g.use_ap) DHT_PR1(N, false, true);                                              \
+        else DHT_PR1(N, false, false);                                                           \
         ok = true;                                                                               \
     }
             UTR_DISPATCH_N(g.nx, DHT_PR)
 #undef DHT_PR
+#undef DHT_PR1
             if (!ok) return set_err(UTR_E_UNSUPPORTED, "unsupported image width for the FFT");
             ok = false;
 #define DHT_PC(N)                                                                                \
     {                                                                                            \
-        constexpr int NB = utr::lds_batch(N, sizeof(cplx<float>), utr::LDS_DHT);                 \
-        constexpr int lds = 2 * utr::lds_len(NB * N) * (int)sizeof(cplx<float>);                \
-        const int gx = (g.nx + NB - 1) / NB, total = gx * utr::dht_slots(g);                     \
-        const unsigned cap = (unsigned)(c->ncu * std::max(1, std::min(8, 163840 / lds))) & ~7u;  \
+        using F = utr::Fft<N>;                                                                   \
+        constexpr int lds = F::LDS * (int)sizeof(cplx<float>);                                   \
+        const int gx = (g.nx + F::NB - 1) / F::NB, total = gx * utr::dht_slots(g);               \
+        const unsigned cap = (unsigned)(c->ncu * std::max(1, std::min(2048 / F::NT, 163840 / lds))) & ~7u; \
         const unsigned grid = std::min(utr::xcd_grid((unsigned)total), cap ? cap : 8u);          \
         if (colsplat)                                                                            \
-            utr::k_dht_prop_cols<N, true><<<grid, 256, 0, c->stream>>>(                          \
+            utr::k_dht_prop_cols<N, true><<<grid, F::NT, 0, c->stream>>>(                          \
                 c->T.p, c->P.p + (size_t)ab * g.nplanes * g.nx * g.ny, g, c->rows.p, a0 + ab,    \
                 c->twy.p, c->pmax.p, gx, total);                                                 \
         else                                                                                     \
-            utr::k_dht_prop_cols<N, false><<<grid, 256, 0, c->stream>>>(                         \
+            utr::k_dht_prop_cols<N, false><<<grid, F::NT, 0, c->stream>>>(                         \
                 c->T.p, c->P.p + (size_t)ab * g.nplanes * g.nx * g.ny, g, c->rows.p, a0 + ab,    \
                 c->twy.p, c->pmax.p, gx, total);                                                 \
         ok = true;                                                                               \

@@ -51,3 +51,27 @@ def test_propagation_shapes(nx, ny, nz, nrows, method, ap):
     w = np.linspace(0.5, 1.5, nrows).astype(np.float32)  # a wrong orientation's weight shows
     got = U.dht_reconstruct(p, dict(rows, weights=w), imgs)
     assert rel(got, oracle.dht_reconstruct(p, rows, imgs, weights=w)) < TOL
+
+
+@pytest.mark.parametrize("method", [1, 2])
+@pytest.mark.parametrize("nx,ny", [(16, 128), (256, 32), (512, 64), (64, 512)])
+def test_series_shapes(nx, ny, method):
+    """Methods 1 and 2 on the register transforms, series of two and three
+    images; tolerances of test_gpu_dht_series.py."""
+    counts = [3, 2, 3]
+    rng = np.random.default_rng(nx + ny)
+    p, rows, _ = case(nx, ny, 6, 3, nx + 2 * ny, method=method, escc=1, dzextra=100.0,
+                      epsilon=0.0 if method == 1 else 1e-8, itermax=6)
+    rows.update(counts=counts, defocus=np.concatenate([[150.0, 230.0, 330.0][:c] for c in counts]))
+    imgs = images(rng, sum(counts), nx, ny)
+    print("series", nx, ny, method, flush=True)
+    with U.DhtReconstructor(p, rows) as r:
+        r.add_images(imgs)
+        vol, waves, its = r.finalize(), r.waves(), r.iterations()
+    assert rel(vol, oracle.dht_reconstruct(p, rows, imgs)) < 2e-5
+    f = 0
+    for a, c in enumerate(counts):
+        psi, _, it = oracle.dht_retrieve(p, imgs[f:f + c], rows["defocus"][f:f + c])
+        assert np.linalg.norm(waves[a] - psi) / np.linalg.norm(psi - 1) < 1e-4
+        assert its[a] == (it if method == 1 else 0)
+        f += c

@@ -40,7 +40,7 @@ def case(nx, ny, nz, nrows, seed, general=True, **kw):
 
 @pytest.mark.parametrize("nx,ny,nz,nrows,method,ap", [
     (16, 512, 5, 3, 3, 0.0), (512, 16, 5, 3, 4, 0.0), (32, 128, 9, 4, 3, 25.0), (128, 32, 8, 4, 4, 25.0),
-    (64, 16, 1, 2, 4, 0.0),
+    (64, 16, 3, 2, 4, 0.0),
     (256, 256, 33, 7, 3, 0.0),  # 17 MB an orientation: launches of five and two
     (256, 64, 35, 5, 4, 0.0),
 ])
@@ -75,3 +75,20 @@ def test_series_shapes(nx, ny, method):
         assert np.linalg.norm(waves[a] - psi) / np.linalg.norm(psi - 1) < 1e-4
         assert its[a] == (it if method == 1 else 0)
         f += c
+
+
+@pytest.mark.parametrize("nx,ny,nz,method,escc", [
+    (32, 16, 9, 3, 1), (16, 64, 30, 3, 0), (64, 128, 33, 4, 1), (32, 256, 7, 3, 1), (16, 512, 5, 3, 1),
+])
+def test_column_splat_shapes(nx, ny, nz, method, escc, monkeypatch):
+    """Columns through y: lines shared by four, two and one group of waves, a
+    height beyond the columns; the bricks form the same sums bit for bit."""
+    kw = dict(dzextra=60.0, epsilon=1.0) if method == 3 else dict(dzextra=0.0, asigma=0.06, epsilon=0.02)
+    p, rows, imgs = case(nx, ny, nz, 5, 70 + nx + ny, general=False, method=method, escc=escc, **kw)
+    rows["angY"] = np.array([0.0, 90.0, 33.0, 135.0, 180.0])
+    print("columns", nx, ny, nz, method, escc, flush=True)
+    got = U.dht_reconstruct(p, rows, imgs)
+    monkeypatch.setenv("UTR_GRID_FORM", "brick")
+    brick = U.dht_reconstruct(p, rows, imgs)
+    assert np.array_equal(got.view(np.uint32), brick.view(np.uint32))
+    assert rel(got, oracle.dht_reconstruct(p, rows, imgs)) < TOL

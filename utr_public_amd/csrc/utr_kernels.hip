@@ -768,9 +768,11 @@ struct PassKind {
 
 // round(d) as a 64-bit integer for |d| < 2^51 (1.5 * 2^52 aligns the units
 // digit with the last mantissa bit; round to nearest even)
+constexpr double DROUND = 6755399441055744.0;  // 1.5 2^52, and its bits
+constexpr long long DROUND_BITS = 0x4338000000000000LL;
 __device__ __forceinline__ long long dround_i64(double d) {
-    const double y = d + 6755399441055744.0;
-    return (long long)(__double_as_longlong(y) - 0x4338000000000000LL);
+    const double y = d + DROUND;
+    return (long long)(__double_as_longlong(y) - DROUND_BITS);
 }
 
 // round(w * k) as a 64-bit integer for |w * k| < 2^51: one fma rounds the

@@ -1,0 +1,42 @@
+"""The 2D and 3D transforms of a reconstruction at every supported length as
+image width, height and volume depth, with the 2D filters of modes 1 and 3, in
+the FP32 and FP64 forms, against the FP64 oracle: 1e-5 for FP32 transforms and
+sums, 1e-10 for FP64 ones (both as test_gpu_parity.py has them)."""
+import numpy as np
+import pytest
+
+import oracle
+import utr_public_amd as U
+from utr_public_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    a = np.asarray(a, np.float64)
+    b = np.asarray(b, np.float64)
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+@pytest.mark.parametrize("nx,ny,nz,mode,kw", [
+    (16, 512, 48, 0, {}), (32, 48, 16, 3, {}), (48, 160, 64, 1, dict(modality=1, asigma=-0.004)), (64, 32, 96, 3, dict(escc=0)),
+    (96, 128, 32, 0, {}), (128, 64, 160, 1, dict(modality=1, asigma=-0.004)), (160, 16, 192, 3, {}), (192, 96, 128, 0, {}),
+    (256, 320, 16, 3, {}), (320, 192, 32, 0, {}), (384, 16, 256, 1, dict(modality=1, asigma=-0.004)), (512, 384, 16, 0, {}),
+    (64, 256, 48, 3, {}), (32, 16, 384, 0, {}), (16, 32, 320, 0, {}), (48, 32, 512, 0, {}),
+])
+@pytest.mark.parametrize("form", ["fp32", "fp64"])
+def test_transform_lengths(nx, ny, nz, mode, kw, form):
+    print("lengths", nx, ny, nz, mode, form, flush=True)
+    xst, rows = 0.4, 5
+    p = U.default_params(nx=nx, ny=ny, xst=xst, zlo=-nz * xst / 2, zhi=nz * xst / 2,
+                         **dict(dict(escc=1, nsr=0.05, ctf_mode=mode), **kw))
+    rng = np.random.default_rng(nx + 2 * ny + 3 * nz)
+    angZ, angY = rng.uniform(0, 360, rows), rng.uniform(0, 180, rows)
+    r = dict(angZ=angZ, angY=angY, defocus=rng.uniform(200, 400, rows))
+    xyz, Z = synth.atoms(3, 20, "cube", min(nx, ny, nz) * xst * 0.4, 1.0, ([6], [1.0]))
+    imgs = synth.project(xyz, Z, nx, ny, xst, angZ, angY, dose=400.0, seed=3)
+    ref = oracle.reconstruct(p, r, imgs)
+    if form == "fp32":
+        assert rel(U.reconstruct(p, r, imgs), ref) < 1e-5
+    else:
+        assert rel(U.reconstruct(p, r, imgs, U.UTR_FP64, f64_out=True), ref) < 1e-10

@@ -127,7 +127,6 @@ struct LocalBuf : DevBuf<T> {
 };
 
 constexpr int kStageRows = 32;  // rows per host->device staging batch
-constexpr int kRowsWgPerCu = 8; // resident workgroups of the persistent row FFT
 
 // ------------------------------------------------ host memory, host copies
 //
@@ -335,10 +334,10 @@ int launch_2d(utr_ctx* c, const float* d_img, int row0, int count, cplx<T>* d_sp
     bool ok = false;
 #define UTR_ROWS(N)                                                                             \
     {                                                                                           \
-        constexpr int NB = utr::lds_batch(N, sizeof(cplx<T>), utr::LDS_ROWS);                      \
-        const int nbr = (g.ny + NB - 1) / NB, nbt = nbr * count;                                \
-        const int grid = std::min(nbt, c->ncu * (c->rows_wpc > 0 ? c->rows_wpc : kRowsWgPerCu)); \
-        utr::k_rows<T, N><<<grid, 256, 0, c->stream>>>(d_img, d_spec, g.ny, g, twx, nbr, nbt);  \
+        using F = utr::Fft<N, T>;                                                               \
+        const int nbr = ((g.ny + 1) / 2 + F::NB - 1) / F::NB, nbt = nbr * count;                \
+        const int grid = std::min(nbt, c->ncu * (c->rows_wpc > 0 ? c->rows_wpc : F::WPC));      \
+        utr::k_rows<T, N><<<grid, F::NT, 0, c->stream>>>(d_img, d_spec, g.ny, g, twx, nbr, nbt); \
         ok = true;                                                                              \
     }
     UTR_DISPATCH_N(g.nx, UTR_ROWS)
@@ -347,15 +346,18 @@ int launch_2d(utr_ctx* c, const float* d_img, int row0, int count, cplx<T>* d_sp
     ok = false;
 #define UTR_COLS(N)                                                                             \
     {                                                                                           \
-        constexpr int NB = utr::lds_batch(N, sizeof(cplx<T>), utr::LDS_COLS);                      \
+        using F = utr::Fft<N, T>;                                                               \
         const int ncol = g.nx / 2 + 1; /* the rest by Hermitian symmetry */                     \
-        const int gx = (ncol + NB - 1) / NB;                                                    \
-        const int lds = 2 * utr::lds_len(NB * N) * (int)sizeof(cplx<T>);                          \
-        int wpc = std::max(1, std::min(8, 163840 / lds)); /* resident per CU */                 \
+        const int gx = (ncol + F::NB - 1) / F::NB;                                              \
+        int wpc = std::max(1, F::WPC); /* resident per CU */                                    \
         if (c->cols_wpc > 0) wpc = std::min(wpc, c->cols_wpc);                                  \
         const unsigned grid = std::min(utr::xcd_grid(gx * count), persistent_cap(c, wpc));      \
-        utr::k_cols<T, N><<<grid, 256, 0, c->stream>>>(d_spec, g.nx, ncol, g, c->rows.p, row0,  \
-                                                       twy, c->rowmax.p, gx, count);            \
+        if (g.ctf_mode == 1 || g.ctf_mode == 3)                                                 \
+            utr::k_cols<T, N, true><<<grid, F::NT, 0, c->stream>>>(d_spec, g.nx, ncol, g, c->rows.p, row0, \
+                                                                   twy, c->rowmax.p, gx, count); \
+        else                                                                                    \
+            utr::k_cols<T, N, false><<<grid, F::NT, 0, c->stream>>>(d_spec, g.nx, ncol, g, c->rows.p, row0, \
+                                                                    twy, c->rowmax.p, gx, count); \
         ok = true;                                                                              \
     }
     UTR_DISPATCH_N(g.ny, UTR_COLS)
@@ -374,9 +376,9 @@ int launch_3d(utr_ctx* c, const cplx<T>* d_V, cplx<T>* d_H, TO* d_vol, const cpl
     bool ok = false;
 #define UTR_PZ(N)                                                                               \
     {                                                                                           \
-        constexpr int CW = utr::lds_batch(N, sizeof(cplx<T>), utr::LDS_PACKZ);                     \
-        const int gx = (W + CW - 1) / CW;                                                       \
-        utr::k_pack_z<T, N><<<utr::xcd_grid(gx * g.ny), 256, 0, c->stream>>>(d_V, d_H, g, twz,  \
+        using F = utr::Fft<N, T>;                                                               \
+        const int gx = (W + F::NB - 1) / F::NB;                                                 \
+        utr::k_pack_z<T, N><<<utr::xcd_grid(gx * g.ny), F::NT, 0, c->stream>>>(d_V, d_H, g, twz, \
                                                                              gx, g.ny);         \
         ok = true;                                                                              \
     }
@@ -386,9 +388,9 @@ int launch_3d(utr_ctx* c, const cplx<T>* d_V, cplx<T>* d_H, TO* d_vol, const cpl
     ok = false;
 #define UTR_FY(N)                                                                               \
     {                                                                                           \
-        constexpr int CW = utr::lds_batch(N, sizeof(cplx<T>), utr::LDS_FFTY);                      \
-        const int gx = (W + CW - 1) / CW;                                                       \
-        utr::k_fft_y<T, N><<<utr::xcd_grid(gx * g.nz), 256, 0, c->stream>>>(d_H, g, twy, gx,    \
+        using F = utr::Fft<N, T>;                                                               \
+        const int gx = (W + F::NB - 1) / F::NB;                                                 \
+        utr::k_fft_y<T, N><<<utr::xcd_grid(gx * g.nz), F::NT, 0, c->stream>>>(d_H, g, twy, gx,  \
                                                                             g.nz);              \
         ok = true;                                                                              \
     }
@@ -398,9 +400,9 @@ int launch_3d(utr_ctx* c, const cplx<T>* d_V, cplx<T>* d_H, TO* d_vol, const cpl
     ok = false;
 #define UTR_CX(N)                                                                               \
     {                                                                                           \
-        constexpr int NB = utr::lds_batch(N, sizeof(cplx<T>), utr::LDS_C2R);                       \
-        const int gx = (g.ny / 2 + NB - 1) / NB;                                                \
-        utr::k_c2r_x<T, N, TO><<<utr::xcd_grid(gx * g.nz), 256, 0, c->stream>>>(d_H, d_vol, g,  \
+        using F = utr::Fft<N, T>;                                                               \
+        const int gx = (g.ny / 2 + F::NB - 1) / F::NB;                                          \
+        utr::k_c2r_x<T, N, TO><<<utr::xcd_grid(gx * g.nz), F::NT, 0, c->stream>>>(d_H, d_vol, g, \
                                                                                twx, gx, g.nz);  \
         ok = true;                                                                              \
     }

@@ -341,26 +341,29 @@ __device__ __forceinline__ void fft_reg(cplx<T>* u, cplx<T>* __restrict__ sm, co
 
 // The transform of columns (neighbouring lanes on neighbouring sequences) or of
 // rows (on neighbouring elements), in place.
-template <int N>
+template <int N, typename T = float>
 struct Fft {
     static constexpr int NT = fft_threads(N);
     using Q = FftReg<N, NT>;
     static constexpr int NB = Q::NB, M = Q::M, LDS = Q::LDS;
-    __device__ static __forceinline__ void cols(cplx<float>* u, cplx<float>* sm, const cplx<float>* tw, int sign, int tid,
+    // workgroups a CU holds at most, by threads and by LDS
+    static constexpr int WPC = 2048 / NT < 163840 / (LDS * (int)sizeof(cplx<T>)) ? 2048 / NT
+                                                                               : 163840 / (LDS * (int)sizeof(cplx<T>));
+    __device__ static __forceinline__ void cols(cplx<T>* u, cplx<T>* sm, const cplx<T>* tw, int sign, int tid,
                                                 bool fresh) {
         const int c = Q::col_c(tid), i = Q::col_i(tid);
-        fft_reg<float, N, NT>(u, sm, tw, sign, tid, c, i, c, i, true, fresh);
+        fft_reg<T, N, NT>(u, sm, tw, sign, tid, c, i, c, i, true, fresh);
     }
-    __device__ static __forceinline__ void rows(cplx<float>* u, cplx<float>* sm, const cplx<float>* tw, int sign, int tid,
+    __device__ static __forceinline__ void rows(cplx<T>* u, cplx<T>* sm, const cplx<T>* tw, int sign, int tid,
                                                 bool fresh) {
         const int c = Q::row_c(tid), i = Q::row_i(tid);
-        fft_reg<float, N, NT>(u, sm, tw, sign, tid, c, i, c, i, false, fresh);
+        fft_reg<T, N, NT>(u, sm, tw, sign, tid, c, i, c, i, false, fresh);
     }
     // columns in, rows out
-    __device__ static __forceinline__ void cols_to_rows(cplx<float>* u, cplx<float>* sm, const cplx<float>* tw, int sign,
+    __device__ static __forceinline__ void cols_to_rows(cplx<T>* u, cplx<T>* sm, const cplx<T>* tw, int sign,
                                                         int tid, bool fresh) {
-        fft_reg<float, N, NT>(u, sm, tw, sign, tid, Q::col_c(tid), Q::col_i(tid), Q::row_c(tid), Q::row_i(tid), true,
-                              fresh);
+        fft_reg<T, N, NT>(u, sm, tw, sign, tid, Q::col_c(tid), Q::col_i(tid), Q::row_c(tid), Q::row_i(tid), true,
+                          fresh);
     }
 };
 

@@ -35,12 +35,8 @@ __device__ __forceinline__ float dev_log<float>(float x) { return logf(x); }
 template <>
 __device__ __forceinline__ double dev_log<double>(float x) { return log((double)x); }
 
-// LDS bytes per FFT buffer, per kernel (measured on gfx950 at 256^3: small
-// batches, and so more resident workgroups, win for the row and 3D passes;
-// the persistent column pass prefers 64-byte column segments, as does the
-// Hermitian pack, which reads mirrored column pairs)
-constexpr int LDS_ROWS = 8192, LDS_COLS = 16384, LDS_PACKZ = 16384, LDS_FFTY = 8192, LDS_C2R = 8192,
-              LDS_DHT = 16384, LDS_DHT_ROWS = 8192;
+// LDS bytes of an FFT buffer of the DHT row and column passes
+constexpr int LDS_DHT = 16384, LDS_DHT_ROWS = 8192;
 
 // sequences per LDS buffer of at most `budget` bytes, between 1 and 16
 __host__ __device__ constexpr int lds_batch(int n, int elem_bytes, int budget) {
@@ -71,67 +67,70 @@ __device__ __forceinline__ bool xcd_tile(int gx, int gy, int& tx, int& ty) {
 // Rows: renormalise, clamp, Log0 (UTR.cpp:951-958, 991), checkerboard
 // (-1)^(i+j) (the input Shuffle of UTR.cpp:993) and forward FFT along x,
 // two real rows per complex transform.
-// Persistent: each workgroup walks batches of NB rows (nbt batches in all,
-// nbr per image) and loads the next batch's pixels into registers while it
-// transforms the current one.
+// Persistent: each workgroup walks batches of NB pairs of rows (nbt batches in
+// all, nbr per image) and loads the next batch's pixels into registers while it
+// transforms the current one (Fft).  Bound by HBM.  Measured for 360 images of
+// 256^2 (189 MB in and out): 43.5 us, against 57 with every pass through LDS;
+// for 720 of 512^2 (1.5 GB): 350 against 437.
 template <typename T, int N>
-__global__ void __launch_bounds__(256) k_rows(const float* __restrict__ img,
+__global__ void __launch_bounds__(fft_threads(N)) k_rows(const float* __restrict__ img,
                                               cplx<T>* __restrict__ out, int ny, GeomDev g,
                                               const cplx<T>* __restrict__ tw, int nbr, int nbt) {
-    constexpr int NB = lds_batch(N, sizeof(cplx<T>), LDS_ROWS);
-    constexpr int PER = (NB * N + 255) / 256;  // pixels per thread and batch
-    __shared__ cplx<T> sm[2 * lds_len(NB * N)];
-    float xn[PER];
+    using F = Fft<N, T>;
+    constexpr int M = F::M;
+    __shared__ cplx<T> sm[F::LDS];
+    const int tid = threadIdx.x, co = F::Q::row_c(tid), i = F::Q::row_i(tid), npair = (ny + 1) >> 1;
+    // rows 2s and 2s+1 are the real and imaginary parts of sequence s
+    float xa[8], xb[8];
     auto fetch = [&](int bt) {
-        const int row = bt / nbr, j0 = (bt - row * nbr) * NB, nb = min(NB, ny - j0);
-        const float* src = img + ((size_t)row * ny + j0) * N;
+        const int row = bt / nbr, s = (bt - row * nbr) * F::NB + co;
+        const float* src = img + ((size_t)row * ny + 2 * s) * N + i;
 #pragma unroll
-        for (int k = 0; k < PER; k++) {
-            const int t = threadIdx.x + 256 * k;
-            xn[k] = t < nb * N ? src[t] : 0.f;
+        for (int r = 0; r < 8; r++) {
+            xa[r] = s < npair ? src[M * r] : 0.f;
+            xb[r] = 2 * s + 1 < ny ? src[N + M * r] : 0.f;
         }
     };
     if ((int)blockIdx.x < nbt) fetch(blockIdx.x);
     for (int bt = blockIdx.x; bt < nbt; bt += gridDim.x) {
-        float xc[PER];
-#pragma unroll
-        for (int k = 0; k < PER; k++) xc[k] = xn[k];
-        if (bt + (int)gridDim.x < nbt) fetch(bt + gridDim.x);
-        const int row = bt / nbr, j0 = (bt - row * nbr) * NB, nb = min(NB, ny - j0);
-        cplx<T>* a = sm;
-        cplx<T>* b = sm + lds_len(NB * N);
-#pragma unroll
-        for (int k = 0; k < PER; k++) {
-            const int t = threadIdx.x + 256 * k;
-            if (t >= nb * N) break;
-            const int jj = t / N, i = t - jj * N;
-            float x = xc[k];
+        const int row = bt / nbr, s = (bt - row * nbr) * F::NB + co;
+        const bool on = s < npair, two = 2 * s + 1 < ny;
+        auto field = [&](float x, int sg) {
             if (g.use_f1) x = x / g.f1;
             if (g.use_f2) x = x + g.f2;
             if (x < 0.f) x = 0.f;
-            T f = (x > 0.f) ? dev_log<T>(x) : T(0);
-            if ((i + j0 + jj) & 1) f = -f;
-            // rows 2s and 2s+1 are the real and imaginary parts of sequence s
-            T* e = reinterpret_cast<T*>(&a[lx((jj >> 1) * N + i)]);
-            e[jj & 1] = f;
-            if ((nb & 1) && jj == nb - 1) e[1] = T(0);
+            const T f = (x > 0.f) ? dev_log<T>(x) : T(0);
+            return (sg & 1) ? -f : f;
+        };
+        cplx<T> u[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            u[r].x = on ? field(xa[r], i + M * r) : T(0);
+            u[r].y = two ? field(xb[r], i + M * r + 1) : T(0);
         }
-        __syncthreads();
-        const int np = (nb + 1) >> 1;
-        fft_lds<T, N>(a, b, np, tw, -1, threadIdx.x, blockDim.x);
+        if (bt + (int)gridDim.x < nbt) fetch(bt + gridDim.x);
+        F::rows(u, sm, tw, -1, tid, false);
         // the two real rows' spectra from Z = X1 + i X2:
         // X1(k) = (Z(k) + conj Z(N-k)) / 2, X2(k) = (Z(k) - conj Z(N-k)) / 2i;
-        // columns 0 .. N/2 only: k_cols forms the others from the Hermitian symmetry
-        cplx<T>* dst = out + ((size_t)row * ny + j0) * N;
-        constexpr int W = N / 2 + 1;
-        for (int t = threadIdx.x; t < np * W; t += blockDim.x) {
-            const int sq = t / W, k = t - sq * W;
-            const cplx<T> z = a[lx(sq * N + k)], zm = a[lx(sq * N + (k == 0 ? 0 : N - k))];
-            dst[(size_t)(2 * sq) * N + k] = {T(0.5) * (z.x + zm.x), T(0.5) * (z.y - zm.y)};
-            if (2 * sq + 1 < nb)
-                dst[(size_t)(2 * sq + 1) * N + k] = {T(0.5) * (z.y + zm.y), T(-0.5) * (z.x - zm.x)};
+        // columns 0 .. N/2 only: k_cols forms the others from the Hermitian
+        // symmetry.  The upper halves go through LDS to their mirrors' threads.
+        __syncthreads();
+#pragma unroll
+        for (int r = 4; r < 8; r++) sm[co * F::Q::SEQ + lx(i + M * r)] = u[r];
+        __syncthreads();
+        cplx<T>* dst = out + ((size_t)row * ny + 2 * s) * N;
+        auto put = [&](int k, cplx<T> z, cplx<T> zm) {
+            if (on) dst[k] = {T(0.5) * (z.x + zm.x), T(0.5) * (z.y - zm.y)};
+            if (two) dst[N + k] = {T(0.5) * (z.y + zm.y), T(-0.5) * (z.x - zm.x)};
+        };
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int k = i + M * r;
+            cplx<T> zm = u[r];  // k = 0 is its own mirror
+            if (k != 0) zm = sm[co * F::Q::SEQ + lx(N - k)];
+            put(k, u[r], zm);
         }
-        __syncthreads();  // the next batch overwrites both buffers
+        if (i == 0) put(N / 2, u[4], u[4]);
     }
 }
 
@@ -259,14 +258,21 @@ __global__ void __launch_bounds__(256) k_prep_img(const float* __restrict__ img,
 // rowmax (optional): per-row max(|re|, |im|) of the result as float bits
 // (non-negative floats order like their bit patterns); it sets the
 // fixed-point scale of the brick gridding.
-template <typename T, int N>
-__global__ void __launch_bounds__(256) k_cols(cplx<T>* __restrict__ spec, int nx, int ncol, GeomDev g,
+// Bound by HBM: 64-byte column pieces through registers (Fft) with two barriers
+// a pass.  Measured for 360 images of 256^2 (284 MB): 58.9 us, against 90 with
+// every pass through LDS and 32-byte pieces; for 720 of 512^2 (2.3 GB): 634
+// against 1004.
+// FILTER: modes 1 and 3.  The values then pass through LDS once more (each
+// thread's own), so that the filter's FP64 code stands once and not eight times.
+template <typename T, int N, bool FILTER>
+__global__ void __launch_bounds__(fft_threads(N)) k_cols(cplx<T>* __restrict__ spec, int nx, int ncol, GeomDev g,
                                               const RowParams* __restrict__ rows, int row0,
                                               const cplx<T>* __restrict__ tw,
                                               unsigned* __restrict__ rowmax, int gx, int gy) {
-    constexpr int NB = lds_batch(N, sizeof(cplx<T>), LDS_COLS);
-    constexpr int PER = (NB * N + 255) / 256;  // elements per thread and tile
-    __shared__ cplx<T> sm[2 * lds_len(NB * N)];
+    using F = Fft<N, T>;
+    constexpr int NB = F::NB, M = F::M, NW = (F::NT + 63) / 64;
+    __shared__ cplx<T> sm[F::LDS];
+    __shared__ float s_wmax[NW];
     const int ny = N;
     const int total = gx * gy;
     // Persistent: in round k this workgroup takes tile tile_of(k); within a
@@ -275,54 +281,33 @@ __global__ void __launch_bounds__(256) k_cols(cplx<T>* __restrict__ spec, int nx
     // while the current one is transformed.  gridDim.x is a multiple of 8.
     const unsigned L = blockIdx.x, G = gridDim.x;
     auto tile_of = [&](int k) { return (int)(k * G + (L & 7u) * (G >> 3) + (L >> 3)); };
-    cplx<T> vn[PER];
+    const int tid = threadIdx.x, c = F::Q::col_c(tid), i = F::Q::col_i(tid);
+    cplx<T> vn[8];
     auto fetch = [&](int w) {
-        const int row = w / gx, x0 = (w - row * gx) * NB, nb = min(NB, ncol - x0);
-        const cplx<T>* src = spec + (size_t)row * ny * nx + x0;
+        const int row = w / gx, x = (w - row * gx) * NB + c;
+        const cplx<T>* src = spec + ((size_t)row * ny + i) * nx + x;
 #pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int t = threadIdx.x + 256 * q;
-            if (t < nb * N) {
-                const int y = t / nb, c = t - y * nb;
-                vn[q] = src[(size_t)y * nx + c];
-            }
-        }
+        for (int r = 0; r < 8; r++) vn[r] = x < ncol ? src[(size_t)(M * r) * nx] : cplx<T>{T(0), T(0)};
     };
     const int rounds = (total + (int)G - 1) / (int)G;
     if (tile_of(0) < total) fetch(tile_of(0));
     for (int rk = 0; rk < rounds; rk++) {
         const int wt = tile_of(rk);
-        cplx<T> vc[PER];
+        cplx<T> u[8];
 #pragma unroll
-        for (int q = 0; q < PER; q++) vc[q] = vn[q];
+        for (int r = 0; r < 8; r++) u[r] = vn[r];
         if (rk + 1 < rounds && tile_of(rk + 1) < total) fetch(tile_of(rk + 1));
         if (wt >= total) continue;  // uniform over the workgroup
-        cplx<T>* a = sm;
-        cplx<T>* b = sm + lds_len(NB * N);
         const int row = wt / gx;
-        const int x0 = (wt - row * gx) * NB;
-        const int nb = min(NB, ncol - x0);
+        const int kx = (wt - row * gx) * NB + c;
         cplx<T>* const rowbase = spec + (size_t)row * ny * nx;
-        cplx<T>* base = rowbase + x0;
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int t = threadIdx.x + 256 * q;
-            if (t < nb * N) {
-                const int y = t / nb, c = t - y * nb;
-                a[lx(c * N + y)] = vc[q];
-            }
-        }
-        __syncthreads();
-        fft_lds<T, N>(a, b, nb, tw, -1, threadIdx.x, blockDim.x);
+        F::cols(u, sm, tw, -1, tid, false);
         const RowParams& R = rows[row0 + row];
         const int gsgn = par_sign(g.nxd2 + g.nyd2);
         const double xap = g.xhi - g.xlo, yap = g.yhi - g.ylo;
         const double pi = 3.14159265358979323846;
         float vmax = 0.f;
-        for (int t = threadIdx.x; t < nb * N; t += blockDim.x) {
-            const int ky = t / nb, c = t - ky * nb;
-            const int kx = x0 + c;
-            cplx<T> v = a[lx(c * N + ky)];
+        auto emit = [&](int ky, cplx<T> v) {
             const T s = T(par_sign(kx + ky) * gsgn);
             v.x *= s;
             v.y *= s;
@@ -332,7 +317,7 @@ __global__ void __launch_bounds__(256) k_cols(cplx<T>* __restrict__ spec, int nx
             // both values
             const bool mirror = kx > 0 && kx < g.nxd2;
             cplx<T> vm = {v.x, -v.y};
-            if (g.ctf_mode == 1 && R.zout != 0) {
+            if (FILTER && g.ctf_mode == 1 && R.zout != 0) {
                 // 2D TIE-Hom restated from UTR.h:159-181 in 2D (unpinned)
                 const double i1 = kx - g.nxd2, j1 = ky - g.nyd2;
                 const double q2 = 4.0 * pi * pi * (i1 * i1 / (xap * xap) + j1 * j1 / (yap * yap));
@@ -341,7 +326,7 @@ __global__ void __launch_bounds__(256) k_cols(cplx<T>* __restrict__ spec, int nx
                 v.y *= f;
                 vm.x *= f;
                 vm.y *= f;
-            } else if (g.ctf_mode == 3) {
+            } else if (FILTER && g.ctf_mode == 3) {
                 // 2D CTF inversion restated from UTR.h:70-128 in 2D (unpinned):
                 // at centred frequency (i1, j1), inside the aperture, u -> u (sr - i cr)
                 const double dk2 = 1.0 / (xap * xap), de2 = 1.0 / (yap * yap);
@@ -390,25 +375,37 @@ __global__ void __launch_bounds__(256) k_cols(cplx<T>* __restrict__ spec, int nx
                 vm.x *= T(R.weight);
                 vm.y *= T(R.weight);
             }
-            base[(size_t)ky * nx + c] = v;
+            rowbase[(size_t)ky * nx + kx] = v;
             if (mirror) {
                 rowbase[(size_t)(ky == 0 ? 0 : ny - ky) * nx + (nx - kx)] = vm;
                 vmax = fmaxf(vmax, fmaxf(fabsf((float)vm.x), fabsf((float)vm.y)));
             }
             vmax = fmaxf(vmax, fmaxf(fabsf((float)v.x), fabsf((float)v.y)));
+        };
+        if constexpr (FILTER) {
+            cplx<T>* own = sm + c * F::Q::SEQ;
+            __syncthreads();  // the transform's last reads
+#pragma unroll
+            for (int r = 0; r < 8; r++) own[lx(i + M * r)] = u[r];
+            if (kx < ncol) {
+#pragma unroll 1
+                for (int r = 0; r < 8; r++) emit(i + M * r, own[lx(i + M * r)]);
+            }
+        } else if (kx < ncol) {
+#pragma unroll
+            for (int r = 0; r < 8; r++) emit(i + M * r, u[r]);
         }
         if (rowmax) {
             // one atomic per workgroup (rowmax is a kernel argument: uniform branch)
-            __shared__ float s_wmax[4];
             for (int off = 32; off > 0; off >>= 1) vmax = fmaxf(vmax, __shfl_xor(vmax, off));
-            if ((threadIdx.x & 63) == 0) s_wmax[threadIdx.x >> 6] = vmax;
+            if ((tid & 63) == 0) s_wmax[tid >> 6] = vmax;
             __syncthreads();
-            if (threadIdx.x == 0) {
-                const float m = fmaxf(fmaxf(s_wmax[0], s_wmax[1]), fmaxf(s_wmax[2], s_wmax[3]));
+            if (tid == 0) {
+                float m = s_wmax[0];
+                for (int w = 1; w < NW; w++) m = fmaxf(m, s_wmax[w]);
                 atomicMax(&rowmax[row0 + row], __float_as_uint(m));
             }
         }
-        __syncthreads();  // the next tile overwrites both buffers
     }
 }
 
@@ -1655,30 +1652,35 @@ __host__ __device__ constexpr int h_stride(int nx) { return (nx / 2 + 1 + 7) & ~
 // Nyquist x-plane (centred i = 0): the serial loop order of the reference
 // gives H = (3a + 5 conj b)/8 when (k,j) precedes its mirror, (5a + 3 conj b)/8
 // when it follows it, and Re(a) when it is its own mirror.
+// Bound by HBM (V read once, half of it through mirrored columns).  Through
+// registers (Fft), 256^3 (202 MB): 50.9 us, against 61 through LDS; 512^3: 482
+// against 651.
 template <typename T, int NZ>
-__global__ void __launch_bounds__(256) k_pack_z(const cplx<T>* __restrict__ V,
+__global__ void __launch_bounds__(fft_threads(NZ)) k_pack_z(const cplx<T>* __restrict__ V,
                                                 cplx<T>* __restrict__ H, GeomDev g,
                                                 const cplx<T>* __restrict__ tw, int gx, int gy) {
-    constexpr int CW = lds_batch(NZ, sizeof(cplx<T>), LDS_PACKZ);
-    __shared__ cplx<T> sm[2 * lds_len(CW * NZ)];
-    cplx<T>* a = sm;
-    cplx<T>* b = sm + lds_len(CW * NZ);
+    using F = Fft<NZ, T>;
+    constexpr int M = F::M;
+    __shared__ cplx<T> sm[F::LDS];
     const int nx = g.nx, ny = g.ny, W = nx / 2 + 1, WP = h_stride(nx);
     int tx, ty;
     if (!xcd_tile(gx, gy, tx, ty)) return;
-    const int j = ty;
-    const int w0 = tx * CW;
-    const int nb = min(CW, W - w0);
+    const int j = ty, tid = threadIdx.x;
+    const int w = tx * F::NB + F::Q::col_c(tid), k0 = F::Q::col_i(tid);
+    const bool on = w < W;
     const int ja = (j == 0) ? 0 : ny - j;
-    for (int t = threadIdx.x; t < nb * NZ; t += blockDim.x) {
-        const int k = t / nb, c = t - k * nb;
-        const int w = w0 + c;
-        const int i = (w == nx / 2) ? 0 : w + g.nxd2;
-        const int ia = (i == 0) ? 0 : nx - i;
+    const int i = (w == nx / 2) ? 0 : w + g.nxd2;
+    const int ia = (i == 0) ? 0 : nx - i;
+    cplx<T> u[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+        const int k = k0 + M * r;
         const int ka = (k == 0) ? 0 : NZ - k;
-        const cplx<T> va = V[((size_t)k * ny + j) * nx + i];
-        const cplx<T> vb = V[((size_t)ka * ny + ja) * nx + ia];
-        cplx<T> h;
+        cplx<T> va = {T(0), T(0)}, vb = {T(0), T(0)}, h;
+        if (on) {
+            va = V[((size_t)k * ny + j) * nx + i];
+            vb = V[((size_t)ka * ny + ja) * nx + ia];
+        }
         if (i != 0) {
             h = {T(0.5) * (va.x + vb.x), T(0.5) * (va.y - vb.y)};
         } else if (k == ka && j == ja) {
@@ -1692,109 +1694,104 @@ __global__ void __launch_bounds__(256) k_pack_z(const cplx<T>* __restrict__ V,
             h.x = -h.x;
             h.y = -h.y;
         }
-        a[lx(c * NZ + k)] = h;
+        u[r] = h;
     }
-    __syncthreads();
-    fft_lds<T, NZ>(a, b, nb, tw, +1, threadIdx.x, blockDim.x);
-    for (int t = threadIdx.x; t < nb * NZ; t += blockDim.x) {
-        const int k = t / nb, c = t - k * nb;
-        H[((size_t)k * ny + j) * WP + w0 + c] = a[lx(c * NZ + k)];
-    }
+    F::cols(u, sm, tw, +1, tid, true);
+    if (!on) return;
+#pragma unroll
+    for (int r = 0; r < 8; r++) H[((size_t)(k0 + M * r) * ny + j) * WP + w] = u[r];
 }
 
-// Inverse FFT along y of the half spectrum, in place.
+// Inverse FFT along y of the half spectrum, in place.  256^3 (136 MB): 27.5 us
+// through registers (Fft), 36 through LDS; 512^3: 220 against 411.
 template <typename T, int NY>
-__global__ void __launch_bounds__(256) k_fft_y(cplx<T>* __restrict__ H, GeomDev g,
+__global__ void __launch_bounds__(fft_threads(NY)) k_fft_y(cplx<T>* __restrict__ H, GeomDev g,
                                                const cplx<T>* __restrict__ tw, int gx, int gy) {
-    constexpr int CW = lds_batch(NY, sizeof(cplx<T>), LDS_FFTY);
-    __shared__ cplx<T> sm[2 * lds_len(CW * NY)];
-    cplx<T>* a = sm;
-    cplx<T>* b = sm + lds_len(CW * NY);
+    using F = Fft<NY, T>;
+    constexpr int M = F::M;
+    __shared__ cplx<T> sm[F::LDS];
     const int W = g.nx / 2 + 1, WP = h_stride(g.nx);
     int tx, ty;
     if (!xcd_tile(gx, gy, tx, ty)) return;
-    const int k = ty;
-    const int w0 = tx * CW;
-    const int nb = min(CW, W - w0);
-    cplx<T>* base = H + (size_t)k * NY * WP + w0;
-    for (int t = threadIdx.x; t < nb * NY; t += blockDim.x) {
-        const int y = t / nb, c = t - y * nb;
-        a[lx(c * NY + y)] = base[(size_t)y * WP + c];
-    }
-    __syncthreads();
-    fft_lds<T, NY>(a, b, nb, tw, +1, threadIdx.x, blockDim.x);
-    for (int t = threadIdx.x; t < nb * NY; t += blockDim.x) {
-        const int y = t / nb, c = t - y * nb;
-        base[(size_t)y * WP + c] = a[lx(c * NY + y)];
-    }
+    const int tid = threadIdx.x, w = tx * F::NB + F::Q::col_c(tid);
+    const bool on = w < W;
+    cplx<T>* base = H + ((size_t)ty * NY + F::Q::col_i(tid)) * WP + w;
+    cplx<T> u[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++) u[r] = on ? base[(size_t)(M * r) * WP] : cplx<T>{T(0), T(0)};
+    F::cols(u, sm, tw, +1, tid, true);
+    if (!on) return;
+#pragma unroll
+    for (int r = 0; r < 8; r++) base[(size_t)(M * r) * WP] = u[r];
 }
 
 // Complex-to-real inverse FFT along x of two rows at once (z = x1 + i x2),
 // then (-1)^(k+j+(nz+ny)/2)/N, sphere mask, cupping compensation and final
-// scale (UTR.cpp:1235-1279).
+// scale (UTR.cpp:1235-1279).  256^3 (135 MB): 35.7 us through registers (Fft),
+// 43 through LDS; 512^3: 305 against 362.
 template <typename T, int NX, typename TO>
-__global__ void __launch_bounds__(256) k_c2r_x(const cplx<T>* __restrict__ H,
+__global__ void __launch_bounds__(fft_threads(NX)) k_c2r_x(const cplx<T>* __restrict__ H,
                                                TO* __restrict__ vol, GeomDev g,
                                                const cplx<T>* __restrict__ tw, int gx, int gy) {
-    constexpr int NB = lds_batch(NX, sizeof(cplx<T>), LDS_C2R);
-    __shared__ cplx<T> sm[2 * lds_len(NB * NX)];
-    cplx<T>* a = sm;
-    cplx<T>* b = sm + lds_len(NB * NX);
-    const int ny = g.ny, WP = h_stride(NX);
+    using F = Fft<NX, T>;
+    constexpr int NB = F::NB, M = F::M;
+    __shared__ cplx<T> sm[F::LDS];
+    __shared__ double s_ex[NX], s_ey[2 * NB];
+    const int ny = g.ny, WP = h_stride(NX), tid = threadIdx.x;
     int tx, ty;
     if (!xcd_tile(gx, gy, tx, ty)) return;
     const int k = ty;
     const int p0 = tx * NB;  // first row pair
-    const int np = min(NB, ny / 2 - p0);
-    for (int t = threadIdx.x; t < np * NX; t += blockDim.x) {
-        const int pp = t / NX, w = t - pp * NX;
-        const int j = 2 * (p0 + pp);
-        const cplx<T>* r1 = H + ((size_t)k * ny + j) * WP;
-        const cplx<T>* r2 = r1 + WP;
-        cplx<T> x1, x2;
-        if (w <= NX / 2) {
-            x1 = r1[w];
-            x2 = r2[w];
-        } else {
-            x1 = r1[NX - w];
-            x2 = r2[NX - w];
-            x1.y = -x1.y;
-            x2.y = -x2.y;
+    const int pp = F::Q::row_c(tid), i = F::Q::row_i(tid), j = 2 * (p0 + pp);
+    const bool on = p0 + pp < ny / 2;
+    const cplx<T>* r1 = H + ((size_t)k * ny + j) * WP;
+    const cplx<T>* r2 = r1 + WP;
+    cplx<T> u[8];
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+        const int w = i + M * r;
+        cplx<T> x1 = {T(0), T(0)}, x2 = {T(0), T(0)};
+        if (on) {
+            const int wm = w <= NX / 2 ? w : NX - w;
+            x1 = r1[wm];
+            x2 = r2[wm];
+            if (w > NX / 2) {
+                x1.y = -x1.y;
+                x2.y = -x2.y;
+            }
         }
-        a[lx(t)] = {x1.x - x2.y, x1.y + x2.x};
+        u[r] = {x1.x - x2.y, x1.y + x2.x};
     }
-    __syncthreads();
-    fft_lds<T, NX>(a, b, np, tw, +1, threadIdx.x, blockDim.x);
-    const double invN = 1.0 / ((double)NX * ny * g.nz);
-    const int gs = par_sign((g.nz + ny) / 2);
     // The cupping factor exp(dtemp*(di^2 + dj^2 + dk^2)) is the product of one
-    // factor per axis: x factors go to the free FFT buffer, the block's 2*NB
-    // y factors to a small table, and the z factor is one value per block.
-    __shared__ double s_ey[2 * NB];
-    double* s_ex = reinterpret_cast<double*>(b);
-    static_assert(sizeof(double) <= NB * sizeof(cplx<T>), "x factors must fit the FFT scratch buffer");
+    // factor per axis: tables of the x factors and of the block's 2*NB y
+    // factors (the transform's barriers come before they are read), and the z
+    // factor is one value per block.
     if (!g.no_mask) {
-        for (int m = threadIdx.x; m < NX; m += blockDim.x)
+        for (int m = tid; m < NX; m += F::NT)
             s_ex[m] = exp(g.mask_dtemp * (double)((long)(m - g.ic) * (m - g.ic)));
-        if (threadIdx.x < 2 * np) {
-            const int jj = 2 * p0 + threadIdx.x;
-            s_ey[threadIdx.x] = g.mask_j ? exp(g.mask_dtemp * (double)((long)(jj - g.jc) * (jj - g.jc))) : 1.0;
+        if (tid < 2 * NB) {
+            const int jj = 2 * p0 + tid;
+            s_ey[tid] = g.mask_j ? exp(g.mask_dtemp * (double)((long)(jj - g.jc) * (jj - g.jc))) : 1.0;
         }
-        __syncthreads();
     }
     const double ez = (g.mask_k && !g.no_mask) ? exp(g.mask_dtemp * (double)((long)(k - g.kc) * (k - g.kc))) : 1.0;
+    F::rows(u, sm, tw, +1, tid, true);
+    if (!on) return;
+    const double invN = 1.0 / ((double)NX * ny * g.nz);
+    const int gs = par_sign((g.nz + ny) / 2);
     const double base_f = g.fnorm * invN * (double)gs;
-    for (int t = threadIdx.x; t < np * NX; t += blockDim.x) {
-        const int pp = t / NX, m = t - pp * NX;
-        const int j = 2 * (p0 + pp);
-        const cplx<T> z = a[lx(t)];
-        for (int h = 0; h < 2; h++) {
-            const int jj = j + h;
-            const T val = h ? z.y : z.x;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int jj = j + h;
+        const double sgn = (double)par_sign(k + jj);
+        TO* dst = vol + ((size_t)k * ny + jj) * NX;
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const int m = i + M * r;
+            const T val = h ? u[r].y : u[r].x;
             long ii2 = (long)(m - g.ic) * (m - g.ic);
             if (g.mask_j) ii2 += (long)(jj - g.jc) * (jj - g.jc);
             if (g.mask_k) ii2 += (long)(k - g.kc) * (k - g.kc);
-            const double sgn = (double)par_sign(k + jj);
             TO o;
             if (g.no_mask) {
                 o = TO((double)val * (base_f * sgn));
@@ -1804,7 +1801,7 @@ __global__ void __launch_bounds__(256) k_c2r_x(const cplx<T>* __restrict__ H,
                 const double f = s_ex[m] * s_ey[2 * pp + h] * ez * base_f * sgn;
                 o = TO((double)val * f);
             }
-            vol[((size_t)k * ny + jj) * NX + m] = o;
+            dst[m] = o;
         }
     }
 }

@@ -25,3 +25,31 @@ def test_multislice_lengths(nx, ny, mode):
     ref = M.images(dict(nx=nx, ny=ny, ctb=ctb, deltaz=1.6, kev=200.0, mode=mode), at, np.radians(angZ),
                    np.radians(angY), defocus, output="complex")
     assert np.linalg.norm(psi - ref) / np.linalg.norm(ref) < 1e-5
+
+
+@pytest.mark.parametrize("nx,ny", [(16, 16), (16, 48), (32, 32), (32, 64), (48, 32), (48, 160), (64, 16)])
+def test_potential_of_narrow_rows(nx, ny, monkeypatch):
+    """Rows summed a pixel a thread (up to 48 pixels) and eight pixels a thread
+    (64), with more atoms in a slice than a workgroup lists at once and a row
+    count that the workgroups do not divide: the tile form's bits, the FP64
+    oracle to 1e-5, and the oracle's Debye-Waller filter of the raw potential
+    to the 1e-5 of test_gpu_msct.py."""
+    print("narrow rows", nx, ny, flush=True)
+    ctb = 19.2
+    p = U.default_msct_params(nx=nx, ny=ny, ctblength=ctb, deltaz=9.6, kev=200.0, output=2)
+    rng = np.random.default_rng(nx + 7 * ny)
+    n = 600
+    xyz = rng.uniform(4.0, 15.0, (3, n)).astype(np.float32)
+    at = dict(Z=rng.choice([6, 8], n).astype(np.int32), x=xyz[0], y=xyz[1], z=xyz[2], occ=np.full(n, 0.05, np.float32),
+              wobble=np.full(n, 0.1, np.float32))
+    ang = [5.0, 250.0], [33.0, 160.0]
+    psi = U.multislice_images(p, at, *ang, [0.0])
+    monkeypatch.setenv("UTR_MSCT_FUSED", "0")
+    assert np.array_equal(psi.view(np.uint32), U.multislice_images(p, at, *ang, [0.0]).view(np.uint32))
+    monkeypatch.delenv("UTR_MSCT_FUSED")
+    op = dict(nx=nx, ny=ny, ctb=ctb, deltaz=9.6, kev=200.0, mode=0)
+    ref = M.images(op, at, np.radians(ang[0]), np.radians(ang[1]), [0.0], output="complex")
+    assert np.linalg.norm(psi - ref) / np.linalg.norm(ref) < 1e-5
+    got = U.multislice_images(dict(p, output=0, nwobble=1), at, *ang, [0.0])
+    ref = M.images(dict(op, nwobble=1, temperature=300.0), at, np.radians(ang[0]), np.radians(ang[1]), [0.0])
+    assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < 1e-5

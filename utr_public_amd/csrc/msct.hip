@@ -161,7 +161,17 @@ __global__ void __launch_bounds__(256) k_ms_potential(const MsAtom* __restrict__
 // so the result are the same bit for bit), kept columns only unless raw.
 // A thread holds pixels i + M r of one row (Fft), M pixels apart: where that is
 // wider than an atom's window at most one of them meets it, found without a
-// test per pixel.  grid (row groups, orientation).
+// test per pixel.  Rows of at most MS_PX pixels, where the window spans several
+// of a thread's pixels and a workgroup would take the whole image, sum a pixel
+// a thread over ms_pot_rows rows instead and pass them to the FFT through LDS:
+// a call of one orientation and 1000 atoms, eight pixels a thread and one, takes
+// 4.06 and 0.98 ms at 16^2, 1.94 and 0.82 at 32^2, 1.50 and 0.87 at 48^2.  At 64^2
+// it is 1.18 and 0.80, but 720 orientations 2.88 and 3.78: the FFT then fills an
+// eighth of the workgroup, and many orientations need no more workgroups.
+// grid (row groups, orientation).
+constexpr int MS_PX = 48;
+template <int N>
+__host__ __device__ constexpr int ms_pot_rows() { return N <= MS_PX ? Fft<N>::NT / N : Fft<N>::NB; }
 template <int N>
 __global__ void __launch_bounds__(Fft<N>::NT) k_ms_potential_rows(const MsAtom* __restrict__ atoms,
                                                            const int* __restrict__ off, int natom, int s,
@@ -170,7 +180,8 @@ __global__ void __launch_bounds__(Fft<N>::NT) k_ms_potential_rows(const MsAtom* 
                                                            cplx<float>* __restrict__ trans,
                                                            const cplx<float>* __restrict__ tw, int raw, int lim) {
     using F = Fft<N>;
-    constexpr int NT = F::NT, NB = F::NB, M = F::M, NW = (NT + 63) / 64;
+    constexpr int NT = F::NT, NB = ms_pot_rows<N>(), M = F::M, NW = (NT + 63) / 64;
+    constexpr bool PX = N <= MS_PX;
     __shared__ cplx<float> sm[F::LDS];
     __shared__ MsAtom sa[NT];
     __shared__ int wcount[NW];
@@ -180,7 +191,8 @@ __global__ void __launch_bounds__(Fft<N>::NT) k_ms_potential_rows(const MsAtom* 
     const int y0 = blockIdx.x * NB;
     const int nb = min(NB, g.ny - y0);
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int row = F::Q::row_c(tid), i = F::Q::row_i(tid), py = y0 + row;
+    // this thread's row, and its pixel (PX) or the first of its eight
+    const int row = PX ? tid / N : F::Q::row_c(tid), i = PX ? tid % N : F::Q::row_i(tid), py = y0 + row;
     const MsAtom* A = atoms + (size_t)o * natom;
     float acc[8];
 #pragma unroll
@@ -223,14 +235,14 @@ __global__ void __launch_bounds__(Fft<N>::NT) k_ms_potential_rows(const MsAtom* 
             const int iy = yw + ms_pmod(py - yw, g.ny);
             if (iy > t.iyo + g.idy || row >= nb) continue;
             const double ry = (double)t.y - (double)iy * g.sy;
-            for (int d = ms_pmod(i - xw, M); d <= 2 * g.idx; d += M) {
+            for (int d = ms_pmod(i - xw, PX ? N : M); d <= 2 * g.idx; d += PX ? N : M) {
                 const int ix = xw + d;
                 const double rx = (double)t.x - (double)ix * g.sx;
                 double r2 = ms_r2(rx, ry);
                 if (r2 > 9.0) continue;
                 if (r2 < g.rminsq) r2 = g.rminsq;
                 const float v = (float)((double)t.occ * ms_lut(knots, coef + (size_t)t.zi * MS_NR, r2, g));
-                const int rr = ms_pmod(ix, N) / M;
+                const int rr = PX ? 0 : ms_pmod(ix, N) / M;
 #pragma unroll
                 for (int r = 0; r < 8; r++)
                     if (r == rr) acc[r] += v;
@@ -239,7 +251,7 @@ __global__ void __launch_bounds__(Fft<N>::NT) k_ms_potential_rows(const MsAtom* 
     }
     cplx<float> u[8];
 #pragma unroll
-    for (int r = 0; r < 8; r++) {
+    for (int r = 0; r < (PX ? 1 : 8); r++) {
         if (raw) {  // the potential itself, for the Debye-Waller filter
             u[r] = {acc[r], 0.f};
         } else {
@@ -251,12 +263,20 @@ __global__ void __launch_bounds__(Fft<N>::NT) k_ms_potential_rows(const MsAtom* 
             u[r] = {cs, sn};
         }
     }
-    F::rows(u, sm, tw, +1, tid, true);
-    if (row >= nb) return;
-    cplx<float>* out = trans + ((size_t)o * g.ny + py) * N;
+    const int frow = F::Q::row_c(tid), fi = F::Q::row_i(tid);
+    if constexpr (PX) {
+        sm[row * F::Q::SEQ + lx(i)] = u[0];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 8; r++)
+            u[r] = frow < NB ? sm[frow * F::Q::SEQ + lx(fi + M * r)] : cplx<float>{0.f, 0.f};
+    }
+    F::rows(u, sm, tw, +1, tid, !PX);
+    if (frow >= nb) return;
+    cplx<float>* out = trans + ((size_t)o * g.ny + y0 + frow) * N;
 #pragma unroll
     for (int r = 0; r < 8; r++)
-        if (raw || ms_kept(i + M * r, N, lim)) out[i + M * r] = u[r];
+        if (raw || ms_kept(fi + M * r, N, lim)) out[fi + M * r] = u[r];
 }
 
 // x FFT (exponent +1) of lines of [B][ny][nx], in place.
@@ -724,7 +744,8 @@ int ms_run_lines(msct_ctx* c, int what, int B, int s, int ndef, int d, float* ou
                 utr::k_ms_mul<N, false><<<groups, NT, 0, st>>>(c->W.p, c->T.p, ny, nlines, c->lim, c->twx.p, \
                                                                c->off.p, c->g.nsl1, s);             \
         } else if (what == 4) {                                                                     \
-            utr::k_ms_potential_rows<N><<<dim3((ny + NB - 1) / NB, B), NT, 0, st>>>(                \
+            constexpr int NR = utr::ms_pot_rows<N>();                                               \
+            utr::k_ms_potential_rows<N><<<dim3((ny + NR - 1) / NR, B), NT, 0, st>>>(                \
                 c->atoms.p, c->off.p, c->natom, s, c->g, c->knots.p, c->coef.p, c->scale, c->T.p,   \
                 c->twx.p, c->p.nwobble == 1 ? 1 : 0, c->lim);                                       \
         } else if (what == 5) {                                                                     \

@@ -262,8 +262,10 @@ __global__ void __launch_bounds__(256) k_prep_img(const float* __restrict__ img,
 // a pass.  Measured for 360 images of 256^2 (284 MB): 58.9 us, against 90 with
 // every pass through LDS and 32-byte pieces; for 720 of 512^2 (2.3 GB): 634
 // against 1004.
-// FILTER: modes 1 and 3.  The values then pass through LDS once more (each
-// thread's own), so that the filter's FP64 code stands once and not eight times.
+// FILTER: modes 1 and 3.  The values then pass through LDS once more, so that
+// the filter's FP64 code stands once and not eight times and all threads share
+// it where a tile has fewer columns than NB (a thread's own values only: 10.1
+// against 4.5 us a row of 16^2 in FP64, 14.1 against 12.3 for 300 of 48^2).
 template <typename T, int N, bool FILTER>
 __global__ void __launch_bounds__(fft_threads(N)) k_cols(cplx<T>* __restrict__ spec, int nx, int ncol, GeomDev g,
                                               const RowParams* __restrict__ rows, int row0,
@@ -307,7 +309,7 @@ __global__ void __launch_bounds__(fft_threads(N)) k_cols(cplx<T>* __restrict__ s
         const double xap = g.xhi - g.xlo, yap = g.yhi - g.ylo;
         const double pi = 3.14159265358979323846;
         float vmax = 0.f;
-        auto emit = [&](int ky, cplx<T> v) {
+        auto emit = [&](int ky, int kx, cplx<T> v) {
             const T s = T(par_sign(kx + ky) * gsgn);
             v.x *= s;
             v.y *= s;
@@ -383,17 +385,21 @@ __global__ void __launch_bounds__(fft_threads(N)) k_cols(cplx<T>* __restrict__ s
             vmax = fmaxf(vmax, fmaxf(fabsf((float)v.x), fabsf((float)v.y)));
         };
         if constexpr (FILTER) {
-            cplx<T>* own = sm + c * F::Q::SEQ;
+            // all threads take values of the tile's columns, also where it has
+            // fewer than NB
+            const int x0 = (wt - row * gx) * NB, nb = min(NB, ncol - x0);
             __syncthreads();  // the transform's last reads
 #pragma unroll
-            for (int r = 0; r < 8; r++) own[lx(i + M * r)] = u[r];
-            if (kx < ncol) {
+            for (int r = 0; r < 8; r++) sm[c * F::Q::SEQ + lx(i + M * r)] = u[r];
+            __syncthreads();
 #pragma unroll 1
-                for (int r = 0; r < 8; r++) emit(i + M * r, own[lx(i + M * r)]);
+            for (int t = tid; t < nb * N; t += F::NT) {
+                const int ky = t / nb, cc = t - ky * nb;
+                emit(ky, x0 + cc, sm[cc * F::Q::SEQ + lx(ky)]);
             }
         } else if (kx < ncol) {
 #pragma unroll
-            for (int r = 0; r < 8; r++) emit(i + M * r, u[r]);
+            for (int r = 0; r < 8; r++) emit(i + M * r, kx, u[r]);
         }
         if (rowmax) {
             // one atomic per workgroup (rowmax is a kernel argument: uniform branch)

@@ -40,3 +40,28 @@ def test_transform_lengths(nx, ny, nz, mode, kw, form):
         assert rel(U.reconstruct(p, r, imgs), ref) < 1e-5
     else:
         assert rel(U.reconstruct(p, r, imgs, U.UTR_FP64, f64_out=True), ref) < 1e-10
+
+
+@pytest.mark.parametrize("nx,ny,rows", [(16, 64, 300), (32, 16, 200), (48, 96, 150), (64, 64, 136)])
+def test_narrow_rows_in_parts_and_at_once(nx, ny, rows):
+    """Up to 64 pixels the row transform takes a pixel pair a thread for few
+    rows and eight for many: a few rows at a time from host memory and all at
+    once on the device give the same bits, and the FP64 oracle to 1e-5."""
+    import torch
+    print("narrow rows", nx, ny, rows, flush=True)
+    xst, nz = 0.4, 32
+    p = U.default_params(nx=nx, ny=ny, xst=xst, zlo=-nz * xst / 2, zhi=nz * xst / 2, escc=1, nsr=0.05)
+    rng = np.random.default_rng(nx + rows)
+    angZ, angY = np.zeros(rows), rng.uniform(0, 180, rows)
+    r = dict(angZ=angZ, angY=angY, defocus=np.full(rows, 300.0))
+    xyz, Z = synth.atoms(3, 10, "cube", min(nx, ny, nz) * xst * 0.4, 1.0, ([6], [1.0]))
+    imgs = synth.project(xyz, Z, nx, ny, xst, angZ, angY, dose=400.0, seed=3)
+    parts = U.reconstruct(p, r, imgs)
+    dev = torch.from_numpy(imgs).cuda()
+    vol = torch.empty(parts.shape, dtype=torch.float32, device="cuda")
+    with U.Reconstructor(p, r) as rec:
+        rec.add_images_device(dev.data_ptr(), rows)
+        rec.finalize_device(vol.data_ptr())
+        torch.cuda.synchronize()
+    assert np.array_equal(parts.view(np.uint32), vol.cpu().numpy().view(np.uint32))
+    assert rel(parts, oracle.reconstruct(p, r, imgs)) < 1e-5

@@ -332,16 +332,28 @@ int launch_2d(utr_ctx* c, const float* d_img, int row0, int count, cplx<T>* d_sp
     const auto& g = c->plan.g;
     if (count <= 0) return UTR_OK;
     bool ok = false;
+    // rows up to 64 pixels: one pixel pair a thread (k_rows) in FP64 and where
+    // the other form has fewer workgroups than half the compute units
+#define UTR_ROWS1(N, ONE)                                                                       \
+    {                                                                                           \
+        constexpr int NP = utr::rows_pairs<N, ONE>();                                           \
+        const int nbr = (npair + NP - 1) / NP, nbt = nbr * count;                               \
+        const int grid = std::min(nbt, c->ncu * (c->rows_wpc > 0 ? c->rows_wpc : F::WPC));      \
+        utr::k_rows<T, N, ONE><<<grid, F::NT, 0, c->stream>>>(d_img, d_spec, g.ny, g, twx, nbr, nbt); \
+    }
 #define UTR_ROWS(N)                                                                             \
     {                                                                                           \
         using F = utr::Fft<N, T>;                                                               \
-        const int nbr = ((g.ny + 1) / 2 + F::NB - 1) / F::NB, nbt = nbr * count;                \
-        const int grid = std::min(nbt, c->ncu * (c->rows_wpc > 0 ? c->rows_wpc : F::WPC));      \
-        utr::k_rows<T, N><<<grid, F::NT, 0, c->stream>>>(d_img, d_spec, g.ny, g, twx, nbr, nbt); \
+        const int npair = (g.ny + 1) / 2;                                                       \
+        if (N <= 64 && (sizeof(T) == 8 || 2L * count * ((npair + F::NB - 1) / F::NB) < c->ncu)) \
+            UTR_ROWS1(N, (N <= 64))                                                             \
+        else                                                                                    \
+            UTR_ROWS1(N, false)                                                                 \
         ok = true;                                                                              \
     }
     UTR_DISPATCH_N(g.nx, UTR_ROWS)
 #undef UTR_ROWS
+#undef UTR_ROWS1
     if (!ok) return set_err(UTR_E_UNSUPPORTED, "unsupported image width for the FFT");
     ok = false;
 #define UTR_COLS(N)                                                                             \

@@ -72,29 +72,36 @@ __device__ __forceinline__ bool xcd_tile(int gx, int gy, int& tx, int& ty) {
 // transforms the current one (Fft).  Bound by HBM.  Measured for 360 images of
 // 256^2 (189 MB in and out): 43.5 us, against 57 with every pass through LDS;
 // for 720 of 512^2 (1.5 GB): 350 against 437.
-template <typename T, int N>
+// ONE: a thread takes the logarithms of one pixel pair and passes them to the
+// FFT through LDS, so that few short rows spread over more workgroups (8 images
+// of 64^2: 3.9 us against 5.2, 720: 16.6 against 12.2; in FP64, an image of 64^2
+// at a time, 4.4 against 6.9).
+template <int N, bool ONE>
+__host__ __device__ constexpr int rows_pairs() { return ONE ? fft_threads(N) / N : Fft<N>::NB; }
+template <typename T, int N, bool ONE>
 __global__ void __launch_bounds__(fft_threads(N)) k_rows(const float* __restrict__ img,
                                               cplx<T>* __restrict__ out, int ny, GeomDev g,
                                               const cplx<T>* __restrict__ tw, int nbr, int nbt) {
     using F = Fft<N, T>;
-    constexpr int M = F::M;
+    constexpr int M = F::M, NB = rows_pairs<N, ONE>(), PER = ONE ? 1 : 8;
     __shared__ cplx<T> sm[F::LDS];
     const int tid = threadIdx.x, co = F::Q::row_c(tid), i = F::Q::row_i(tid), npair = (ny + 1) >> 1;
+    const int pco = ONE ? tid / N : co, pi = ONE ? tid % N : i;  // the pixels this thread loads
     // rows 2s and 2s+1 are the real and imaginary parts of sequence s
-    float xa[8], xb[8];
+    float xa[PER], xb[PER];
     auto fetch = [&](int bt) {
-        const int row = bt / nbr, s = (bt - row * nbr) * F::NB + co;
-        const float* src = img + ((size_t)row * ny + 2 * s) * N + i;
+        const int row = bt / nbr, s = (bt - row * nbr) * NB + pco;
+        const float* src = img + ((size_t)row * ny + 2 * s) * N + pi;
 #pragma unroll
-        for (int r = 0; r < 8; r++) {
+        for (int r = 0; r < PER; r++) {
             xa[r] = s < npair ? src[M * r] : 0.f;
             xb[r] = 2 * s + 1 < ny ? src[N + M * r] : 0.f;
         }
     };
     if ((int)blockIdx.x < nbt) fetch(blockIdx.x);
     for (int bt = blockIdx.x; bt < nbt; bt += gridDim.x) {
-        const int row = bt / nbr, s = (bt - row * nbr) * F::NB + co;
-        const bool on = s < npair, two = 2 * s + 1 < ny;
+        const int row = bt / nbr, s0 = (bt - row * nbr) * NB, s = s0 + co;
+        const bool on = co < NB && s < npair, two = co < NB && 2 * s + 1 < ny;
         auto field = [&](float x, int sg) {
             if (g.use_f1) x = x / g.f1;
             if (g.use_f2) x = x + g.f2;
@@ -104,9 +111,16 @@ __global__ void __launch_bounds__(fft_threads(N)) k_rows(const float* __restrict
         };
         cplx<T> u[8];
 #pragma unroll
-        for (int r = 0; r < 8; r++) {
-            u[r].x = on ? field(xa[r], i + M * r) : T(0);
-            u[r].y = two ? field(xb[r], i + M * r + 1) : T(0);
+        for (int r = 0; r < PER; r++) {
+            u[r].x = s0 + pco < npair ? field(xa[r], pi + M * r) : T(0);
+            u[r].y = 2 * (s0 + pco) + 1 < ny ? field(xb[r], pi + M * r + 1) : T(0);
+        }
+        if constexpr (ONE) {
+            __syncthreads();  // the last batch's reads
+            sm[pco * F::Q::SEQ + lx(pi)] = u[0];
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < 8; r++) u[r] = on ? sm[co * F::Q::SEQ + lx(i + M * r)] : cplx<T>{T(0), T(0)};
         }
         if (bt + (int)gridDim.x < nbt) fetch(bt + gridDim.x);
         F::rows(u, sm, tw, -1, tid, false);

@@ -388,7 +388,7 @@ int launch_3d(utr_ctx* c, const cplx<T>* d_V, cplx<T>* d_H, TO* d_vol, const cpl
     bool ok = false;
 #define UTR_PZ(N)                                                                               \
     {                                                                                           \
-        using F = utr::Fft<N, T>;                                                               \
+        using F = utr::Fft<N, T, utr::vol_threads(N)>;                                          \
         const int gx = (W + F::NB - 1) / F::NB;                                                 \
         utr::k_pack_z<T, N><<<utr::xcd_grid(gx * g.ny), F::NT, 0, c->stream>>>(d_V, d_H, g, twz, \
                                                                              gx, g.ny);         \
@@ -400,7 +400,7 @@ int launch_3d(utr_ctx* c, const cplx<T>* d_V, cplx<T>* d_H, TO* d_vol, const cpl
     ok = false;
 #define UTR_FY(N)                                                                               \
     {                                                                                           \
-        using F = utr::Fft<N, T>;                                                               \
+        using F = utr::Fft<N, T, utr::vol_threads(N)>;                                          \
         const int gx = (W + F::NB - 1) / F::NB;                                                 \
         utr::k_fft_y<T, N><<<utr::xcd_grid(gx * g.nz), F::NT, 0, c->stream>>>(d_H, g, twy, gx,  \
                                                                             g.nz);              \
@@ -412,7 +412,7 @@ int launch_3d(utr_ctx* c, const cplx<T>* d_V, cplx<T>* d_H, TO* d_vol, const cpl
     ok = false;
 #define UTR_CX(N)                                                                               \
     {                                                                                           \
-        using F = utr::Fft<N, T>;                                                               \
+        using F = utr::Fft<N, T, utr::vol_threads(N)>;                                          \
         const int gx = (g.ny / 2 + F::NB - 1) / F::NB;                                          \
         utr::k_c2r_x<T, N, TO><<<utr::xcd_grid(gx * g.nz), F::NT, 0, c->stream>>>(d_H, d_vol, g, \
                                                                                twx, gx, g.nz);  \

@@ -341,9 +341,9 @@ __device__ __forceinline__ void fft_reg(cplx<T>* u, cplx<T>* __restrict__ sm, co
 
 // The transform of columns (neighbouring lanes on neighbouring sequences) or of
 // rows (on neighbouring elements), in place.
-template <int N, typename T = float>
+template <int N, typename T = float, int NT_ = fft_threads(N)>
 struct Fft {
-    static constexpr int NT = fft_threads(N);
+    static constexpr int NT = NT_;
     using Q = FftReg<N, NT>;
     static constexpr int NB = Q::NB, M = Q::M, LDS = Q::LDS;
     // workgroups a CU holds at most, by threads and by LDS

@@ -1659,7 +1659,11 @@ __global__ void __launch_bounds__(256) k_normalize(cplx<T>* __restrict__ V,
 
 // ------------------------------------------------------ 3D inverse FFT
 
-constexpr int CW_MAX = 16;
+// Threads of a workgroup: 8 sequences from 64 on (fft_threads: up to 256
+// threads).  The passes share nothing between sequences, so more workgroups
+// cost nothing, and a small volume has few: k_pack_z of 64^3 6.6 -> 5.6 us, of
+// 128^3 9.6 -> 8.8, k_fft_y 3.9 -> 3.3 and 6.8 -> 6.2; 192^3 and above the same.
+__host__ __device__ constexpr int vol_threads(int n) { return n >= 64 ? n : n == 48 ? 96 : 64; }
 
 // Row stride of the half spectrum H: nx/2 + 1 entries rounded up to 8, so
 // that every row starts on a 64-byte boundary and the column segments the 3D
@@ -1676,10 +1680,10 @@ __host__ __device__ constexpr int h_stride(int nx) { return (nx / 2 + 1 + 7) & ~
 // registers (Fft), 256^3 (202 MB): 50.9 us, against 61 through LDS; 512^3: 482
 // against 651.
 template <typename T, int NZ>
-__global__ void __launch_bounds__(fft_threads(NZ)) k_pack_z(const cplx<T>* __restrict__ V,
+__global__ void __launch_bounds__(vol_threads(NZ)) k_pack_z(const cplx<T>* __restrict__ V,
                                                 cplx<T>* __restrict__ H, GeomDev g,
                                                 const cplx<T>* __restrict__ tw, int gx, int gy) {
-    using F = Fft<NZ, T>;
+    using F = Fft<NZ, T, vol_threads(NZ)>;
     constexpr int M = F::M;
     __shared__ cplx<T> sm[F::LDS];
     const int nx = g.nx, ny = g.ny, W = nx / 2 + 1, WP = h_stride(nx);
@@ -1725,9 +1729,9 @@ __global__ void __launch_bounds__(fft_threads(NZ)) k_pack_z(const cplx<T>* __res
 // Inverse FFT along y of the half spectrum, in place.  256^3 (136 MB): 27.5 us
 // through registers (Fft), 36 through LDS; 512^3: 220 against 411.
 template <typename T, int NY>
-__global__ void __launch_bounds__(fft_threads(NY)) k_fft_y(cplx<T>* __restrict__ H, GeomDev g,
+__global__ void __launch_bounds__(vol_threads(NY)) k_fft_y(cplx<T>* __restrict__ H, GeomDev g,
                                                const cplx<T>* __restrict__ tw, int gx, int gy) {
-    using F = Fft<NY, T>;
+    using F = Fft<NY, T, vol_threads(NY)>;
     constexpr int M = F::M;
     __shared__ cplx<T> sm[F::LDS];
     const int W = g.nx / 2 + 1, WP = h_stride(g.nx);
@@ -1750,10 +1754,10 @@ __global__ void __launch_bounds__(fft_threads(NY)) k_fft_y(cplx<T>* __restrict__
 // scale (UTR.cpp:1235-1279).  256^3 (135 MB): 35.7 us through registers (Fft),
 // 43 through LDS; 512^3: 305 against 362.
 template <typename T, int NX, typename TO>
-__global__ void __launch_bounds__(fft_threads(NX)) k_c2r_x(const cplx<T>* __restrict__ H,
+__global__ void __launch_bounds__(vol_threads(NX)) k_c2r_x(const cplx<T>* __restrict__ H,
                                                TO* __restrict__ vol, GeomDev g,
                                                const cplx<T>* __restrict__ tw, int gx, int gy) {
-    using F = Fft<NX, T>;
+    using F = Fft<NX, T, vol_threads(NX)>;
     constexpr int NB = F::NB, M = F::M;
     __shared__ cplx<T> sm[F::LDS];
     __shared__ double s_ex[NX], s_ey[2 * NB];

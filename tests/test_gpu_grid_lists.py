@@ -40,3 +40,37 @@ def test_brick_gridding_point_lists(name):
     got = U.reconstruct(p, r, imgs)
     ref = oracle.reconstruct(p, r, imgs)
     assert rel(got, ref) < TOL
+
+
+@pytest.mark.parametrize("n,extra", [(32, 0), (48, 0), (32, 40), (32, 400)])
+def test_brick_gridding_tiny_weights(n, extra, monkeypatch):
+    """Rows on and a millionth of a voxel beside the grid planes, with and
+    without rotation about Z, alone (more points with tiny corners than a
+    brick's record holds) and under many random rows (voxels that have larger
+    weights as well): the sampled voxels are the oracle's, and V3/Samp3 keeps
+    its precision where only tiny weights fall (no noise filter: such voxels
+    count in the volume as any other)."""
+    monkeypatch.setenv("UTR_GRID_FORM", "brick")
+    rng = np.random.default_rng(n + extra)
+    angZ = np.concatenate([[0.0, 0.0, 0.0, 90.0, 1e-6, 90.000001, 45.0, 1e-6], rng.uniform(0, 360, extra)])
+    angY = np.concatenate([[0.0, 90.0, 89.999999, 0.0, 0.0, 90.0, 89.999999, 180.000002],
+                           np.degrees(np.arccos(rng.uniform(-1, 1, extra)))])
+    rows = len(angZ)
+    print("tiny weights", n, rows, flush=True)
+    xst = 0.4
+    p = U.default_params(nx=n, ny=n, xst=xst, zlo=-n * xst / 2, zhi=n * xst / 2, escc=0, nsr=0.0)
+    r = dict(angZ=angZ, angY=angY, defocus=np.full(rows, 300.0))
+    xyz, Z = synth.atoms(4, 20, "cube", n * xst * 0.4, 1.0, ([6], [1.0]))
+    imgs = synth.project(xyz, Z, n, n, xst, angZ, angY, dose=400.0, seed=4)
+    ref, S = oracle.reconstruct(p, r, imgs, samp=True)
+    if extra < 400:
+        assert ((S > 0) & (S < 2.0 ** -20)).sum() > 100
+    with U.Reconstructor(p, r) as rec:
+        rec.keep_sampling()
+        rec.add_images(imgs)
+        got = rec.finalize()
+        S32 = rec.sampling()
+    assert np.array_equal(S32 == 0, S == 0)
+    low = (S > 0) & (S < 2.0 ** -20)
+    assert np.abs(S32[low] / S[low] - 1.0).max(initial=0.0) < 1e-4
+    assert rel(got, ref) < TOL

@@ -721,23 +721,25 @@ __global__ void __launch_bounds__(256) k_gather(const cplx<float>* __restrict__ 
 // component and the row count so that no sum can overflow: V3 is resolved to
 // about 1e-11 (in units of K), Samp3 to about 1e-15.  A one-cell halo takes
 // the corners outside the brick, so corners need no bounds tests.
-// Weights below 2^-20 (rare: cells crossed within a millionth of a grid
-// plane, mostly at exact grid alignments) stay out of the fixed-point sums,
-// so a voxel reached only by such weights keeps the relative precision that
-// V3/Samp3 needs there and counts as sampled exactly as in the reference:
-// their points are recorded, the sums converted to FP64 in place and just
-// those corners' FP32 terms added in FP64 (in a second pass over all points
-// when more were met than the record holds).  Corners of weight exactly zero
-// add nothing.
+// A voxel reached only by weights below 2^-20 (cells crossed within a
+// millionth of a grid plane, mostly at exact grid alignments) needs the
+// relative precision of its V3/Samp3 and counts as sampled exactly as in the
+// reference: points with such a corner where the weights so far sum to less
+// than 2^-20 are recorded, and at the end the voxels still below it take
+// those corners' FP32 terms, added in FP64, instead of their fixed-point sums
+// (in a second pass over all points when more were met than the record
+// holds).  About three points a row have a tiny corner in a central brick;
+// recording all of them took the densest bricks of more than about 100 random
+// rows through the second pass: 720 of 48^2 into 48^3 744 us against 459, 300 of
+// 128^2 286 against 195 (a line per lane, before the lists: 629 and 347).
+// Corners of weight exactly zero add nothing.
 //
 // The strides are odd (17 along y, 153 along z) so that points along x, y or
 // z address distinct LDS banks.  Bricks start from the volume's centre
 // outwards: every row's sheet passes it, so the central bricks hold 25 times
 // the points of an average one and would set the tail.
-// Of 553 us for 216 random rows of 256^2 into 256^3 (764 us before), the
-// points take about 230, listing the lines 180 (latency of a few rounds a
-// brick), zeroing, row tests and the V3 write 112, the CTF epilogue 70.  One
-// row per wave without barriers (rows in scalar registers) measured 523 us
+// 216 random rows of 256^2 into 256^3 take 548 us (764 with a line per lane).
+// One row per wave without barriers (rows in scalar registers) measured 523 us
 // there but 192 against 118 us for 108 rows of 192 x 160 into 192 x 160 x 96,
 // where a brick has fewer rows than waves.
 
@@ -811,14 +813,14 @@ __global__ void __launch_bounds__(256, ROT ? 2 : 3) k_grid_fx(const cplx<float>*
     __shared__ float s_red[4];
     __shared__ int s_list[S_LIST];     // rows reaching the brick, in row order
     __shared__ int s_lo[S_LIST];       // first detector line of each listed row
-    __shared__ int s_pre[S_LIST + 1];  // line counts, then their exclusive prefix
+    __shared__ int s_pre[S_LIST];      // exclusive prefix of their line counts
     __shared__ int s_cnt[4], s_wsum[4];
-    __shared__ int s_n;
     __shared__ int2 s_line[2][256];                  // row; b << 16 | (a - point number) & 0xffff
     __shared__ unsigned char s_pt[2][S_POINTS];      // line of each listed point
     __shared__ int s_tot[3];                         // points of a round
     __shared__ int2 s_tq[S_TQ];                      // points with a corner weight below 2^-20 (row; b << 16 | a)
     __shared__ int s_tn;                             // their count (may exceed S_TQ)
+    __shared__ unsigned s_only[SVOX / 32];           // voxels whose weights sum to less than 2^-20
     double* const accd = reinterpret_cast<double*>(acc);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -846,6 +848,7 @@ __global__ void __launch_bounds__(256, ROT ? 2 : 3) k_grid_fx(const cplx<float>*
     const int sw = min(61 - ea, 50);
     const double vscale = ldexp(1.0, sv), wscale = ldexp(1.0, sw);
     const double vinv = ldexp(1.0, -sv), winv = ldexp(1.0, -sw);
+    const unsigned long long low = 1ull << (sw - 20);
 
     const float fx2 = (float)(g.fxst * g.fxst), fy2 = (float)(g.fyst * g.fyst);
     const float wl2f = (float)g.wl2;
@@ -858,9 +861,9 @@ __global__ void __launch_bounds__(256, ROT ? 2 : 3) k_grid_fx(const cplx<float>*
     const float cgrid[3] = {(float)g.nxd2, (float)g.nyd2, (float)g.nzd2};
 
     // One point (a, b) of row r.  FIX false: the fixed-point terms of every
-    // corner of weight >= 2^-20, and the point recorded when a smaller nonzero
-    // one is in the brick.  FIX true: only those small corners, their FP32
-    // terms added in FP64 to the converted sums.
+    // corner, and the point recorded when one of weight below 2^-20 falls on a
+    // voxel of the brick that has no more yet.  FIX true: only such corners on
+    // voxels that stayed below (s_only), their FP32 terms added in FP64.
     struct Point {
         int r, a, b;
         cplx<float> k;
@@ -908,26 +911,29 @@ __global__ void __launch_bounds__(256, ROT ? 2 : 3) k_grid_fx(const cplx<float>*
 #pragma unroll
         for (int c = 0; c < 8; c++) wds[c] = wxs[c & 1] * wys[(c >> 1) & 1] * wzs[c >> 2];
         if (near) {
-            bool any_tiny = false;
+            bool record = false;
 #pragma unroll
             for (int c = 0; c < 8; c++) {
                 const bool tny = wds[c] != 0.0 && wds[c] < S_TINY_D;
                 const bool inb = (unsigned)(ii + (c & 1)) < (unsigned)SBX &&
                                  (unsigned)(jj + ((c >> 1) & 1)) < (unsigned)SBY &&
                                  (unsigned)(nn + (c >> 2)) < (unsigned)SBZ;
+                if (!(tny && inb)) continue;
+                const int li = li0 + (c & 1) + SPY * ((c >> 1) & 1) + SPZ * (c >> 2);
                 if (FIX) {
-                    if (!(tny && inb)) continue;
-                    const int li = li0 + (c & 1) + SPY * ((c >> 1) & 1) + SPZ * (c >> 2);
+                    const int v = (ii + (c & 1)) + SBX * ((jj + ((c >> 1) & 1)) + SBY * (nn + (c >> 2)));
+                    if (!(s_only[v >> 5] >> (v & 31) & 1u)) continue;
                     const float w = (float)wds[c];
                     atomicAdd(&accd[li], (double)(w * kv.x));
                     atomicAdd(&accd[SPAD + li], (double)(w * kv.y));
                     atomicAdd(&accd[2 * SPAD + li], (double)w);
                 } else {
-                    any_tiny |= tny && inb;
-                    if (tny) wds[c] = 0.0;
+                    // sums of weights only grow: what is below at the end is below now
+                    record |= __hip_atomic_load(&acc[2 * SPAD + li], __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_WORKGROUP) < low;
                 }
             }
-            if (!FIX && any_tiny) {
+            if (!FIX && record) {
                 const int slot = atomicAdd(&s_tn, 1);
                 if (slot < S_TQ) s_tq[slot] = int2{r, (int)((unsigned)b << 16 | ((unsigned)a & 0xffffu))};
             }
@@ -936,13 +942,14 @@ __global__ void __launch_bounds__(256, ROT ? 2 : 3) k_grid_fx(const cplx<float>*
         // the spectrum value on the V3 fixed-point grid (exact: a power of two)
         const double kxs = (double)kv.x * vscale, kys = (double)kv.y * vscale;
         unsigned long long* A = acc + li0;
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
+        auto corner = [&](int c) {
             const int li = (c & 1) + SPY * ((c >> 1) & 1) + SPZ * (c >> 2);
             atomicAdd(&A[li], (unsigned long long)fx_term(wds[c], kxs));
             atomicAdd(&A[SPAD + li], (unsigned long long)fx_term(wds[c], kys));
             atomicAdd(&A[2 * SPAD + li], (unsigned long long)fx_term(wds[c], wscale));
-        }
+        };
+#pragma unroll
+        for (int c = 0; c < 8; c++) corner(c);
     };
 
     int round = 0;
@@ -1091,10 +1098,16 @@ __global__ void __launch_bounds__(256, ROT ? 2 : 3) k_grid_fx(const cplx<float>*
         for (int k = 0; k < SOWN; k++) {
             const int v = tid + 256 * k;
             const int li = lds_idx(v % SBX, (v / SBX) % SBY, v / (SBX * SBY));
+            const bool only = acc[2 * SPAD + li] < low;
+            const unsigned long long m = __ballot(only);
+            if (lane == 0) {
+                s_only[v >> 5] = (unsigned)m;
+                s_only[(v >> 5) + 1] = (unsigned)(m >> 32);
+            }
 #pragma unroll
             for (int c = 0; c < 3; c++) {
                 const double d = (double)(long long)acc[c * SPAD + li] * (c < 2 ? vinv : winv);
-                accd[c * SPAD + li] = d;
+                accd[c * SPAD + li] = only ? 0.0 : d;
             }
         }
         __syncthreads();

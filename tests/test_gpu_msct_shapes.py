@@ -53,3 +53,24 @@ def test_potential_of_narrow_rows(nx, ny, monkeypatch):
     got = U.multislice_images(dict(p, output=0, nwobble=1), at, *ang, [0.0])
     ref = M.images(dict(op, nwobble=1, temperature=300.0), at, np.radians(ang[0]), np.radians(ang[1]), [0.0])
     assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < 1e-5
+
+
+@pytest.mark.parametrize("nx,ny,na", [(384, 96, 24), (320, 128, 17), (512, 64, 33)])
+def test_long_lines_of_many_and_of_single_orientations(nx, ny, na):
+    """Products of long lines split over more workgroups where there are few
+    of them: the orientations together and one by one give the same bits."""
+    print("long lines", nx, ny, na, flush=True)
+    ctb = 19.2
+    p = U.default_msct_params(nx=nx, ny=ny, ctblength=ctb, deltaz=3.2, kev=200.0, output=2)
+    xyz, Z = synth.atoms(nx + ny, 12, "sphere", 5.0, 1.4)
+    at = dict(Z=Z, occ=np.ones(len(Z), np.float32),
+              **{k: (xyz[:, i] + ctb / 2).astype(np.float32) for i, k in enumerate("xyz")})
+    angZ, angY = np.linspace(0, 300, na), np.linspace(5, 170, na)
+    psi = U.multislice_images(p, at, angZ, angY, [100.0])
+    m = U.Multislice(p, at)
+    try:
+        for a in (0, na // 2, na - 1):
+            one = m.images(angZ[a:a + 1], angY[a:a + 1], [100.0])
+            assert np.array_equal(one[0].view(np.uint32), psi[a].view(np.uint32)), a
+    finally:
+        m.close()

@@ -413,11 +413,11 @@ __global__ void __launch_bounds__(Fft<N>::NT) k_ms_cols(const cplx<float>* __res
 // both, W * T where the slice holds atoms for this orientation, x FFT of the
 // product back into W (kept columns).  Projection (PROJ true): W is real-space;
 // inverse x FFT of T only and W *= T.
-template <int N, bool PROJ>
-__global__ void __launch_bounds__(Fft<N>::NT) k_ms_mul(cplx<float>* __restrict__ W, const cplx<float>* __restrict__ T,
+template <int N, bool PROJ, int NT>
+__global__ void __launch_bounds__(NT) k_ms_mul(cplx<float>* __restrict__ W, const cplx<float>* __restrict__ T,
                                                 int ny, int nlines, int lim, const cplx<float>* __restrict__ tw,
                                                 const int* __restrict__ off, int nsl1, int s) {
-    using F = Fft<N>;
+    using F = Fft<N, float, NT>;
     constexpr int M = F::M;
     __shared__ cplx<float> sm[F::LDS];
     const int tid = threadIdx.x, i = F::Q::row_i(tid), l = blockIdx.x * F::NB + F::Q::row_c(tid);
@@ -730,6 +730,13 @@ int ms_run_lines(msct_ctx* c, int what, int B, int s, int ndef, int d, float* ou
     const bool proj = c->p.mode != 0;
     bool ok = false;
     const int wlim = ms_wave_lim(c);
+    // k_ms_mul is three transforms in a row: where workgroups of eight long lines
+    // would be fewer than the compute units, two lines each (one image of 384^2:
+    // 8.3 -> 6.9 us a slice, of 512^2 7.5 -> 5.8)
+    constexpr unsigned kMsCus = 256;
+#define MS_MUL(N, PROJ, T_)                                                                         \
+    utr::k_ms_mul<N, PROJ, T_><<<(unsigned)((nlines + 8 * T_ / N - 1) / (8 * T_ / N)), T_, 0, st>>>( \
+        c->W.p, c->T.p, ny, nlines, c->lim, c->twx.p, c->off.p, c->g.nsl1, s)
 #define MS_LINES(N)                                                                                 \
     {                                                                                               \
         constexpr int NB = utr::Fft<N>::NB, NT = utr::Fft<N>::NT;                                   \
@@ -737,12 +744,13 @@ int ms_run_lines(msct_ctx* c, int what, int B, int s, int ndef, int d, float* ou
         if (what == 0) {                                                                            \
             utr::k_ms_lines<N><<<groups, NT, 0, st>>>(c->T.p, nlines, c->twx.p);                    \
         } else if (what == 1) {                                                                     \
+            constexpr int NQ = N >= 320 ? NT / 4 : NT;                                              \
             if (proj)                                                                               \
-                utr::k_ms_mul<N, true><<<groups, NT, 0, st>>>(c->W.p, c->T.p, ny, nlines, c->lim, c->twx.p, \
-                                                              c->off.p, c->g.nsl1, s);              \
+                MS_MUL(N, true, NT);                                                                \
+            else if (N >= 320 && groups < kMsCus)                                                   \
+                MS_MUL(N, false, NQ);                                                               \
             else                                                                                    \
-                utr::k_ms_mul<N, false><<<groups, NT, 0, st>>>(c->W.p, c->T.p, ny, nlines, c->lim, c->twx.p, \
-                                                               c->off.p, c->g.nsl1, s);             \
+                MS_MUL(N, false, NT);                                                               \
         } else if (what == 4) {                                                                     \
             constexpr int NR = utr::ms_pot_rows<N>();                                               \
             utr::k_ms_potential_rows<N><<<dim3((ny + NR - 1) / NR, B), NT, 0, st>>>(                \
@@ -760,6 +768,7 @@ int ms_run_lines(msct_ctx* c, int what, int B, int s, int ndef, int d, float* ou
     }
     UTR_DISPATCH_N(nx, MS_LINES)
 #undef MS_LINES
+#undef MS_MUL
     if (!ok) return set_err(UTR_E_UNSUPPORTED, "msct: unsupported image width for the FFT");
     UTR_HIP_TRY(hipGetLastError());
     return UTR_OK;

@@ -487,11 +487,13 @@ int msct_images_device(msct_ctx* ctx, int nang, const double* angZ_rad, const do
 /* Slices per orientation: k * deltaz for k = 1, 2, ... while below the cube
  * side + deltaz (autoslic.cpp:727-744). */
 int msct_slices(const msct_ctx* ctx);
-/* Orientations simulated together per batch: as many as fit the
- * UTR_MSCT_BATCH_BYTES budget (default 6 GiB) of device memory held per
- * orientation (three complex planes, the rotated atom records and the slice
- * table).  No counterpart in the reference (it runs one orientation at a
- * time per thread, MultisliceT.cpp:398-450). */
+/* Most orientations simulated together: as many as keep their wave and
+ * transmission planes within 200 MiB (they stay in the memory-side cache) and
+ * everything held per orientation (three complex planes, the rotated atom
+ * records and the slice table) within 6 GiB, or, where UTR_MSCT_BATCH_BYTES is
+ * set, as many as fit that budget.  More orientations run in passes of equal
+ * size.  No counterpart in the reference (it runs one orientation at a time per
+ * thread, MultisliceT.cpp:398-450). */
 int msct_batch(const msct_ctx* ctx);
 int msct_destroy(msct_ctx* ctx);
 

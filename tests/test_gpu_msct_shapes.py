@@ -74,3 +74,29 @@ def test_long_lines_of_many_and_of_single_orientations(nx, ny, na):
             assert np.array_equal(one[0].view(np.uint32), psi[a].view(np.uint32)), a
     finally:
         m.close()
+
+
+def test_batch_is_what_a_pass_takes(monkeypatch):
+    """By default a pass holds at most 200 MiB of wave and transmission planes;
+    a set budget rules alone, in either direction; the images do not depend on
+    it."""
+    monkeypatch.delenv("UTR_MSCT_BATCH_BYTES", raising=False)
+    p = U.default_msct_params(nx=512, ny=256, ctblength=38.4, deltaz=12.8, kev=200.0)
+    at = dict(Z=np.array([6, 8], np.int32), x=np.array([15.0, 20.0], np.float32), y=np.array([17.0, 20.0], np.float32),
+              z=np.array([10.0, 25.0], np.float32))
+    plane = 512 * 256 * 8
+    ang = np.linspace(0.0, 200.0, 5), np.linspace(10.0, 150.0, 5)
+    per = None
+    for budget in (None, 1 << 30, 2 * 10 ** 7):
+        if budget:
+            monkeypatch.setenv("UTR_MSCT_BATCH_BYTES", str(budget))
+        m = U.Multislice(p, at)
+        try:
+            print("batch", budget, m.batch, flush=True)
+            want = budget // (3 * plane + 2 * 32 + (m.slices + 1) * 8) if budget else (200 << 20) // (2 * plane)
+            assert m.batch == want
+            img = m.images(*ang, [0.0])
+        finally:
+            m.close()
+        assert per is None or np.array_equal(per, img)
+        per = img

@@ -754,7 +754,7 @@ class Multislice:
 
     @property
     def batch(self):
-        """Orientations simulated together (the UTR_MSCT_BATCH_BYTES budget)."""
+        """Most orientations simulated together (msct_batch)."""
         return self._L.msct_batch(self._ctx)
 
     def images(self, angZ_deg, angY_deg, defocus, out=None):

@@ -930,12 +930,8 @@ int ms_images(msct_ctx* c, int nang, const double* angZ, const double* angY, int
     const int nx = c->g.nx, ny = c->g.ny;
     const size_t plane = (size_t)nx * ny;
     const size_t per_img = plane * (c->p.output == 2 ? 2 : 1);
-    // orientations taken together: those of the budget, in equal batches whose
-    // wave and transmission planes stay in the 256 MB memory-side cache between
-    // the passes of a slice (360 of 256^2 in two batches 46.1 ms, in one 56.4, in
-    // three 49.3: below about 10^7 pixels a pass the launches show)
-    const int fit = (int)std::max<size_t>(1, (size_t(200) << 20) / (2 * plane * sizeof(cplx<float>)));
-    const int most = std::min(c->batch, fit), groups = (nang + most - 1) / most;
+    // orientations taken together: at most c->batch, in passes of equal size
+    const int groups = (nang + c->batch - 1) / c->batch;
     const int B = (nang + groups - 1) / groups;
     UTR_HIP_TRY(c->W.alloc(plane * B));
     UTR_HIP_TRY(c->T.alloc(plane * B));
@@ -1200,11 +1196,18 @@ int msct_create(const msct_params* p, const double* fe_params, int natom, const 
         (e = up(c->twy, make_twiddles<float>(ny))) != hipSuccess)
         return fail(set_err(e == hipErrorOutOfMemory ? UTR_E_NOMEM : UTR_E_DEVICE,
                             std::string("msct_create: upload failed: ") + hipGetErrorString(e)));
-    // orientations per batch: UTR_MSCT_BATCH_BYTES caps the device memory of
-    // everything held per orientation of a batch
-    size_t budget = (size_t)6 << 30;
-    if (const char* s = std::getenv("UTR_MSCT_BATCH_BYTES")) budget = std::max<size_t>(1, std::strtoull(s, nullptr, 10));
-    c->batch = ms_batch_size(nx, ny, natom, c->nsl, budget);
+    // orientations of a pass: those whose wave and transmission planes stay in the
+    // 256 MB memory-side cache between the passes of a slice (360 of 256^2 in two
+    // passes 46.1 ms, in one 56.4, in three 49.3: below about 10^7 pixels a pass
+    // the launches show), or UTR_MSCT_BATCH_BYTES of device memory for everything
+    // held per orientation
+    const char* bytes = std::getenv("UTR_MSCT_BATCH_BYTES");
+    c->batch = ms_batch_size(nx, ny, natom, c->nsl,
+                             bytes ? std::max<size_t>(1, std::strtoull(bytes, nullptr, 10)) : (size_t)6 << 30);
+    if (!bytes) {
+        const size_t two = 2 * (size_t)nx * ny * sizeof(cplx<float>);
+        c->batch = (int)std::min<size_t>(c->batch, std::max<size_t>(1, ((size_t)200 << 20) / two));
+    }
     *out = c;
     return UTR_OK;
 }

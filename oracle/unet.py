@@ -146,23 +146,27 @@ def loss_and_grad(theta, vol, tgt, tile, halo, scale=1.0, bf=True):
     gd1b = r(g[..., None] * w1 * pos(c["d1b"]))
     dhead = np.concatenate([np.tensordot(g, c["d1b"], axes=4), [g.sum(), np.sum(g * c["x0f"])]])
 
-    def back(i, x, dy, mask):
+    def back(i, x, dy, mask, up=0):
+        # the gradient of the first `up` channels (an upsampled tensor's) is
+        # summed over its voxels before it is stored, and so rounded only there
         dx, dW, db = conv_back(x, Ws[i][0], dy)
         grads[i] = (dW, db)
-        return r(dx * pos(mask)) if mask is not None else r(dx)
+        if mask is not None:
+            dx = dx * pos(mask)
+        return (dx[..., :up], r(dx[..., up:])) if up else r(dx)
 
     gd1a = back(9, c["d1a"], gd1b, c["d1a"])
-    gC1 = back(8, c["C1"], gd1a, c["C1"])
-    gd2b = r(up_back(gC1[..., :32]))
+    gup, gskip1 = back(8, c["C1"], gd1a, c["C1"], 32)
+    gd2b = r(up_back(gup))
     gd2a = back(7, c["d2a"], gd2b, c["d2a"])
-    gC2 = back(6, c["C2"], gd2a, c["C2"])
-    ge3b = r(up_back(gC2[..., :64]))
+    gup, gskip2 = back(6, c["C2"], gd2a, c["C2"], 64)
+    ge3b = r(up_back(gup))
     ge3a = back(5, c["e3a"], ge3b, c["e3a"])
     gp2 = back(4, c["p2"], ge3a, None)
-    ge2b = r((gC2[..., 64:] + pool_back(gp2)) * pos(c["C2"][..., 64:]))
+    ge2b = r((gskip2 + pool_back(gp2)) * pos(c["C2"][..., 64:]))
     ge2a = back(3, c["e2a"], ge2b, c["e2a"])
     gp1 = back(2, c["p1"], ge2a, None)
-    ge1b = r((gC1[..., 32:] + pool_back(gp1)) * pos(c["C1"][..., 32:]))
+    ge1b = r((gskip1 + pool_back(gp1)) * pos(c["C1"][..., 32:]))
     ge1a = back(1, c["e1a"], ge1b, c["e1a"])
     _, dW0, db0 = conv_back(c["x0"], Ws[0][0], ge1a)
     grads[0] = (dW0, db0)

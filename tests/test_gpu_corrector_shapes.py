@@ -23,6 +23,16 @@ def rel(a, b):
     return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
 
 
+def assert_layers(g, rg):
+    off = 0
+    for ci, co in N.LAYERS:
+        nw = 27 * ci * co
+        assert rel(g[off:off + nw], rg[off:off + nw]) <= 2e-2, (ci, co)
+        assert rel(g[off + nw:off + nw + co], rg[off + nw:off + nw + co]) <= 2e-2, (ci, co)
+        off += nw + co
+    assert rel(g[off:], rg[off:]) <= 2e-2
+
+
 @pytest.mark.parametrize("tile,halo,batch,nb", [(8, 0, 1, 1), (4, 4, 2, 2), (4, 8, 3, 2), (12, 4, 1, 1), (24, 2, 2, 1),
                                                 (20, 8, 1, 1)])
 def test_forward_and_gradient_at_block_edges(tile, halo, batch, nb):
@@ -47,13 +57,7 @@ def test_forward_and_gradient_at_block_edges(tile, halo, batch, nb):
         c.close()
     rloss, rg = N.loss_and_grad(theta.astype(np.float64), vol, tgt, tile, halo, SCALE, bf=True)
     assert abs(loss - rloss) <= 1e-3 * rloss
-    off = 0
-    for ci, co in N.LAYERS:
-        nw = 27 * ci * co
-        assert rel(g[off:off + nw], rg[off:off + nw]) <= 2e-2, (ci, co)
-        assert rel(g[off + nw:off + nw + co], rg[off + nw:off + nw + co]) <= 2e-2, (ci, co)
-        off += nw + co
-    assert rel(g[off:], rg[off:]) <= 2e-2
+    assert_layers(g, rg)
 
 
 @pytest.mark.parametrize("tile,halo,batch,shape", [(8, 4, 3, (17, 8, 11)), (12, 2, 2, (5, 30, 13)), (20, 0, 1, (20, 7, 33))])
@@ -83,3 +87,110 @@ def test_apply_ragged_volumes(tile, halo, batch, shape):
         o = N.forward(theta.astype(np.float64), crop[None], SCALE, bf=True)[0][0] / SCALE
         ref[a[0]:a[0] + tile, a[1]:a[1] + tile, a[2]:a[2] + tile] = o[halo:halo + tile, halo:halo + tile, halo:halo + tile]
     assert rel(got, ref[:shape[0], :shape[1], :shape[2]]) <= 1e-2
+
+
+@pytest.fixture
+def gpu_convolutions(monkeypatch):
+    """The oracle's convolutions by torch in FP64 on the GPU, for crops whose
+    products take minutes on the CPU."""
+    import torch
+
+    def dev(a):
+        return torch.from_numpy(np.ascontiguousarray(a, np.float64)).cuda()
+
+    def taps(x):
+        D, H, W = x.shape[1:4]
+        p = torch.nn.functional.pad(x, (0, 0, 1, 1, 1, 1, 1, 1))
+        for t in range(27):
+            z, y, w = t // 9, t // 3 % 3, t % 3
+            yield t, p[:, z:z + D, y:y + H, w:w + W].reshape(-1, x.shape[4])
+
+    def conv(x, W, b=None):
+        out = torch.zeros((int(np.prod(x.shape[:4])), W.shape[2]), dtype=torch.float64, device="cuda")
+        Wd = dev(W)
+        for t, v in taps(dev(x)):
+            out.addmm_(v, Wd[t])
+        out = out.cpu().numpy().reshape(x.shape[:4] + (W.shape[2],))
+        return out if b is None else out + b
+
+    def conv_back(x, W, dy):
+        Wd, g = dev(W), dev(dy)
+        flat = g.reshape(-1, g.shape[4])
+        dW = torch.stack([v.T.contiguous() @ flat for _, v in taps(dev(x))])
+        dx = torch.zeros((flat.shape[0], x.shape[4]), dtype=torch.float64, device="cuda")
+        for t, v in taps(g):
+            dx.addmm_(v, Wd[26 - t].T.contiguous())
+        return dx.cpu().numpy().reshape(x.shape), dW.cpu().numpy(), flat.sum(0).cpu().numpy()
+
+    monkeypatch.setattr(N, "conv", conv)
+    monkeypatch.setattr(N, "conv_back", conv_back)
+
+
+def blocks(n, e):
+    """Blocks of 16 x 8 x 4 voxels of n cubes of edge e: the work-groups of a
+    convolution's larger form, which takes over from 512 of them, and the steps
+    that at most 768 weight-gradient work-groups share."""
+    return n * -(-e // 16) * -(-e // 8) * -(-e // 4)
+
+
+def test_large_batch_forward_and_gradient(gpu_convolutions):
+    """A training batch as large as real ones: the two finer levels take the
+    larger convolution form, with a remainder along every axis, and every
+    work-group of the finer weight gradients several voxel blocks."""
+    import torch
+    tile, halo, nb = 72, 2, 4
+    T = tile + 2 * halo
+    for e in (T, T // 2):
+        assert blocks(nb, e) >= 512 and e % 16 and e % 8 and (e == T or e % 4)
+    assert blocks(nb, tile) > 2 * 768
+    rng = np.random.default_rng(11)
+    theta = N.init(11, scale_head=0.3).astype(np.float32)
+    vol = rng.normal(0, 1, (nb, T, T, T)).astype(np.float32)
+    tgt = (0.5 * vol + rng.normal(0, 0.5, vol.shape)).astype(np.float32)
+    c = U.Corrector(tile=tile, halo=halo, batch=nb, seed=5)
+    try:
+        c.set_params(theta, SCALE)
+        dv, dt = torch.from_numpy(vol).cuda(), torch.from_numpy(tgt).cuda()
+        out = torch.empty_like(dv)
+        c.forward(dv, out)
+        loss, g = c.gradient(dv, dt)
+    finally:
+        c.close()
+    print("large batch: gradient done", flush=True)
+    ref = N.forward(theta.astype(np.float64), vol, SCALE, bf=True)[0] / SCALE
+    print("large batch: output rel-L2 %.2e" % rel(out.cpu().numpy(), ref), flush=True)
+    assert rel(out.cpu().numpy(), ref) <= 1e-2
+    rloss, rg = N.loss_and_grad(theta.astype(np.float64), vol, tgt, tile, halo, SCALE, bf=True)
+    print("large batch: loss %.6f, oracle %.6f, gradient rel-L2 %.2e" % (loss, rloss, rel(g, rg)), flush=True)
+    assert abs(loss - rloss) <= 1e-3 * rloss
+    assert_layers(g, rg)
+
+
+def test_apply_four_tiles_of_64(gpu_convolutions):
+    """Inference with the default tile, halo and batch: four crops of 80^3 in
+    one pass, the larger convolution form on the finer levels."""
+    import torch
+    tile, halo, shape = 64, 8, (70, 60, 128)
+    T = tile + 2 * halo
+    assert blocks(4, tile) >= 512 and blocks(4, 34) >= 512  # d1b, d2b
+    rng = np.random.default_rng(12)
+    theta = N.init(12, scale_head=0.3).astype(np.float32)
+    vol = rng.normal(0, 1, shape).astype(np.float32)
+    c = U.Corrector(tile=tile, halo=halo, batch=4, seed=5)
+    try:
+        c.set_params(theta, SCALE)
+        dv = torch.from_numpy(vol).cuda()
+        out = torch.full_like(dv, float("nan"))
+        c.apply(dv, out)
+        got = out.cpu().numpy()
+    finally:
+        c.close()
+    pad = np.zeros((2 * tile + 2 * halo, tile + 2 * halo, 2 * tile + 2 * halo))
+    pad[halo:halo + 70, halo:halo + 60, halo:halo + 128] = vol
+    ref = np.zeros((2 * tile, tile, 2 * tile))
+    for k, i in np.ndindex(2, 2):
+        a, b = k * tile, i * tile
+        o = N.forward(theta.astype(np.float64), pad[None, a:a + T, :, b:b + T], SCALE, bf=True)[0][0] / SCALE
+        ref[a:a + tile, :, b:b + tile] = o[halo:halo + tile, halo:halo + tile, halo:halo + tile]
+        print("apply: tile", k, i, flush=True)
+    assert rel(got, ref[:70, :60]) <= 1e-2

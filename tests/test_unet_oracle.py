@@ -88,3 +88,47 @@ def test_adam_first_step_is_signed_lr():
     t, m, v = N.adam(th, g, np.zeros(3), np.zeros(3), 1, 1e-2)
     # first step: m_hat / sqrt(v_hat) = sign(g)
     assert np.allclose(t, th - 1e-2 * np.sign(g), atol=1e-9)
+
+
+def test_conv_flops_counts_the_voxels_formed():
+    """conv_flops against the voxels a brute-force walk through the network
+    needs: all of them without a halo, and with one at least those and at most a
+    voxel more per side of a layer (cubes are made even where voxels pair)."""
+    from utr_public_amd import corrector as C
+
+    def dilate(m):
+        p = np.pad(m, 1)
+        for ax in range(3):
+            p = p | np.roll(p, 1, ax) | np.roll(p, -1, ax)
+        return p[1:-1, 1:-1, 1:-1]
+
+    def coarse(m):
+        n = m.shape[0] // 2
+        return m.reshape(n, 2, n, 2, n, 2).any(axis=(1, 3, 5))
+
+    def fine(m):
+        return m.repeat(2, 0).repeat(2, 1).repeat(2, 2)
+    per = [2.0 * 27 * (1 if k == 0 else ci) * co for k, (ci, co, _) in enumerate(C.LAYERS)]
+    for T, h in ((24, 0), (24, 4), (80, 8), (40, 3)):
+        d1b = np.zeros((T, T, T), bool)
+        d1b[h:T - h, h:T - h, h:T - h] = True
+        d1a = dilate(d1b)
+        c1 = dilate(d1a)
+        d2b = coarse(c1)
+        d2a = dilate(d2b)
+        c2 = dilate(d2a)
+        e3b = coarse(c2)
+        e3a = dilate(e3b)
+        e2b = c2 | fine(dilate(e3a))
+        e2a = dilate(e2b)
+        e1b = c1 | fine(dilate(e2a))
+        need = [dilate(e1b), e1b, e2a, e2b, e3a, e3b, d2a, d2b, d1a, d1b]
+        got = [q for q, _ in C.conv_cubes(T, h)]
+        edge = [round(m.sum() ** (1 / 3)) for m in need]
+        assert all(e <= q <= e + 2 for e, q in zip(edge, got)), (T, h, edge, got)
+        if h == 0:
+            assert got == edge
+        fwd, trn = C.conv_flops(T, h)
+        assert fwd == sum(p * q ** 3 for p, q in zip(per, got)) and 2 * fwd < trn < 3 * fwd * 1.2
+    # one 80^3 crop with an 8-voxel halo: 71 % of the whole crop's operations
+    assert abs(C.conv_flops(80, 8)[0] / C.conv_flops(80)[0] - 0.71) < 0.02

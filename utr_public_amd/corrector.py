@@ -262,13 +262,48 @@ LAYERS = [(16, 16, 1), (16, 16, 1), (16, 32, 2), (32, 32, 2), (32, 64, 3), (64, 
           (48, 16, 1), (16, 16, 1)]
 
 
-def conv_flops(T):
-    """(forward, training step) matrix-core FLOPs of one T^3 crop: 2 * 27 *
-    cin * cout per output voxel and layer forward; training adds the weight
-    gradients (the same count) and the input gradients (the same, except the
-    first layer's)."""
-    fwd = [2.0 * 27 * ci * co * (T // (1 << (lv - 1))) ** 3 for ci, co, lv in LAYERS]
-    return sum(fwd), 3 * sum(fwd) - fwd[0]
+def conv_cubes(T, halo=0):
+    """Edges, per layer, of the cubes the convolutions form for T^3 crops whose
+    outputs count inside the halo: (of the layer's output, of its input
+    gradient).  Each cube is grown by a voxel per convolution behind it, halved
+    outwards at a coarser level and made even where voxels are pooled or
+    upsampled, as the library does."""
+    def grow(q, e):
+        return max(0, q[0] - 1), min(e, q[1] + 1)
+
+    def half(q):
+        return q[0] // 2, (q[1] + 1) // 2
+
+    def twice(q):
+        return 2 * q[0], 2 * q[1]
+
+    def both(a, b):
+        return min(a[0], b[0]), max(a[1], b[1])
+    d1b = halo, T - halo
+    d1a = grow(d1b, T)
+    d2b = half(grow(d1a, T))
+    d2a = grow(d2b, T // 2)
+    e3b = half(grow(d2a, T // 2))
+    e3a = grow(e3b, T // 4)
+    e2b = both(twice(e3b), twice(grow(e3a, T // 4)))
+    e2a = grow(e2b, T // 2)
+    e1b = both(twice(d2b), twice(grow(e2a, T // 2)))
+    e1a = grow(e1b, T)
+    out = e1a, e1b, e2a, e2b, e3a, e3b, d2a, d2b, d1a, d1b
+    grad = None, e1a, half(e1b), e2a, half(e2b), e3a, twice(e3b), d2a, twice(d2b), d1a
+    return [(q[1] - q[0], g[1] - g[0] if g else 0) for q, g in zip(out, grad)]
+
+
+def conv_flops(T, halo=0):
+    """(forward, training step) matrix-core FLOPs of one T^3 crop whose outputs
+    count inside the halo: 2 * 27 * cin * cout per voxel a layer forms (one input
+    channel for the first layer); training adds the weight gradients (the same
+    count) and the input gradients (2 * 27 * cin * cout per voxel formed, none
+    for the first layer)."""
+    per = [2.0 * 27 * (1 if k == 0 else ci) * co for k, (ci, co, _) in enumerate(LAYERS)]
+    cubes = conv_cubes(T, halo)
+    fwd = sum(p * q ** 3 for p, (q, _) in zip(per, cubes))
+    return fwd, 2 * fwd + sum(p * g ** 3 for p, (_, g) in zip(per, cubes))
 
 
 def run(name="c5", log=print, heldout=4, seed0=1000):
@@ -318,7 +353,7 @@ def run(name="c5", log=print, heldout=4, seed0=1000):
         torch.cuda.synchronize()
         out["infer_s"] = (time.time() - t1) / 3
         ntiles = -(-wl.n // cfg["tile"]) ** 3
-        fwd, trn = conv_flops(corr.T)
+        fwd, trn = conv_flops(corr.T, cfg["halo"])
         out["train_tflops"] = trn * cfg["batch"] * cfg["steps"] / out["train_s"] / 1e12
         out["infer_tflops"] = fwd * ntiles / out["infer_s"] / 1e12
     finally:

@@ -65,6 +65,23 @@ def test_batch_autotune():
         assert rel(o, oracle.reconstruct(p, rows, imgs)) < 1e-5
 
 
+def test_autotune_is_per_kind_of_job():
+    """A job of random orientations does not take the settings tuned for a tilt
+    series of its size (which may name planes per workgroup of a gridding it
+    does not use), nor the other way round."""
+    for n, rows in ((32, 17), (48, 19), (64, 21), (96, 23)):
+        p, r, imgs = job(n, rows, 6, 1)
+        turned = dict(r, angZ=np.linspace(10.0, 300.0, rows))
+        for first, second in (((p, r, imgs), (p, turned, imgs)), ((dict(p, escc=0), turned, imgs), (dict(p, escc=0), r, imgs))):
+            got = []
+            for j in (first, second):
+                with U.Batch([j], autotune=True) as B:
+                    got.append(B.tuning(0))
+                    assert rel(B.run()[0], oracle.reconstruct(*j)) < 1e-5
+            print("tuned", n, got, flush=True)
+            assert got[0 if first[1] is turned else 1]["planes"] == 0
+
+
 def test_device_batch_launch_replays_equal_the_stream_form():
     """Device-resident jobs: utr_batch_launch replays the captured graph back
     to back; every replay (with eager reconstructions in between) gives the

@@ -361,7 +361,7 @@ int launch_2d(utr_ctx* c, const float* d_img, int row0, int count, cplx<T>* d_sp
         using F = utr::Fft<N, T>;                                                               \
         const int ncol = g.nx / 2 + 1; /* the rest by Hermitian symmetry */                     \
         const int gx = (ncol + F::NB - 1) / F::NB;                                              \
-        int wpc = std::max(1, F::WPC); /* resident per CU */                                    \
+        int wpc = std::max(1, F::WPC); /* per CU, at most as many as its threads and LDS take */ \
         if (c->cols_wpc > 0) wpc = std::min(wpc, c->cols_wpc);                                  \
         const unsigned grid = std::min(utr::xcd_grid(gx * count), persistent_cap(c, wpc));      \
         if (g.ctf_mode == 1 || g.ctf_mode == 3)                                                 \
@@ -1143,7 +1143,20 @@ struct JobTune {
     int form = UTR_FP32, planes = 0, rows_wpc = 0, cols_wpc = 0;
 };
 std::mutex g_tune_mu;
-std::map<std::tuple<int, int, int, int>, JobTune> g_tune;  // (nx, ny, nz, rows) -> tuning
+using TuneKey = std::tuple<int, int, int, int, int>;  // nx, ny, nz, rows, tune_kind
+std::map<TuneKey, JobTune> g_tune;
+
+// What else decides which kernels a job runs: the gridding form (rows without
+// rotation about Z, centre shift, noise gate), the 2D filter's column kernel
+// and the voxel epilogue's filters.
+int tune_kind(const utr_ctx* c) {
+    const auto& g = c->plan.g;
+    const bool bits[] = {c->plan.all_y_exact != 0, g.escc != 0, g.rot_centre_shift != 0, g.nsr2 > 0, g.do_tie3d != 0,
+                         g.do_ctf3d != 0, g.do_invlap != 0};
+    int k = g.ctf_mode;
+    for (bool b : bits) k = 2 * k + (b ? 1 : 0);
+    return k;
+}
 
 int time_job(utr_ctx* c, const float* d_img, float* d_vol, float* ms) {
     hipEvent_t a = c->ev[4], b = c->ev[5];
@@ -1231,7 +1244,7 @@ int utr_batch_create(const utr_job* jobs, int njobs, int autotune, utr_batch** o
         if (hipEventCreateWithFlags(&b->join[j], hipEventDisableTiming) != hipSuccess)
             return fail(set_err(UTR_E_DEVICE, "event creation failed"));
         if (autotune) {
-            const auto key = std::make_tuple(g.nx, g.ny, g.nz, J.nrows);
+            const TuneKey key{g.nx, g.ny, g.nz, J.nrows, tune_kind(c)};
             bool have = false;
             JobTune T;
             {

@@ -29,12 +29,7 @@ typedef short cr_s4 __attribute__((ext_vector_type(4)));
 typedef float cr_f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 cr_b8 __attribute__((ext_vector_type(8)));
 
-// BF16 <-> FP32 (round to nearest even; NaN stays NaN)
-__host__ __device__ __forceinline__ float cr_bf2f(unsigned short h) {
-    union { unsigned u; float f; } v;
-    v.u = (unsigned)h << 16;
-    return v.f;
-}
+// FP32 to BF16 (round to nearest even; NaN stays NaN)
 __host__ __device__ __forceinline__ unsigned short cr_f2bf(float f) {
     union { unsigned u; float f; } v;
     v.f = f;

@@ -797,8 +797,8 @@ __device__ __forceinline__ long long dround_i64(double d) {
 // round(w * k) as a 64-bit integer for |w * k| < 2^51: one fma rounds the
 // exact product once, as dround_i64 of the exact product would
 __device__ __forceinline__ long long fx_term(double w, double k) {
-    const double y = __fma_rn(w, k, 6755399441055744.0);
-    return (long long)(__double_as_longlong(y) - 0x4338000000000000LL);
+    const double y = __fma_rn(w, k, DROUND);
+    return (long long)(__double_as_longlong(y) - DROUND_BITS);
 }
 
 // ROT: rows carry the centre-shift phase (compiled separately: its FP64

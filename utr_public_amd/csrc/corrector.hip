@@ -142,7 +142,7 @@ struct CrConv {
     float* part;               // [work-group][20]: {dw1[16], db1, dalpha, loss, 0}
 };
 
-constexpr int CR_Z = 4;  // output planes of a work-group's block
+constexpr int CR_PX = 2, CR_PY = 2, CR_Z = 4;  // patches in x and y, and planes, of a work-group's block
 
 // Waves per SIMD the register budget is set for.
 constexpr int cr_occ(int nb) { return nb == 3 ? 3 : 4; }
@@ -150,9 +150,12 @@ constexpr int cr_occ(int nb) { return nb == 3 ? 3 : 4; }
 // 3x3x3 convolution, stride 1, zero padding 1, as an implicit GEMM: output
 // channels are the matrix rows, 16 voxels (a 4 x 4 patch of one z plane) its
 // columns, K = 32 is two (dy, dx) taps of 16 input channels.  A work-group
-// owns PX x PY patches in x and y, CR_Z planes in z and NB blocks of 16 output
-// channels; each of its PX PY waves takes one patch through all planes (two
-// patches a wave spilled registers at four waves per SIMD).
+// owns CR_PX x CR_PY patches in x and y, CR_Z planes in z and NB blocks of 16
+// output channels; each of its waves takes one patch through all planes (two
+// patches a wave spilled registers at four waves per SIMD; eight patches and
+// waves, 16 x 8 voxels with 2.1 times the input staged instead of 2.3, took
+// 1.0 to 1.4 times the time over the layers of 24^3 to 112^3 crops: waves wait
+// for the others of their work-group at every slice).
 //
 // What bounds it: for 16 channels the activations' traffic, for more the LDS
 // reads against the matrix cores.  Rows = channels lets a lane hold four
@@ -167,8 +170,9 @@ constexpr int cr_occ(int nb) { return nb == 3 ? 3 : 4; }
 // The passes around a convolution are its own loads and stores (CrIn, CrEpi):
 // upsampling and concatenation, pooling, their adjoints, the head and the loss
 // each read and wrote whole activations in kernels of their own before.
-template <int PX, int PY, int NB, int EPI>
-__global__ void __launch_bounds__(64 * PX * PY, cr_occ(NB)) k_cr_conv(CrConv A) {
+template <int NB, int EPI>
+__global__ void __launch_bounds__(64 * CR_PX * CR_PY, cr_occ(NB)) k_cr_conv(CrConv A) {
+    constexpr int PX = CR_PX, PY = CR_PY;
     constexpr int HX = 4 * PX + 2, HY = 4 * PY + 2, HZ = CR_Z + 2;
     constexpr int PITCH = 4 * PX + 4, HALF = HZ * HY * PITCH + 4;  // 16-byte units; HALF = 4 mod 8
     constexpr int NV = HX * HY * HZ, NT = 64 * PX * PY;
@@ -858,25 +862,18 @@ CrCubes cr_cubes(int T, int h) {
     return Q;
 }
 
-// Work-groups a convolution's cube [lo, hi)^3 of n crops splits into: blocks
-// of 16 x 8 voxels in x and y where they make at least two work-groups per CU,
-// 8 x 8 otherwise (the coarsest level of a few crops).
-long cr_conv_tiles(int px, int py, int n, CrCube q) {
+// Work-groups that a cube [lo, hi)^3 of n crops splits into: blocks of px x py
+// patches and CR_Z planes.
+long cr_tiles(int px, int py, int n, CrCube q) {
     const long e = q.hi - q.lo;
     return n * ((e + 4 * px - 1) / (4 * px)) * ((e + 4 * py - 1) / (4 * py)) * ((e + utr::CR_Z - 1) / utr::CR_Z);
 }
-bool cr_conv_big(int n, CrCube q) { return cr_conv_tiles(4, 2, n, q) >= 512; }
+long cr_conv_tiles(int n, CrCube q) { return cr_tiles(utr::CR_PX, utr::CR_PY, n, q); }
 
 template <int NB, int EPI>
 int cr_conv_launch(utr_corr* c, const utr::CrConv& A) {
-    const CrCube q = {A.lo, A.hi};
-    if (cr_conv_big(A.s.n, q)) {
-        const unsigned grid = utr::xcd_grid((unsigned)cr_conv_tiles(4, 2, A.s.n, q) * (unsigned)(A.nbt / NB));
-        utr::k_cr_conv<4, 2, NB, EPI><<<grid, 512, 0, c->st>>>(A);
-    } else {
-        const unsigned grid = utr::xcd_grid((unsigned)cr_conv_tiles(2, 2, A.s.n, q) * (unsigned)(A.nbt / NB));
-        utr::k_cr_conv<2, 2, NB, EPI><<<grid, 256, 0, c->st>>>(A);
-    }
+    const unsigned tiles = (unsigned)cr_conv_tiles(A.s.n, CrCube{A.lo, A.hi}) * (unsigned)(A.nbt / NB);
+    utr::k_cr_conv<NB, EPI><<<utr::xcd_grid(tiles), 64 * utr::CR_PX * utr::CR_PY, 0, c->st>>>(A);
     UTR_HIP_TRY(hipGetLastError());
     return UTR_OK;
 }
@@ -997,7 +994,7 @@ int cr_alloc(utr_corr* c) {
     const size_t n2 = n1 / 8, n3 = n1 / 64;
     // the loss's partial sums: one row per work-group of the last convolution
     const CrCube q = {c->halo, c->T - c->halo};
-    const size_t hp = (size_t)std::max(cr_conv_tiles(4, 2, c->batch, q), cr_conv_tiles(2, 2, c->batch, q)) * 20;
+    const size_t hp = (size_t)cr_conv_tiles(c->batch, q) * 20;
     const hipError_t e[] = {
         c->e1a.alloc(n1 * 16), c->e1b.alloc(n1 * 16), c->p1.alloc(n2 * 16), c->e2a.alloc(n2 * 32),
         c->e2b.alloc(n2 * 32), c->p2.alloc(n3 * 32), c->e3a.alloc(n3 * 64), c->e3b.alloc(n3 * 64),
@@ -1032,7 +1029,7 @@ int cr_forward(utr_corr* c, int nb, const utr::CrVol& V, const CrCubes& Q) {
     const int T = c->T;
     const utr::CrShape s1 = cr_shape(nb, T), s2 = cr_shape(nb, T / 2), s3 = cr_shape(nb, T / 4);
     int rc;
-    utr::k_cr_first<<<utr::xcd_grid((unsigned)cr_conv_tiles(4, 2, nb, Q.e1a)), 256, 0, c->st>>>(
+    utr::k_cr_first<<<utr::xcd_grid((unsigned)cr_tiles(4, 2, nb, Q.e1a)), 256, 0, c->st>>>(
         V, c->wfirst.p, c->w.p + c->L[0].boff, c->e1a.p, s1, Q.e1a.lo, Q.e1a.hi);
     UTR_HIP_TRY(hipGetLastError());
     if ((rc = cr_act(c, 1, cr_in(c->e1a, 16), c->e1b.p, s1, Q.e1b, c->p1.p))) return rc;
@@ -1071,7 +1068,7 @@ int cr_backward(utr_corr* c, int nb, const utr::CrVol& V, const CrCubes& Q, cons
     A.tscale = c->scale;
     A.inv_count = (float)(1.0 / cnt);
     A.part = c->hpart.p;
-    const long nwg = cr_conv_big(nb, Q.d1b) ? cr_conv_tiles(4, 2, nb, Q.d1b) : cr_conv_tiles(2, 2, nb, Q.d1b);
+    const long nwg = cr_conv_tiles(nb, Q.d1b);
     if ((size_t)nwg * 20 > c->hpart.n) return set_err(UTR_E_STATE, "corrector: loss workspace too small");
     if ((rc = cr_conv_launch<1, utr::CR_LOSS>(c, A))) return rc;
     utr::k_cr_head_reduce<<<1, 640, 0, c->st>>>(c->hpart.p, (int)nwg, kCrHead, c->res.p, c->g.p + c->headoff);

@@ -73,7 +73,7 @@ constexpr int DHT_VOX = DHT_BX * DHT_BY * DHT_BZ;
 constexpr int DHT_LINES = 512;    // source lines listed together (two a thread)
 // and their samples: the map to grid positions is a rotation, so the unit
 // cubes about the samples of a 17.1 x 9.1 x 9.1 box lie in that box grown by
-// sqrt(3)/2 on every side, whose volume is 2214
+// sqrt(3)/2 on every side, whose volume is 2210
 constexpr int DHT_POINTS = 2304;
 
 __device__ __forceinline__ double dht_freq(int k, int n, double xst) {
@@ -360,17 +360,18 @@ __device__ __forceinline__ double dht_quot(double a, double b, double r) {
 // (y_j - yc) cosZ; (z_n - zc) sinY, (z_n - zc) cosY, as DHT.cpp:1083-1107.
 //
 // Per orientation the threads clip the source lines (n, j) that can reach the
-// brick to it (about 400 lines of 4 samples on average, 1.34 times the brick's
-// voxels in all), give each line a run of the brick's point list (a wave
+// brick to it (some hundred lines of a few samples, 1416 samples on average: 1.38
+// times the brick's voxels), give each line a run of the brick's point list (a wave
 // prefix sum and one LDS add per wave) and write the line's number into its
 // run; then every thread takes points, one sample each, so all lanes work
 // (with a line per lane they waited for the wave's longest line).  The order
 // of the points does not matter: the sums are exact.  Lists are double
 // buffered, so one barrier separates a list's writing from its reading.  A
 // sample's eight corners go to LDS without bounds tests (the halo takes those
-// outside).  Bound by the FP64 instructions of a sample.  Measured with 108
-// random orientations of 256 x 128 x 151 samples: 5.11 ms, against 11.75 ms
-// with a line per lane and IEEE divisions.
+// outside).  The vector unit is busy 37 % of the time and the LDS 23 %, half of
+// that in bank conflicts: the rest is the latency of a brick's rounds.  Measured
+// with 108 random orientations of 256 x 128 x 151 samples: 5.11 ms, against
+// 11.75 ms with a line per lane and IEEE divisions.
 __global__ void __launch_bounds__(256) k_dht_splat(const float* __restrict__ P, DhtGeom g,
                                                    const DhtRow* __restrict__ rows,
                                                    const double* __restrict__ xs,
@@ -561,9 +562,9 @@ namespace utr {
 // Images lower than a workgroup's threads split the listed samples between
 // groups of waves; all sums meet in LDS at the end.
 // The fixed-point terms are those of k_dht_splat expression by expression,
-// so both kernels form the same sums.  Bound by the FP64 instructions of a
-// term.  Measured for 96 orientations of 256^3 samples: 4.28 ms,
-// against 5.42 ms with an LDS addition per term.
+// so both kernels form the same sums.  The vector unit is busy half of the time;
+// for the rest the waves wait for the values (1.4 times the stack passes the L2).  Measured for 96 orientations of 256^3 samples: 4.28 ms, against
+// 5.32 ms with an LDS addition per term.
 constexpr int DC_X = 4, DC_Z = 4;
 // candidate half-width (source samples): the cells a column's corners reach
 // form a 5 x 5 square about its centre, whose corners lie 2.5 sqrt(2) = 3.54

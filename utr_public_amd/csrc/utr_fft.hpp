@@ -346,7 +346,7 @@ struct Fft {
     static constexpr int NT = NT_;
     using Q = FftReg<N, NT>;
     static constexpr int NB = Q::NB, M = Q::M, LDS = Q::LDS;
-    // workgroups a CU holds at most, by threads and by LDS
+    // workgroups a CU holds at most, by threads and by LDS (registers may allow fewer)
     static constexpr int WPC = 2048 / NT < 163840 / (LDS * (int)sizeof(cplx<T>)) ? 2048 / NT
                                                                                : 163840 / (LDS * (int)sizeof(cplx<T>));
     __device__ static __forceinline__ void cols(cplx<T>* u, cplx<T>* sm, const cplx<T>* tw, int sign, int tid,
